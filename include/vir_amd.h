@@ -34,8 +34,9 @@ extern "C" {
 #define VIR_SEQUENTIAL 2u   /* plain sequential f32 sums in reference order */
 #define VIR_UNGUARDED 4u    /* Siddon FP/BP: vir_siddon_count_guarded gave 0
                                for these rays and grid */
-#define VIR_PER_OUTPUT 8u   /* DD 2-D / SF: the one-thread-per-output kernels
-                               instead of the tiled ones (same bits) */
+#define VIR_PER_OUTPUT 8u   /* the one-thread-per-output kernels instead of the
+                               tiled ones (DD 2-D and SF: same bits; ray-driven
+                               backprojection: float32 rounding apart) */
 #define VIR_SF_UNIT_AMPLITUDE 16u  /* SF parallel modes: footprint amplitude 1
                                instead of 1/(|sin|+|cos|) -- the rectangle
                                footprint of fp_2d_par.py:67-125 */

@@ -47,6 +47,8 @@ struct RDGeo {
     float out_scale;
     float bmin[3], bmax[3], c0[3];
     int compat;   // VIR_COMPAT: axis-parallel rays outside the image hit (clamped)
+    float inv_du, inv_dv;
+    float mar;    // rounding margin of projected bin indices, in bins (rd_u_range)
 };
 
 struct RDRay {
@@ -408,6 +410,345 @@ __global__ __launch_bounds__(256) void k_rd_bp(RDGeo G, const float* __restrict_
     img[t] = r;
 }
 
+// ------------------------------------------------- backward from ray tables
+//
+// The per-voxel gather above sets up every ray (a square root and nine
+// divisions) again for each voxel and bin it tests, and is bound by that VALU
+// work: 74.4 ms for Joseph cone at 128^3, 180 views of 192^2 (6.9 ms here);
+// 0.71 ms for path lengths at 129 x 127, 181 views of 223 (0.03 ms here, where
+// the views are split over waves as well).  The kernels below
+// set each ray up once per block and view, in an LDS table, and leave a voxel
+// with the bins its shadow really meets.  Path lengths are the differences of
+// the same quotients as in the forward traversal (the pair stays an exact
+// transpose).  Joseph's samples are taken in voxel units from the ray's entry
+// point: the position there is formed in float64 from the float32 ray and has
+// the size of the grid, not of the source distance, so it rounds less than
+// o + t h does.  They run over the same k with t0 + k/2 <= t1 in float32 as the
+// forward projection's.
+
+// Bins [u0, u1] whose rays can meet the box [x0, x1] x [y0, y1] (the convex
+// hull of the projected corners, widened by G.mar for rounding), and the
+// least and largest magnification of its corners.
+template <int MODE>
+__device__ __forceinline__ void rd_u_range(const RDGeo& G, float c, float s, float x0, float x1, float y0, float y1,
+                                           int& u0, int& u1, float& mmin, float& mmax) {
+    float umin = VIR_INF, umax = -VIR_INF;
+    mmin = VIR_INF;
+    mmax = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const float x = (k & 1) ? x1 : x0, y = (k & 2) ? y1 : y0;
+        const float p = c * y - s * x;
+        float m = 1.0f;
+        if (MODE != RD_PAR2) m = G.DSD * __builtin_amdgcn_rcpf(G.DSO - (c * x + s * y));
+        umin = fminf(umin, m * p);
+        umax = fmaxf(umax, m * p);
+        mmin = fminf(mmin, m);
+        mmax = fmaxf(mmax, m);
+    }
+    const float off = G.ucen - G.su;
+    u0 = (int)fmaxf(ceilf(umin * G.inv_du + off - G.mar), 0.0f);
+    u1 = (int)fminf(floorf(umax * G.inv_du + off + G.mar), (float)(G.nu - 1));
+}
+
+// Detector rows [v0, v1] of the heights [z0, z1] at magnifications [mmin, mmax].
+__device__ __forceinline__ void rd_v_range(const RDGeo& G, float z0, float z1, float mmin, float mmax, int& v0,
+                                           int& v1) {
+    const float off = G.ucen - G.sv;
+    const float lo = z0 * (z0 < 0.0f ? mmax : mmin), hi = z1 * (z1 < 0.0f ? mmin : mmax);
+    v0 = (int)fmaxf(ceilf(lo * G.inv_dv + off - G.mar), 0.0f);
+    v1 = (int)fminf(floorf(hi * G.inv_dv + off + G.mar), (float)(G.nv - 1));
+}
+
+// A ray of an LDS table.  Joseph: position at t0 (p) and step per sample (h)
+// in voxels, the reciprocals of the step (r) and the last sample's index (t1).
+// Path lengths: origin, direction and its reciprocal in world units and
+// [t0, t1], so that plane crossings come out as the forward traversal's
+// quotients.  t1 < t0: dead.
+template <int NA>
+struct RDTab {
+    float p[NA], h[NA], r[NA], t0, t1, y;
+};
+
+template <int MODE, bool JOSEPH, int NA>
+__device__ __forceinline__ RDTab<NA> rd_tab(const RDGeo& G, float c, float s, int iu, int iv, float y) {
+    const int n[3] = {G.nx, G.ny, G.nz};
+    RDTab<NA> T;
+    T.y = y;
+    T.t0 = 0.0f;
+    T.t1 = -1.0f;
+    const RDRay R = rd_ray<MODE>(G, c, s, iu, iv);
+    const bool live = R.hit && y != 0.0f;
+    const double inv_d = 1.0 / (double)G.d;
+#pragma unroll
+    for (int a = 0; a < NA; ++a) {
+        if (JOSEPH) {
+            T.p[a] = (float)(((double)R.o[a] + (double)R.t0 * (double)R.h[a] - (double)G.c0[a]) * inv_d);
+            T.h[a] = (float)((double)(kRdStep * R.h[a]) * inv_d);
+        } else {
+            T.p[a] = R.o[a];
+            T.h[a] = R.h[a];
+            if (!(fabsf(R.h[a]) > kRdEps)) {  // parallel to the axis: in one voxel row, from its centre
+                T.p[a] = G.bmin[a] + ((float)rd_index(G, a, R.o[a], n[a]) + 0.5f) * G.d;
+                T.h[a] = 1e-30f;
+            }
+        }
+        // finite reciprocals: a ray that does not move along an axis gets
+        // interval ends far beyond [t0, t1], both of one sign outside
+        T.r[a] = fminf(fmaxf(1.0f / T.h[a], -1e30f), 1e30f);
+    }
+    if (!live) return T;
+    if (JOSEPH) {
+        int k = (int)((R.t1 - R.t0) * (1.0f / kRdStep));
+        // (bounded: far sources, where t0 + 1/2 rounds to t0, end it too)
+        for (int i = 0; i < 65536 && R.t0 + (float)(k + 1) * kRdStep <= R.t1; ++i) ++k;
+        while (k > 0 && !(R.t0 + (float)k * kRdStep <= R.t1)) --k;
+        T.t1 = (float)k;
+    } else {
+        T.t0 = R.t0;
+        T.t1 = R.t1;
+    }
+    return T;
+}
+
+// a / b from the correctly rounded reciprocal r of b (Markstein's correction)
+__device__ __forceinline__ float rd_quot(float a, float b, float r) {
+    const float q = a * r;
+    return __builtin_fmaf(__builtin_fmaf(-q, b, a), r, q);
+}
+
+// The voxel a lane works on: index coordinates (Joseph) or its lower and
+// upper planes (path lengths).
+template <bool JOSEPH>
+__device__ __forceinline__ void rd_voxel(const RDGeo& G, int a, int i, float& f0, float& f1) {
+    f0 = JOSEPH ? (float)i : G.bmin[a] + (float)i * G.d;
+    f1 = JOSEPH ? 0.0f : G.bmin[a] + (float)(i + 1) * G.d;
+}
+
+// Weight of a table ray on that voxel: the summed hat-function products of
+// its samples (Joseph; samples outside the voxel's 2-voxel box weigh zero, so
+// the sample range only has to cover it), or its path length.
+template <bool JOSEPH, int NA>
+__device__ __forceinline__ float rd_tab_w(const RDTab<NA>& T, const float* f0, const float* f1) {
+    float x[NA], lo = T.t0, hi = T.t1;
+    if (!JOSEPH) {
+#pragma unroll
+        for (int a = 0; a < NA; ++a) {
+            const float p = rd_quot(f0[a] - T.p[a], T.h[a], T.r[a]), q = rd_quot(f1[a] - T.p[a], T.h[a], T.r[a]);
+            lo = fmaxf(lo, fminf(p, q));
+            hi = fminf(hi, fmaxf(p, q));
+        }
+        return hi > lo ? hi - lo : 0.0f;
+    }
+    float pl = -VIR_INF, ph = VIR_INF;
+#pragma unroll
+    for (int a = 0; a < NA; ++a) {
+        x[a] = T.p[a] - f0[a];
+        const float p = (-1.0f - x[a]) * T.r[a], q = (1.0f - x[a]) * T.r[a];
+        pl = fmaxf(pl, fminf(p, q));
+        ph = fminf(ph, fmaxf(p, q));
+    }
+    lo = fmaxf(lo, ceilf(pl - 0.02f));
+    hi = fminf(hi, floorf(ph + 0.02f));
+    float w = 0.0f;
+    for (float k = lo; k <= hi; k += 1.0f) {
+        float wk = 1.0f;
+#pragma unroll
+        for (int a = 0; a < NA; ++a)
+            wk *= fmaxf(1.0f - fabsf(__builtin_fmaf(k, T.h[a], x[a])), 0.0f);
+        w += wk;
+    }
+    return w * kRdStep;
+}
+
+// Cone beam: a block of eight waves takes 8 x NC columns of 64 voxels, NC
+// columns a wave (lane = voxel of the column), one view at a time.
+constexpr int kRdWaves = 8;
+constexpr int kRdCap = 832;  // rays of one table: 39 KiB, four blocks a CU
+
+template <bool JOSEPH, int NC>
+__global__ __launch_bounds__(64 * kRdWaves) void k_rd_bp_cone_tab(RDGeo G, const float* __restrict__ cs,
+                                                                 const float* __restrict__ sn,
+                                                                 const float* __restrict__ sino,
+                                                                 float* __restrict__ img, int accumulate, int nby,
+                                                                 int nbz) {
+    // columns x = bx .. bx + 3, y = by .. by + 2 NC - 1
+    constexpr int BX = 4, BY = 2 * NC, NCOL = BX * BY;
+    __shared__ float4 ta[kRdCap], tb[kRdCap], tc[kRdCap];
+    __shared__ int cu0[NCOL], cu1[NCOL];
+    __shared__ float cm0[NCOL], cm1[NCOL];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int blk = (int)xcd_remap(blockIdx.x, gridDim.x);
+    const int bz = (blk % nbz) * 64;
+    blk /= nbz;
+    const int by = (blk % nby) * BY, bx = (blk / nby) * BX;
+    const int iz = bz + lane;
+    // the box of voxel index range [i, j] along axis a: voxels (path length)
+    // or one voxel around the centres (Joseph)
+    auto box_lo = [&](int a, int i) { return JOSEPH ? G.c0[a] + (float)(i - 1) * G.d : G.bmin[a] + (float)i * G.d; };
+    auto box_hi = [&](int a, int j) { return JOSEPH ? G.c0[a] + (float)(j + 1) * G.d : G.bmin[a] + (float)(j + 1) * G.d; };
+    const int ex = min(bx + BX, G.nx) - 1, ey = min(by + BY, G.ny) - 1, ez = min(bz + 64, G.nz) - 1;
+    const float X0 = box_lo(0, bx), X1 = box_hi(0, ex), Y0 = box_lo(1, by), Y1 = box_hi(1, ey);
+    const float Z0 = box_lo(2, bz), Z1 = box_hi(2, ez);
+    const float z0 = box_lo(2, iz), z1 = box_hi(2, iz);
+    double acc[NC];
+#pragma unroll
+    for (int q = 0; q < NC; ++q) acc[q] = 0.0;
+    for (int ia = 0; ia < G.na; ++ia) {
+        const float c = cs[ia], s = sn[ia];
+        int U0, U1, V0, V1;
+        float m0, m1;
+        rd_u_range<RD_CONE3>(G, c, s, X0, X1, Y0, Y1, U0, U1, m0, m1);
+        rd_v_range(G, Z0, Z1, m0, m1, V0, V1);
+        if (U1 < U0 || V1 < V0) continue;  // the same in every thread
+        const int cv = min(V1 - V0 + 1, kRdCap), cu = min(U1 - U0 + 1, kRdCap / cv);
+        const float* plane = sino + (int64_t)ia * G.nu * G.nv;
+        for (int ub = U0; ub <= U1; ub += cu)
+            for (int vb = V0; vb <= V1; vb += cv) {
+                const int ue = min(ub + cu - 1, U1), ve = min(vb + cv - 1, V1);
+                __syncthreads();  // the table's last readers are done
+                for (int e = tid; e < (ue - ub + 1) * cv; e += 64 * kRdWaves) {
+                    const int iu = ub + e / cv, iv = vb + e % cv;
+                    const bool in = iv <= ve;
+                    const RDTab<3> T = rd_tab<RD_CONE3, JOSEPH, 3>(G, c, s, iu, iv, in ? plane[(int64_t)iu * G.nv + iv] : 0.0f);
+                    ta[e] = make_float4(T.p[0], T.p[1], T.p[2], T.y);
+                    tb[e] = make_float4(T.r[0], T.r[1], T.r[2], T.t1);
+                    tc[e] = make_float4(T.h[0], T.h[1], T.h[2], T.t0);
+                }
+                if (tid < NCOL) {
+                    const int ix = bx + tid % BX, iy = by + tid / BX;
+                    rd_u_range<RD_CONE3>(G, c, s, box_lo(0, ix), box_hi(0, ix), box_lo(1, iy), box_hi(1, iy), cu0[tid],
+                                         cu1[tid], cm0[tid], cm1[tid]);
+                }
+                __syncthreads();
+#pragma unroll
+                for (int q = 0; q < NC; ++q) {
+                    const int col = wave + kRdWaves * q;  // x = col % BX, y = col / BX
+                    float f0[3], f1[3];
+                    rd_voxel<JOSEPH>(G, 0, bx + col % BX, f0[0], f1[0]);
+                    rd_voxel<JOSEPH>(G, 1, by + col / BX, f0[1], f1[1]);
+                    rd_voxel<JOSEPH>(G, 2, iz, f0[2], f1[2]);
+                    int v0, v1;
+                    rd_v_range(G, z0, z1, cm0[col], cm1[col], v0, v1);
+                    v0 = max(v0, vb);
+                    v1 = min(v1, ve);
+                    if (iz >= G.nz) v1 = -1;
+                    const int u1 = min(cu1[col], ue);
+                    for (int iu = max(cu0[col], ub); iu <= u1; ++iu)
+                        for (int iv = v0; iv <= v1; ++iv) {
+                            const int e = (iu - ub) * cv + iv - vb;
+                            const float4 a = ta[e], b = tb[e], h = tc[e];
+                            const RDTab<3> T = {{a.x, a.y, a.z}, {h.x, h.y, h.z}, {b.x, b.y, b.z}, h.w, b.w, a.w};
+                            const float w = rd_tab_w<JOSEPH, 3>(T, f0, f1);
+                            if (w != 0.0f) acc[q] += (double)(T.y * w);
+                        }
+                }
+            }
+    }
+    if (iz >= G.nz) return;
+#pragma unroll
+    for (int q = 0; q < NC; ++q) {
+        const int col = wave + kRdWaves * q;
+        const int ix = bx + col % BX, iy = by + col / BX;
+        if (ix >= G.nx || iy >= G.ny) continue;
+        const int64_t o = ((int64_t)ix * G.ny + iy) * G.nz + iz;
+        float r = (float)acc[q] * G.out_scale;
+        if (accumulate) r += img[o];
+        img[o] = r;
+    }
+}
+
+// Parallel and fan beam: a block takes a tile of 16 x 8 pixels, two a lane;
+// its NW waves share the views (wave w takes the view pairs w, w + NW, ...)
+// and keep a table each, so the view loop has no barrier; the waves' float64
+// sums are added in wave order.  A table holds 32 rays of two views; a tile
+// that meets more is done in several rounds.
+constexpr int kRd2X = 16, kRd2Y = 8;
+
+template <int MODE, bool JOSEPH, int NW>
+__global__ __launch_bounds__(64 * NW) void k_rd_bp_2d_tab(RDGeo G, const float* __restrict__ cs,
+                                                          const float* __restrict__ sn,
+                                                          const float* __restrict__ sino, float* __restrict__ img,
+                                                          int accumulate, int nby) {
+    __shared__ float4 tab[NW][64][2];
+    __shared__ float tab_y[NW][64];
+    __shared__ double part[NW][kRd2X * kRd2Y];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int bx = (blockIdx.x / nby) * kRd2X, by = (blockIdx.x % nby) * kRd2Y;
+    auto box_lo = [&](int a, int i) { return JOSEPH ? G.c0[a] + (float)(i - 1) * G.d : G.bmin[a] + (float)i * G.d; };
+    auto box_hi = [&](int a, int j) { return JOSEPH ? G.c0[a] + (float)(j + 1) * G.d : G.bmin[a] + (float)(j + 1) * G.d; };
+    const float X0 = box_lo(0, bx), X1 = box_hi(0, min(bx + kRd2X, G.nx) - 1);
+    const float Y0 = box_lo(1, by), Y1 = box_hi(1, min(by + kRd2Y, G.ny) - 1);
+    // this lane's pixels: (bx + lane / 8, by + lane % 8) and eight rows on
+    const int ix = bx + (lane >> 3), iy = by + (lane & 7);
+    const int slot = lane >> 5, j = lane & 31;
+    float4(*t)[2] = tab[wave];
+    float* ty = tab_y[wave];
+    double acc[2] = {0.0, 0.0};
+    for (int a0 = 2 * wave; a0 < G.na; a0 += 2 * NW) {
+        const int ia = min(a0 + slot, G.na - 1);
+        int U0, U1;
+        float m0, m1;
+        rd_u_range<MODE>(G, cs[ia], sn[ia], X0, X1, Y0, Y1, U0, U1, m0, m1);
+        if (a0 + slot >= G.na) U1 = U0 - 1;
+        // the two views' ranges, the same in every lane
+        const int A0 = __builtin_amdgcn_readlane(U0, 0), A1 = __builtin_amdgcn_readlane(U1, 0);
+        const int B0 = __builtin_amdgcn_readlane(U0, 32), B1 = __builtin_amdgcn_readlane(U1, 32);
+        const int rounds = (max(max(A1 - A0, B1 - B0), -1) + 32) / 32;
+        for (int rd = 0; rd < rounds; ++rd) {
+            const int iu = U0 + 32 * rd + j;
+            if (iu <= U1) {
+                const RDTab<2> T = rd_tab<MODE, JOSEPH, 2>(G, cs[ia], sn[ia], iu, 0, sino[(int64_t)ia * G.nu + iu]);
+                t[lane][0] = make_float4(T.p[0], T.p[1], T.t0, T.t1);
+                t[lane][1] = make_float4(T.r[0], T.r[1], T.h[0], T.h[1]);
+                ty[lane] = T.y;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // a wave's LDS accesses are in order
+#pragma unroll
+            for (int sl = 0; sl < 2; ++sl) {
+                const int base = (sl ? B0 : A0) + 32 * rd, end = min(base + 31, sl ? B1 : A1);
+                if (end < base) continue;
+                const float c = cs[a0 + sl], s = sn[a0 + sl];
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const int px = ix + 8 * q;
+                    int u0, u1;
+                    rd_u_range<MODE>(G, c, s, box_lo(0, px), box_hi(0, px), box_lo(1, iy), box_hi(1, iy), u0, u1, m0, m1);
+                    u0 = max(u0, base);
+                    u1 = min(u1, end);
+                    float f0[2], f1[2];
+                    rd_voxel<JOSEPH>(G, 0, px, f0[0], f1[0]);
+                    rd_voxel<JOSEPH>(G, 1, iy, f0[1], f1[1]);
+                    for (int u = u0; u <= u1; ++u) {
+                        const int e = 32 * sl + u - base;
+                        const float4 a = t[e][0], b = t[e][1];
+                        const RDTab<2> T = {{a.x, a.y}, {b.z, b.w}, {b.x, b.y}, a.z, a.w, ty[e]};
+                        const float w = rd_tab_w<JOSEPH, 2>(T, f0, f1);
+                        if (w != 0.0f) acc[q] += (double)(T.y * w);
+                    }
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
+    }
+    part[wave][lane] = acc[0];
+    part[wave][64 + lane] = acc[1];
+    __syncthreads();
+    for (int e = tid; e < kRd2X * kRd2Y; e += 64 * NW) {
+        const int px = bx + (e >> 3), py = by + (e & 7);
+        if (px >= G.nx || py >= G.ny) continue;
+        double sum = part[0][e];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) sum += part[w][e];
+        const int64_t o = (int64_t)px * G.ny + py;
+        float r = (float)sum * G.out_scale;
+        if (accumulate) r += img[o];
+        img[o] = r;
+    }
+}
+
 static int rd_setup(const vir_rd_geom* g, RDGeo& G) {
     if (!g) return fail_arg("geometry is NULL");
     if (g->mode < 0 || g->mode > 2) return fail_arg("mode must be 0 (par), 1 (fan) or 2 (cone)");
@@ -427,12 +768,64 @@ static int rd_setup(const vir_rd_geom* g, RDGeo& G) {
         G.bmax[a] = G.d * (float)n[a] / 2.0f;
         G.c0[a] = -G.d * ((float)n[a] / 2.0f - 0.5f);
     }
+    G.inv_du = 1.0f / G.du;
+    G.inv_dv = 1.0f / G.dv;
     if (g->mode != RD_PAR2) {
         if (!(G.DSO > 0.0f) || !(G.DSD > G.DSO)) return fail_arg("need 0 < DSO < DSD");
         const double hx = 0.5 * G.nx * (double)G.d, hy = 0.5 * G.ny * (double)G.d;
         if (!(std::sqrt(hx * hx + hy * hy) + 2.0 * G.d < G.DSO)) return fail_arg("grid reaches the source");
     }
+    // bin indices are sums of terms as large as the detector, its offset and
+    // the grid's shadow (in bins): a few float32 roundings of those
+    const double hz = 0.5 * G.nz * (double)G.d, hr = std::sqrt(0.25 * ((double)G.nx * G.nx + (double)G.ny * G.ny)) * G.d;
+    const double mag = g->mode == RD_PAR2 ? 1.0 : (double)G.DSD / (G.DSO - hr - G.d);
+    const double terms = (double)G.nu + G.nv + std::fabs((double)G.su) + std::fabs((double)G.sv) +
+                         mag * (hr / G.du + (is3 ? hz / G.dv : 0.0));
+    G.mar = (float)(0.02 + 2e-6 * terms);
     return VIR_OK;
+}
+
+// The table kernels' launch.  Cone: four columns a wave (a 4 x 8 x 64 brick,
+// its rays set up once per 2048 voxels) where that gives the chip two blocks
+// a CU, else one column a wave.  2-D: sixteen waves share a tile's views
+// while the tiles alone would leave CUs idle, else four.
+static int rd_bp_tab(const RDGeo& G, int mode, bool jo, const float* cosv, const float* sinv, const float* sino,
+                     float* img, int acc, hipStream_t st) {
+    if (mode == RD_CONE3) {
+        const int nbx = (G.nx + 3) / 4, nbz = (G.nz + 63) / 64;
+        const bool wide = (int64_t)nbx * ((G.ny + 7) / 8) * nbz >= 512;
+        const int nby = wide ? (G.ny + 7) / 8 : (G.ny + 1) / 2;
+        const dim3 grd((unsigned)((int64_t)nbx * nby * nbz)), blk(64 * kRdWaves);
+        if (jo && wide)
+            hipLaunchKernelGGL((k_rd_bp_cone_tab<true, 4>), grd, blk, 0, st, G, cosv, sinv, sino, img, acc, nby, nbz);
+        else if (jo)
+            hipLaunchKernelGGL((k_rd_bp_cone_tab<true, 1>), grd, blk, 0, st, G, cosv, sinv, sino, img, acc, nby, nbz);
+        else if (wide)
+            hipLaunchKernelGGL((k_rd_bp_cone_tab<false, 4>), grd, blk, 0, st, G, cosv, sinv, sino, img, acc, nby, nbz);
+        else
+            hipLaunchKernelGGL((k_rd_bp_cone_tab<false, 1>), grd, blk, 0, st, G, cosv, sinv, sino, img, acc, nby, nbz);
+        return check_hip(hipGetLastError(), "vir_rd_bp launch");
+    }
+    const int nbx = (G.nx + kRd2X - 1) / kRd2X, nby = (G.ny + kRd2Y - 1) / kRd2Y;
+    const int64_t tiles = (int64_t)nbx * nby;
+    const bool many = tiles >= 1024;
+    const dim3 grd((unsigned)tiles);
+#define VIR_RD_BP2(M, J)                                                                                            \
+    do {                                                                                                            \
+        if (many)                                                                                                   \
+            hipLaunchKernelGGL((k_rd_bp_2d_tab<M, J, 4>), grd, dim3(256), 0, st, G, cosv, sinv, sino, img, acc, nby);  \
+        else                                                                                                        \
+            hipLaunchKernelGGL((k_rd_bp_2d_tab<M, J, 16>), grd, dim3(1024), 0, st, G, cosv, sinv, sino, img, acc, nby); \
+    } while (0)
+    if (mode == RD_PAR2) {
+        if (jo) VIR_RD_BP2(RD_PAR2, true);
+        else VIR_RD_BP2(RD_PAR2, false);
+    } else {
+        if (jo) VIR_RD_BP2(RD_FAN2, true);
+        else VIR_RD_BP2(RD_FAN2, false);
+    }
+#undef VIR_RD_BP2
+    return check_hip(hipGetLastError(), "vir_rd_bp launch");
 }
 
 }  // namespace vir
@@ -475,11 +868,14 @@ int vir_rd_bp(const vir_rd_geom* geom, const float* cosv, const float* sinv, con
     if ((G.na > 0 && (!cosv || !sinv || !sino)) || !img) return fail_arg("NULL pointer argument");
     G.out_scale = out_scale;
     G.compat = (flags & VIR_COMPAT) ? 1 : 0;
-    const int64_t n = (int64_t)G.nx * G.ny * G.nz;
-    dim3 grd((unsigned)((n + 255) / 256));
-    hipStream_t st = as_stream(stream);
     const int acc = (flags & VIR_ACCUMULATE) ? 1 : 0;
     const bool jo = geom->joseph != 0;
+    hipStream_t st = as_stream(stream);
+    // VIR_COMPAT's clamped rays reach voxels they do not pass through: only
+    // the per-voxel gather visits those
+    if (!G.compat && !(flags & VIR_PER_OUTPUT)) return rd_bp_tab(G, geom->mode, jo, cosv, sinv, sino, img, acc, st);
+    const int64_t n = (int64_t)G.nx * G.ny * G.nz;
+    dim3 grd((unsigned)((n + 255) / 256));
 #define VIR_RD_BP(M)                                                                                        \
     do {                                                                                                      \
         if (jo) hipLaunchKernelGGL((k_rd_bp<M, true>), grd, dim3(256), 0, st, G, cosv, sinv, sino, img, acc);  \
