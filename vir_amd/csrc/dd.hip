@@ -17,6 +17,7 @@
 #include <algorithm>
 #include <cmath>
 
+#include "cone_tile.h"
 #include "vir_common.h"
 
 namespace vir {
@@ -320,6 +321,46 @@ __device__ __forceinline__ float cone_zmag(const DDGeo& G, const DDView& V, floa
     return G.DSD / (G.DSO - V.oo * orth_c);
 }
 
+// One view of the cone geometry as cone_tile.h's model: weights and ranges of
+// the one-thread-per-output kernels below.
+struct DDCone {
+    static constexpr bool kLineMag = true;
+    const DDGeo& G;
+    DDView V;
+    bool xd;
+    int nd, no;
+    __device__ DDCone(const DDGeo& g, float c, float s, float) : G(g), V(dd_view(c, s)) {
+        xd = V.xd;
+        nd = xd ? G.nx : G.ny;
+        no = xd ? G.ny : G.nx;
+    }
+    __device__ bool range(float ul, float ur, int io, int& k0, int& k1) const {
+        const float oc = cell_cen(no, G.d, io), inv_d = 1.0f / G.d;
+        const float x0 = dd_invert<DD_FAN_FLAT>(G, V, dd_slope<DD_FAN_FLAT>(G, ul), oc);
+        const float x1 = dd_invert<DD_FAN_FLAT>(G, V, dd_slope<DD_FAN_FLAT>(G, ur), oc);
+        const float k0f = fminf(x0, x1) * inv_d + 0.5f * (float)nd, k1f = fmaxf(x0, x1) * inv_d + 0.5f * (float)nd;
+        if (!(k0f < (float)nd + 2.0f) || !(k1f > -2.0f)) return false;
+        k0 = (int)fmaxf(floorf(k0f) - 1.0f, 0.0f);
+        k1 = (int)fminf(floorf(k1f) + 1.0f, (float)(nd - 1));
+        return true;
+    }
+    __device__ void foot(int k, int io, float& lo, float& hi) const {
+        const float oc = cell_cen(no, G.d, io);
+        const float pa = dd_bound<DD_FAN_FLAT>(G, V, cell_bnd(nd, G.d, k), oc);
+        const float pb = dd_bound<DD_FAN_FLAT>(G, V, cell_bnd(nd, G.d, k + 1), oc);
+        lo = fminf(pa, pb);
+        hi = fmaxf(pa, pb);
+    }
+    __device__ float weight(int k, int io, float ul, float ur) const {
+        float lo, hi;
+        foot(k, io, lo, hi);
+        return (fminf(hi, ur) - fmaxf(lo, ul)) * dd_scale<DD_FAN_FLAT>(G, V, cell_cen(no, G.d, io));
+    }
+    __device__ float zmag(int, int io) const { return cone_zmag(G, V, cell_cen(no, G.d, io)); }
+    __host__ __device__ static float fp_unit(const DDGeo& g) { return g.d; }
+    __host__ __device__ static float bp_unit(const DDGeo& g) { return g.dv; }
+};
+
 // One thread per (view, u, v) bin; sino is (na, nu, nv), vol (nx, ny, nz).
 __global__ __launch_bounds__(256) void k_ddcone_fp(DDGeo G, const float* __restrict__ cs,
                                                   const float* __restrict__ sn, const float* __restrict__ vol,
@@ -487,6 +528,16 @@ __global__ __launch_bounds__(256) void k_ddcone_bp(DDGeo G, const float* __restr
     vol[t] = r;
 }
 
+// Slabs a detector row (forward) or rows a slab (backward) can meet, from the
+// magnifications DSD/(DSO + R) and DSD/(DSO - R) of the grid's rim; 0: the
+// tiles do not apply.
+static int ddcone_slots(const DDGeo& G, bool fp, uint32_t flags) {
+    if (flags & VIR_PER_OUTPUT) return 0;
+    const double R = 0.5 * std::sqrt((double)G.nx * G.nx + (double)G.ny * G.ny) * G.d;
+    return fp ? ct_slots((double)G.dv * ((double)G.DSO + R) / ((double)G.DSD * G.d), G.nz)
+              : ct_slots((double)G.d * G.DSD / (((double)G.DSO - R) * G.dv), G.nv);
+}
+
 static int dd_check(const vir_dd_geom* g, DDGeo& G, bool cone) {
     if (!g) return fail_arg("geometry is NULL");
     G.nx = g->nx; G.ny = g->ny; G.nz = cone ? g->nz : 1;
@@ -600,6 +651,9 @@ int vir_ddcone_fp(const vir_dd_geom* geom, const float* cosv, const float* sinv,
                            G, cosv, sinv, vol, sino, (flags & VIR_ACCUMULATE) ? 1 : 0);
         return check_hip(hipGetLastError(), "vir_ddcone_fp launch");
     }
+    if (const int ns = ddcone_slots(G, true, flags))
+        return ct_fp<DDCone>(G, 1, ns, nullptr, cosv, sinv, vol, sino, (flags & VIR_ACCUMULATE) ? 1 : 0,
+                             as_stream(stream), "vir_ddcone_fp launch");
     int64_t n = (int64_t)G.na * G.nu * G.nv;
     hipLaunchKernelGGL(k_ddcone_fp, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, as_stream(stream), G, cosv,
                        sinv, vol, sino, (flags & VIR_ACCUMULATE) ? 1 : 0);
@@ -613,6 +667,9 @@ int vir_ddcone_bp(const vir_dd_geom* geom, const float* cosv, const float* sinv,
     if (rc) return rc;
     if ((G.na > 0 && (!cosv || !sinv || !sino)) || !vol) return fail_arg("NULL pointer argument");
     G.out_scale = out_scale;
+    if (const int ns = ddcone_slots(G, false, flags))
+        return ct_bp<DDCone>(G, 1, ns, nullptr, cosv, sinv, sino, vol, (flags & VIR_ACCUMULATE) ? 1 : 0,
+                             as_stream(stream), "vir_ddcone_bp launch");
     int64_t n = (int64_t)G.nx * G.ny * G.nz;
     hipLaunchKernelGGL(k_ddcone_bp, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, as_stream(stream), G, cosv,
                        sinv, sino, vol, (flags & VIR_ACCUMULATE) ? 1 : 0);

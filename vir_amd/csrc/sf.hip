@@ -25,6 +25,7 @@
 #include <cmath>
 #include <type_traits>
 
+#include "cone_tile.h"
 #include "vir_common.h"
 
 namespace vir {
@@ -119,13 +120,13 @@ __device__ __forceinline__ SFFoot sf_foot(const SFGeo& G, const SFView& V, int i
     const float pxc = (pxl + pxr) * 0.5f, oxc = (oxl + oxr) * 0.5f;
     const float pyc = (pyl + pyr) * 0.5f, oyc = (oyl + oyr) * 0.5f;
     const float den_c = G.DSO - (oxc + oyc);
-    const float uc = G.DSD * (pxc + pyc) / den_c;
-    const float gam = atanf(uc / G.DSD);
     const float fm = G.DSD / den_c;
     float u0 = fm * (pxl + pyl), u1 = fm * (pxr + pyl), u2 = fm * (pxl + pyr), u3 = fm * (pxr + pyr);
     f.u0 = fminf(fminf(u0, u1), fminf(u2, u3));
     f.u1 = fmaxf(fmaxf(u0, u1), fmaxf(u2, u3));
-    f.cm = fm / cosf(gam);
+    // 1/cos of the fan angle atan(t), t = uc/DSD
+    const float t = (pxc + pyc) / den_c;
+    f.cm = fm * __builtin_sqrtf(1.0f + t * t);
     return f;
 }
 
@@ -206,6 +207,45 @@ __device__ __forceinline__ float sf_invert(const SFGeo& G, bool xd, float c, flo
     float t = u / G.DSD;
     return (t * (G.DSO - oo * oc) - po * oc) / (pd + t * od);
 }
+
+// One view of the cone geometry as cone_tile.h's model: weights and ranges of
+// the one-thread-per-output kernels below.
+struct SFCone {
+    static constexpr bool kLineMag = false;
+    const SFGeo& G;
+    SFView V;
+    bool xd;
+    int nd, no;
+    __device__ SFCone(const SFGeo& g, float c, float s, float ang) : G(g), V(sf_view(g, c, s, ang)) {
+        xd = fabsf(s) >= fabsf(c);
+        nd = xd ? G.nx : G.ny;
+        no = xd ? G.ny : G.nx;
+    }
+    __device__ bool range(float ul, float ur, int io, int& k0, int& k1) const {
+        const float oc = (sf_bnd(no, G.d, io) + sf_bnd(no, G.d, io + 1)) * 0.5f, inv_d = 1.0f / G.d;
+        const float x0 = sf_invert<SF_CONE3>(G, xd, V.c, V.s, ul - G.wmax, oc);
+        const float x1 = sf_invert<SF_CONE3>(G, xd, V.c, V.s, ur + G.wmax, oc);
+        const float k0f = fminf(x0, x1) * inv_d + 0.5f * (float)nd - 0.5f;
+        const float k1f = fmaxf(x0, x1) * inv_d + 0.5f * (float)nd - 0.5f;
+        if (!(k0f < (float)nd + 1.0f) || !(k1f > -2.0f)) return false;
+        k0 = (int)fmaxf(floorf(k0f) - 1.0f, 0.0f);
+        k1 = (int)fminf(floorf(k1f) + 2.0f, (float)(nd - 1));
+        return true;
+    }
+    __device__ SFFoot at(int k, int io) const { return sf_foot<SF_CONE3>(G, V, xd ? k : io, xd ? io : k); }
+    __device__ void foot(int k, int io, float& lo, float& hi) const {
+        const SFFoot f = at(k, io);
+        lo = f.u0;
+        hi = f.u1;
+    }
+    __device__ float weight(int k, int io, float ul, float ur) const {
+        const SFFoot f = at(k, io);
+        return ((fminf(f.u1, ur) - fmaxf(f.u0, ul)) * (1.0f / G.du)) * f.amp;
+    }
+    __device__ float zmag(int k, int io) const { return at(k, io).cm; }
+    __host__ __device__ static float fp_unit(const SFGeo& g) { return g.d * (1.0f / g.dv); }
+    __host__ __device__ static float bp_unit(const SFGeo&) { return 1.0f; }
+};
 
 template <int MODE>
 __global__ __launch_bounds__(256) void k_sf_fp(SFGeo G, const float* __restrict__ ang,
@@ -832,6 +872,16 @@ __global__ __launch_bounds__(256) void k_sf_bp(SFGeo G, const float* __restrict_
     img[t] = res;
 }
 
+// Slabs a detector row (forward) or rows a slab (backward) of the cone
+// geometry can meet, from the magnifications at the grid's rim (times 1/cos of
+// the largest fan angle, tan <= R/sqrt(DSO^2 - R^2)); 0: the tiles do not apply.
+static int sf_cone_slots(const SFGeo& G, bool fp, uint32_t flags) {
+    if (flags & VIR_PER_OUTPUT) return 0;
+    const double R = 0.5 * std::sqrt((double)G.nx * G.nx + (double)G.ny * G.ny) * G.d, D = G.DSO;
+    return fp ? ct_slots((double)G.dv * (D + R) / ((double)G.DSD * G.d), G.nz)
+              : ct_slots((double)G.d * G.DSD / (D - R) * (D / std::sqrt(D * D - R * R)) / G.dv, G.nv);
+}
+
 static int sf_setup(const vir_sf_geom* g, SFGeo& G) {
     if (!g) return fail_arg("geometry is NULL");
     if (g->mode < 0 || g->mode > 3) return fail_arg("mode must be 0..3");
@@ -899,7 +949,10 @@ int vir_sf_fp(const vir_sf_geom* geom, const float* ang, const float* cosv, cons
     switch (geom->mode) {
         case SF_PAR2: hipLaunchKernelGGL(k_sf_fp<SF_PAR2>, grd, dim3(256), 0, st, G, ang, cosv, sinv, img, sino, acc); break;
         case SF_FAN2: hipLaunchKernelGGL(k_sf_fp<SF_FAN2>, grd, dim3(256), 0, st, G, ang, cosv, sinv, img, sino, acc); break;
-        case SF_CONE3: hipLaunchKernelGGL(k_sf_fp<SF_CONE3>, grd, dim3(256), 0, st, G, ang, cosv, sinv, img, sino, acc); break;
+        case SF_CONE3:
+            if (const int ns = sf_cone_slots(G, true, flags))
+                return ct_fp<SFCone>(G, G.nb, ns, ang, cosv, sinv, img, sino, acc, st, "vir_sf_fp launch");
+            hipLaunchKernelGGL(k_sf_fp<SF_CONE3>, grd, dim3(256), 0, st, G, ang, cosv, sinv, img, sino, acc); break;
         default:
             if (sf_par3_tiled_ok(G) && !(flags & VIR_PER_OUTPUT)) {
                 const int nut = (G.nu + kTUB - 1) / kTUB, nmt = (G.nv + kTV - 1) / kTV;
@@ -936,7 +989,10 @@ int vir_sf_bp(const vir_sf_geom* geom, const float* ang, const float* cosv, cons
     switch (geom->mode) {
         case SF_PAR2: hipLaunchKernelGGL(k_sf_bp<SF_PAR2>, grd, dim3(256), 0, st, G, ang, cosv, sinv, sino, img, acc); break;
         case SF_FAN2: hipLaunchKernelGGL(k_sf_bp<SF_FAN2>, grd, dim3(256), 0, st, G, ang, cosv, sinv, sino, img, acc); break;
-        case SF_CONE3: hipLaunchKernelGGL(k_sf_bp<SF_CONE3>, grd, dim3(256), 0, st, G, ang, cosv, sinv, sino, img, acc); break;
+        case SF_CONE3:
+            if (const int ns = sf_cone_slots(G, false, flags))
+                return ct_bp<SFCone>(G, G.nb, ns, ang, cosv, sinv, sino, img, acc, st, "vir_sf_bp launch");
+            hipLaunchKernelGGL(k_sf_bp<SF_CONE3>, grd, dim3(256), 0, st, G, ang, cosv, sinv, sino, img, acc); break;
         default:
             if (sf_par3_bp_col_ok(G) && !(flags & VIR_PER_OUTPUT)) {
                 const int nzt = (G.nz + 63) / 64;
