@@ -34,9 +34,9 @@ extern "C" {
 #define VIR_SEQUENTIAL 2u   /* plain sequential f32 sums in reference order */
 #define VIR_UNGUARDED 4u    /* Siddon FP/BP: vir_siddon_count_guarded gave 0
                                for these rays and grid */
-#define VIR_PER_OUTPUT 8u   /* the one-thread-per-output kernels instead of the
-                               tiled ones (DD 2-D and SF: same bits; ray-driven
-                               backprojection: float32 rounding apart) */
+#define VIR_PER_OUTPUT 8u   /* DD, SF and ray-driven BP: the one-thread-per-output
+                               kernels instead of the tiled ones (same sums;
+                               float32 rounding of the weights apart) */
 #define VIR_SF_UNIT_AMPLITUDE 16u  /* SF parallel modes: footprint amplitude 1
                                instead of 1/(|sin|+|cos|) -- the rectangle
                                footprint of fp_2d_par.py:67-125 */
@@ -304,15 +304,15 @@ typedef struct vir_dd_geom {
     float d_pix, du, dv, su, sv, DSO, DSD;
 } vir_dd_geom;
 
-/* sino[a, u] = out_scale * sum_pixels img * overlap * ray_scale, one thread
- * per bin (gather).  The reference's dd_fp_par_2d / dd_fp_fan_2d use
+/* sino[a, u] = out_scale * sum_pixels img * overlap * ray_scale, a gather per
+ * bin in tiles of 128 bins (VIR_PER_OUTPUT: one thread per bin).  The reference's dd_fp_par_2d / dd_fp_fan_2d use
  * out_scale = d_pix/du (dd.py:725, 803). */
 int vir_dd2d_fp(const vir_dd_geom *geom, const float *cosv, const float *sinv,
                 const float *img, float *sino, float out_scale, uint32_t flags,
                 void *stream);
 
-/* Exact transpose of vir_dd2d_fp (same weights), one thread per pixel.  The
- * reference's dd_bp_par_2d / dd_bp_fan_2d use out_scale = 1/(na*d_pix)
+/* Exact transpose of vir_dd2d_fp (same weights), a gather per pixel in tiles
+ * of 16 x 16 pixels (VIR_PER_OUTPUT: one thread per pixel).  The reference's dd_bp_par_2d / dd_bp_fan_2d use out_scale = 1/(na*d_pix)
  * (dd.py:721-722, 799-800); out_scale = d_pix/du gives the exact adjoint. */
 int vir_dd2d_bp(const vir_dd_geom *geom, const float *cosv, const float *sinv,
                 const float *sino, float *img, float out_scale, uint32_t flags,

@@ -18,6 +18,7 @@
 #include <cmath>
 
 #include "cone_tile.h"
+#include "flat_tile.h"
 #include "vir_common.h"
 
 namespace vir {
@@ -100,6 +101,7 @@ __device__ __forceinline__ float dd_invert(const DDGeo& G, const DDView& V, floa
 }
 
 // dd_invert as x = A - oc B for a fixed slope t (the tiled forward's range).
+// The inverse only bounds pixel ranges, which are widened by its rounding.
 template <int MODE>
 __device__ __forceinline__ void dd_invert_lin(const DDGeo& G, const DDView& V, float t, float& A, float& B) {
     if (MODE == DD_PAR) {
@@ -159,126 +161,73 @@ __global__ __launch_bounds__(256) void k_dd2d_fp(DDGeo G, const float* __restric
     sirt_store(E, sino, t, r);
 }
 
-// Tiled forward: one workgroup per (view, 256 bins).  For every orthogonal
-// line the projected boundaries of the pixels that can meet the tile's bins
-// (the union of the per-bin ranges of k_dd2d_fp, widened by one) are
-// evaluated once into LDS with the pixel values, and each bin merges its own
-// pixels from there -- on the equiangular detector that is one atan2 per
-// boundary instead of one per (bin, boundary).  The per-line ray scale and
-// the tile's pixel band are computed once per workgroup, and two lines share
-// each pair of barriers.  Same functions, pixel order and arithmetic as
-// k_dd2d_fp: the same bits.
-constexpr int kDDKMax = 256;    // pixels of one line staged at once (per line of a pair)
-constexpr int kDDLines = 2048;  // lines whose scale and band are tabulated per workgroup
-
+// One view as flat_tile.h's model: pixels share their edges along a line, the
+// ray scale is the line's.  The forward tile adds the terms of k_dd2d_fp in
+// float64 as that kernel does, grouped by wave.
 template <int MODE>
-__global__ __launch_bounds__(256) void k_dd2d_fp_tile(DDGeo G, const float* __restrict__ cs,
-                                                     const float* __restrict__ sn, const float* __restrict__ img,
-                                                     float* __restrict__ sino, int accumulate, int nut, SirtEpi E) {
-    __shared__ float bnd[2][kDDKMax + 1];  // projected boundary kc + e of the two lines
-    __shared__ float val[2][kDDKMax];      // pixel kc + e
-    // per-line tables sized by the launch to max(nx, ny) lines (<= kDDLines):
-    // 8 bytes a line, so small images keep more workgroups resident
-    extern __shared__ float dyn_lds[];
-    float* lsc = dyn_lds;                                                        // ray scale of line io
-    short2* lband = reinterpret_cast<short2*>(dyn_lds + max(G.nx, G.ny));  // the tile's pixel band of line io (empty: y < x)
-    const int ut = blockIdx.x % nut, ia = blockIdx.x / nut;
-    const int u_lo = ut * 256, u_n = min(256, G.nu - u_lo);
-    const int iu = u_lo + (int)threadIdx.x;
-    const bool ubin = (int)threadIdx.x < u_n;
-    const DDView V = dd_view(cs[ia], sn[ia]);
-    const int nd = V.xd ? G.nx : G.ny, no = V.xd ? G.ny : G.nx;
-    const float ul = det_bnd(G.nu, G.du, G.su, iu), ur = det_bnd(G.nu, G.du, G.su, iu + 1);
-    const float tl = dd_slope<MODE>(G, ul), tr = dd_slope<MODE>(G, ur);
-    // dd_invert(t, oc) = A(t) - oc B(t): its denominator depends on the bin
-    // only.  The inverse only bounds the pixel range, which is widened by a
-    // pixel, so this rounding (~1e-5 pixel) leaves the range covering every
-    // pixel of positive overlap and the sum unchanged.
-    float Al, Bl, Ar, Br;
-    dd_invert_lin<MODE>(G, V, tl, Al, Bl);
-    dd_invert_lin<MODE>(G, V, tr, Ar, Br);
-    const float tt0 = dd_slope<MODE>(G, det_bnd(G.nu, G.du, G.su, u_lo));
-    const float tt1 = dd_slope<MODE>(G, det_bnd(G.nu, G.du, G.su, u_lo + u_n));
-    const float inv_d = 1.0f / G.d;
-    // per-line table (host guarantees no <= kDDLines)
-    for (int io = threadIdx.x; io < no; io += 256) {
-        const float oc = cell_cen(no, G.d, io);
-        const float y0 = dd_invert<MODE>(G, V, tt0, oc), y1 = dd_invert<MODE>(G, V, tt1, oc);
-        const float t0f = fminf(y0, y1) * inv_d + 0.5f * (float)nd;
-        const float t1f = fmaxf(y0, y1) * inv_d + 0.5f * (float)nd;
-        short2 bandv = make_short2(0, -1);  // pixel indices < kDDLines fit 16 bits
-        if (t0f < (float)nd + 3.0f && t1f > -3.0f) {
-            bandv.x = (short)fmaxf(floorf(t0f) - 2.0f, 0.0f);
-            bandv.y = (short)fminf(floorf(t1f) + 2.0f, (float)(nd - 1));
+struct DDFlat {
+    static constexpr int kFixed = 3;
+    static constexpr bool kShared = true, kCentre = false;
+    struct Trig {
+        float c, s;
+        __device__ Trig(float c_, float s_, float) : c(c_), s(s_) {}
+        __device__ Trig lane(int l) const { return Trig(ft_lane(c, l), ft_lane(s, l), 0.0f); }
+    };
+    const DDGeo& G;
+    DDView V;
+    bool xd;
+    int nd, no;
+    float tmax;  // slope of the rays that touch the grid's circle
+    __device__ DDFlat(const DDGeo& g, const Trig& t) : G(g), V(dd_view(t.c, t.s)) {
+        xd = V.xd;
+        nd = xd ? G.nx : G.ny;
+        no = xd ? G.ny : G.nx;
+        if (MODE != DD_PAR) {
+            const float r2 = 0.25f * G.d * G.d * ((float)G.nx * (float)G.nx + (float)G.ny * (float)G.ny);
+            tmax = 1.01f * sqrtf(r2 / fmaxf(G.DSO * G.DSO - r2, 1e-6f * r2)) + 1e-3f;
         }
-        lband[io] = bandv;
-        lsc[io] = dd_scale<MODE>(G, V, oc);
     }
-    __syncthreads();
-    // stage boundaries and values of pixels kc .. kc + nk - 1 of line io into slot h
-    auto stage = [&](int h, int io, int kc, int nk) {
-        const float oc = cell_cen(no, G.d, io);
-        for (int e = threadIdx.x; e <= nk; e += 256) {
-            bnd[h][e] = dd_bound<MODE>(G, V, cell_bnd(nd, G.d, kc + e), oc);
-            if (e < nk) {
-                const int k = kc + e;
-                const int ix = V.xd ? k : io, iy = V.xd ? io : k;
-                val[h][e] = img[(int64_t)ix * G.ny + iy];
-            }
-        }
-    };
-    double acc = 0.0;
-    // this bin's pixels of line io within the staged chunk, as k_dd2d_fp
-    auto merge = [&](int h, int io, int kc, int nk) {
-        const float oc = cell_cen(no, G.d, io);
-        const float x0 = __builtin_fmaf(-oc, Bl, Al), x1 = __builtin_fmaf(-oc, Br, Ar);
-        const float k0f = fminf(x0, x1) * inv_d + 0.5f * (float)nd;
-        const float k1f = fmaxf(x0, x1) * inv_d + 0.5f * (float)nd;
-        if (!(k0f < (float)nd + 2.0f) || !(k1f > -2.0f)) return;
-        const int k0 = (int)fmaxf(floorf(k0f) - 1.0f, 0.0f);
-        const int k1 = (int)fminf(floorf(k1f) + 1.0f, (float)(nd - 1));
-        const float sc = lsc[io];
-        const int ka = max(k0, kc), kz = min(k1, kc + nk - 1);
-        for (int k = ka; k <= kz; ++k) {
-            const float ov = overlap(bnd[h][k - kc], bnd[h][k - kc + 1], ul, ur);
-            if (ov > 0.0f) acc += (double)(val[h][k - kc] * (ov * sc));
-        }
-    };
-    for (int io0 = 0; io0 < no; io0 += 2) {
-        const short2 s0 = lband[io0];
-        const short2 s1 = io0 + 1 < no ? lband[io0 + 1] : make_short2(0, -1);
-        const int2 b0 = make_int2(s0.x, s0.y), b1 = make_int2(s1.x, s1.y);
-        const int n0 = b0.y - b0.x + 1, n1 = b1.y - b1.x + 1;
-        if (n0 <= 0 && n1 <= 0) continue;
-        if (n0 <= kDDKMax && n1 <= kDDKMax) {
-            // both lines in one chunk each: one pair of barriers for two lines
-            __syncthreads();
-            if (n0 > 0) stage(0, io0, b0.x, n0);
-            if (n1 > 0) stage(1, io0 + 1, b1.x, n1);
-            __syncthreads();
-            if (ubin && n0 > 0) merge(0, io0, b0.x, n0);
-            if (ubin && n1 > 0) merge(1, io0 + 1, b1.x, n1);
-            continue;
-        }
-        // a long band: each line on its own, chunk by chunk
+    __device__ float centre(int io) const { return cell_cen(no, G.d, io); }
+    // bins past the grid's shadow are inverted at its rim (the inverse turns
+    // over at 45 degrees, and they meet no pixel)
+    __device__ void lin(float u, float& A, float& B) const {
+        float t = dd_slope<MODE>(G, u);
+        if (MODE == DD_FAN_ARC && fabsf(u) > 1.5f * G.DSD) t = u > 0.0f ? tmax : -tmax;
+        if (MODE != DD_PAR) t = fminf(fmaxf(t, -tmax), tmax);
+        dd_invert_lin<MODE>(G, V, t, A, B);
+    }
+    __device__ float margin() const { return 0.0f; }
+    __device__ float line_factor(float oc) const { return dd_scale<MODE>(G, V, oc); }
+    __device__ float edge(int k, float oc) const { return dd_bound<MODE>(G, V, cell_bnd(nd, G.d, k), oc); }
+    // pixel (ix + i, iy + j) at 2 i + j: the block's two lines hold three
+    // edges each
+    __device__ void quad(int ix, int iy, float* lo, float* hi, float* f) const {
+        const int k = xd ? ix : iy, io = xd ? iy : ix;
+        float l[2][2], h[2][2], sc[2];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int2 bb = h ? b1 : b0;
-            for (int kc = bb.x; kc <= bb.y; kc += kDDKMax) {
-                const int nk = min(kDDKMax, bb.y - kc + 1);
-                __syncthreads();
-                stage(0, io0 + h, kc, nk);
-                __syncthreads();
-                if (ubin) merge(0, io0 + h, kc, nk);
+        for (int t = 0; t < 2; ++t) {
+            const float oc = cell_cen(no, G.d, io + t);
+            sc[t] = dd_scale<MODE>(G, V, oc);
+            float b[3];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) b[i] = dd_bound<MODE>(G, V, cell_bnd(nd, G.d, k + i), oc);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                l[t][i] = fminf(b[i], b[i + 1]);
+                h[t][i] = fmaxf(b[i], b[i + 1]);
             }
         }
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                lo[2 * i + j] = xd ? l[j][i] : l[i][j];
+                hi[2 * i + j] = xd ? h[j][i] : h[i][j];
+                f[2 * i + j] = xd ? sc[j] : sc[i];
+            }
     }
-    if (!ubin) return;
-    const int64_t t = (int64_t)ia * G.nu + iu;
-    float r = (float)acc * G.out_scale;
-    if (accumulate) r += sino[t];
-    sirt_store(E, sino, t, r);
-}
+    __host__ __device__ static float bp_unit(const DDGeo& g) { return g.du; }
+};
 
 // One thread per pixel.
 template <int MODE>
@@ -574,16 +523,12 @@ static int dd2d_fp(const vir_dd_geom* geom, const float* cosv, const float* sinv
     dim3 grd((unsigned)((n + 255) / 256));
     int acc = (flags & VIR_ACCUMULATE) ? 1 : 0;
     hipStream_t st = as_stream(stream);
-    if (!(flags & VIR_PER_OUTPUT) && std::max(G.nx, G.ny) <= kDDLines) {
-        const int nut = (G.nu + 255) / 256;
-        dim3 tg((unsigned)((int64_t)G.na * nut));
-        const size_t tables = (size_t)std::max(G.nx, G.ny) * (sizeof(float) + sizeof(short2));
+    if (!(flags & VIR_PER_OUTPUT)) {
         if (geom->mode == DD_PAR)
-            hipLaunchKernelGGL(k_dd2d_fp_tile<DD_PAR>, tg, dim3(256), tables, st, G, cosv, sinv, img, sino, acc, nut, E);
-        else if (geom->mode == DD_FAN_FLAT)
-            hipLaunchKernelGGL(k_dd2d_fp_tile<DD_FAN_FLAT>, tg, dim3(256), tables, st, G, cosv, sinv, img, sino, acc, nut, E);
-        else hipLaunchKernelGGL(k_dd2d_fp_tile<DD_FAN_ARC>, tg, dim3(256), tables, st, G, cosv, sinv, img, sino, acc, nut, E);
-        return check_hip(hipGetLastError(), "vir_dd2d_fp launch");
+            return ft_fp<DDFlat<DD_PAR>>(G, 1, nullptr, cosv, sinv, img, sino, acc, st, E, "vir_dd2d_fp launch");
+        if (geom->mode == DD_FAN_FLAT)
+            return ft_fp<DDFlat<DD_FAN_FLAT>>(G, 1, nullptr, cosv, sinv, img, sino, acc, st, E, "vir_dd2d_fp launch");
+        return ft_fp<DDFlat<DD_FAN_ARC>>(G, 1, nullptr, cosv, sinv, img, sino, acc, st, E, "vir_dd2d_fp launch");
     }
     if (geom->mode == DD_PAR) hipLaunchKernelGGL(k_dd2d_fp<DD_PAR>, grd, dim3(256), 0, st, G, cosv, sinv, img, sino, acc, E);
     else if (geom->mode == DD_FAN_FLAT)
@@ -604,6 +549,13 @@ static int dd2d_bp(const vir_dd_geom* geom, const float* cosv, const float* sinv
     dim3 grd((unsigned)((n + 255) / 256));
     int acc = (flags & VIR_ACCUMULATE) ? 1 : 0;
     hipStream_t st = as_stream(stream);
+    if (!(flags & VIR_PER_OUTPUT)) {
+        if (geom->mode == DD_PAR)
+            return ft_bp<DDFlat<DD_PAR>>(G, 1, nullptr, cosv, sinv, sino, img, acc, st, E, "vir_dd2d_bp launch");
+        if (geom->mode == DD_FAN_FLAT)
+            return ft_bp<DDFlat<DD_FAN_FLAT>>(G, 1, nullptr, cosv, sinv, sino, img, acc, st, E, "vir_dd2d_bp launch");
+        return ft_bp<DDFlat<DD_FAN_ARC>>(G, 1, nullptr, cosv, sinv, sino, img, acc, st, E, "vir_dd2d_bp launch");
+    }
     if (geom->mode == DD_PAR) hipLaunchKernelGGL(k_dd2d_bp<DD_PAR>, grd, dim3(256), 0, st, G, cosv, sinv, sino, img, acc, E);
     else if (geom->mode == DD_FAN_FLAT)
         hipLaunchKernelGGL(k_dd2d_bp<DD_FAN_FLAT>, grd, dim3(256), 0, st, G, cosv, sinv, sino, img, acc, E);

@@ -26,6 +26,7 @@
 #include <type_traits>
 
 #include "cone_tile.h"
+#include "flat_tile.h"
 #include "vir_common.h"
 
 namespace vir {
@@ -54,16 +55,18 @@ struct SFFoot {
 
 // Per-view constants.
 struct SFView {
-    float c, s, ang;
-    float amp;  // 1/(|sin| + |cos|)
-    float h;    // half the projected width of a pixel in parallel beam
+    float c, s;
+    float ca, sa;  // cosine and sine of the float32 angle (fan amplitude)
+    float amp;     // 1/(|sin| + |cos|)
+    float h;       // half the projected width of a pixel in parallel beam
 };
 
 __device__ __forceinline__ SFView sf_view(const SFGeo& G, float c, float s, float ang) {
     SFView V;
     V.c = c;
     V.s = s;
-    V.ang = ang;
+    V.ca = cosf(ang);
+    V.sa = sinf(ang);
     const float w = fabsf(s) + fabsf(c);
     V.amp = G.unit_amp ? 1.0f : 1.0f / w;
     V.h = 0.5f * G.d * w;
@@ -72,17 +75,17 @@ __device__ __forceinline__ SFView sf_view(const SFGeo& G, float c, float s, floa
 
 // Fan amplitude 1/(|cos(a+g)| + |sin(a+g)|) of pixel (ix, iy), g the angle
 // of the ray through its centre, whose o coordinate takes the pixel's lower
-// y boundary at boundary ky (ky = iy: the pixel's own).
+// y boundary at boundary ky (ky = iy: the pixel's own).  With t = tan g it is
+// sqrt(1 + t^2) / (|cos a - t sin a| + |sin a + t cos a|): no trigonometry per
+// pixel, and no rounding of a + g.
 __device__ __forceinline__ float sf_fan_amp(const SFGeo& G, const SFView& V, int ix, int iy, int ky) {
     const float c = V.c, s = V.s;
     const float xl = sf_bnd(G.nx, G.d, ix), xr = sf_bnd(G.nx, G.d, ix + 1);
     const float yl = sf_bnd(G.ny, G.d, iy), yr = sf_bnd(G.ny, G.d, iy + 1);
     const float pxc = (-s * xl + -s * xr) * 0.5f, oxc = (c * xl + c * xr) * 0.5f;
     const float pyc = (c * yl + c * yr) * 0.5f, oyc = (s * sf_bnd(G.ny, G.d, ky) + s * yr) * 0.5f;
-    const float uc = G.DSD * (pxc + pyc) / (G.DSO - (oxc + oyc));
-    const float gam = atanf(uc / G.DSD);
-    const float rx = cosf(V.ang + gam), ry = sinf(V.ang + gam);
-    return 1.0f / (fabsf(rx) + fabsf(ry));
+    const float t = (pxc + pyc) / (G.DSO - (oxc + oyc));
+    return __builtin_sqrtf(1.0f + t * t) / (fabsf(V.ca - t * V.sa) + fabsf(V.sa + t * V.ca));
 }
 
 // Footprint of pixel (ix, iy) in view V.  In parallel beam the four
@@ -207,6 +210,88 @@ __device__ __forceinline__ float sf_invert(const SFGeo& G, bool xd, float c, flo
     float t = u / G.DSD;
     return (t * (G.DSO - oo * oc) - po * oc) / (pd + t * od);
 }
+
+// One view of the 2-D geometries as flat_tile.h's model.  The forward tile
+// adds the terms of k_sf_fp in float64 as that kernel does, grouped by wave.
+template <int MODE>
+struct SFFlat {
+    static constexpr int kFixed = 4;
+    static constexpr bool kShared = false, kCentre = true;
+    struct Trig {
+        SFView V;
+        __device__ Trig(float c, float s, float ang) {
+            V.c = c;
+            V.s = s;
+            V.ca = MODE == SF_FAN2 ? cosf(ang) : 0.0f;
+            V.sa = MODE == SF_FAN2 ? sinf(ang) : 0.0f;
+        }
+        __device__ Trig lane(int l) const {
+            Trig t = *this;
+            t.V.c = ft_lane(V.c, l);
+            t.V.s = ft_lane(V.s, l);
+            t.V.ca = ft_lane(V.ca, l);
+            t.V.sa = ft_lane(V.sa, l);
+            return t;
+        }
+    };
+    const SFGeo& G;
+    SFView V;
+    bool xd;
+    int nd, no;
+    __device__ SFFlat(const SFGeo& g, const Trig& t) : G(g), V(t.V) {
+        const float w = fabsf(V.s) + fabsf(V.c);
+        V.amp = G.unit_amp ? 1.0f : 1.0f / w;
+        V.h = 0.5f * G.d * w;
+        xd = fabsf(V.s) >= fabsf(V.c);
+        nd = xd ? G.nx : G.ny;
+        no = xd ? G.ny : G.nx;
+    }
+    __device__ float centre(int io) const { return (sf_bnd(no, G.d, io) + sf_bnd(no, G.d, io + 1)) * 0.5f; }
+    __device__ void lin(float u, float& A, float& B) const {
+        const float pd = xd ? -V.s : V.c, po = xd ? V.c : -V.s;
+        const float od = xd ? V.c : V.s, oo = xd ? V.s : V.c;
+        const float t = MODE == SF_PAR2 ? u : u / G.DSD, r = 1.0f / (MODE == SF_PAR2 ? pd : pd + t * od);
+        A = MODE == SF_PAR2 ? t * r : t * G.DSO * r;
+        B = MODE == SF_PAR2 ? po * r : (t * oo + po) * r;
+    }
+    __device__ float margin() const { return G.wmax; }
+    __device__ float line_factor(float) const { return 1.0f / G.du; }
+    __device__ float pixel(int k, int io, float& u0, float& u1) const {
+        const SFFoot f = sf_foot<MODE>(G, V, xd ? k : io, xd ? io : k);
+        u0 = f.u0;
+        u1 = f.u1;
+        return f.amp;
+    }
+    __device__ float corner(int ix, int iy) const {
+        const float x = sf_bnd(G.nx, G.d, ix), y = sf_bnd(G.ny, G.d, iy);
+        return G.DSD * (-V.s * x + V.c * y) / (G.DSO - (V.c * x + V.s * y));
+    }
+    // pixel (ix + i, iy + j) at 2 i + j; a fan block has nine corners
+    __device__ void quad(int ix, int iy, float* lo, float* hi, float* f) const {
+        float p[3][3];
+        if (MODE == SF_FAN2) {
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+#pragma unroll
+                for (int j = 0; j < 3; ++j) p[i][j] = corner(ix + i, iy + j);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int i = q >> 1, j = q & 1;
+            if (MODE == SF_PAR2) {
+                const SFFoot t = sf_foot<SF_PAR2>(G, V, ix + i, iy + j);
+                lo[q] = t.u0;
+                hi[q] = t.u1;
+                f[q] = t.amp;
+                continue;
+            }
+            lo[q] = fminf(fminf(p[i][j], p[i + 1][j]), fminf(p[i][j + 1], p[i + 1][j + 1]));
+            hi[q] = fmaxf(fmaxf(p[i][j], p[i + 1][j]), fmaxf(p[i][j + 1], p[i + 1][j + 1]));
+            f[q] = sf_fan_amp(G, V, ix + i, iy + j, iy + j);
+        }
+    }
+    __host__ __device__ static float bp_unit(const SFGeo&) { return 1.0f; }
+};
 
 // One view of the cone geometry as cone_tile.h's model: weights and ranges of
 // the one-thread-per-output kernels below.
@@ -946,6 +1031,12 @@ int vir_sf_fp(const vir_sf_geom* geom, const float* ang, const float* cosv, cons
     dim3 grd((unsigned)((n + 255) / 256));
     hipStream_t st = as_stream(stream);
     int acc = (flags & VIR_ACCUMULATE) ? 1 : 0;
+    // VIR_COMPAT's amplitudes depend on the pixels before: the gather looks back
+    const bool flat = !G.compat && !(flags & VIR_PER_OUTPUT);
+    if (flat && geom->mode == SF_PAR2)
+        return ft_fp<SFFlat<SF_PAR2>>(G, G.nb, ang, cosv, sinv, img, sino, acc, st, SirtEpi{}, "vir_sf_fp launch");
+    if (flat && geom->mode == SF_FAN2)
+        return ft_fp<SFFlat<SF_FAN2>>(G, G.nb, ang, cosv, sinv, img, sino, acc, st, SirtEpi{}, "vir_sf_fp launch");
     switch (geom->mode) {
         case SF_PAR2: hipLaunchKernelGGL(k_sf_fp<SF_PAR2>, grd, dim3(256), 0, st, G, ang, cosv, sinv, img, sino, acc); break;
         case SF_FAN2: hipLaunchKernelGGL(k_sf_fp<SF_FAN2>, grd, dim3(256), 0, st, G, ang, cosv, sinv, img, sino, acc); break;
@@ -986,6 +1077,11 @@ int vir_sf_bp(const vir_sf_geom* geom, const float* ang, const float* cosv, cons
     dim3 grd((unsigned)((n + 255) / 256));
     hipStream_t st = as_stream(stream);
     int acc = (flags & VIR_ACCUMULATE) ? 1 : 0;
+    const bool flat = !(flags & VIR_PER_OUTPUT);
+    if (flat && geom->mode == SF_PAR2)
+        return ft_bp<SFFlat<SF_PAR2>>(G, G.nb, ang, cosv, sinv, sino, img, acc, st, SirtEpi{}, "vir_sf_bp launch");
+    if (flat && geom->mode == SF_FAN2)
+        return ft_bp<SFFlat<SF_FAN2>>(G, G.nb, ang, cosv, sinv, sino, img, acc, st, SirtEpi{}, "vir_sf_bp launch");
     switch (geom->mode) {
         case SF_PAR2: hipLaunchKernelGGL(k_sf_bp<SF_PAR2>, grd, dim3(256), 0, st, G, ang, cosv, sinv, sino, img, acc); break;
         case SF_FAN2: hipLaunchKernelGGL(k_sf_bp<SF_FAN2>, grd, dim3(256), 0, st, G, ang, cosv, sinv, sino, img, acc); break;
