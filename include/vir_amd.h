@@ -580,6 +580,15 @@ int vir_tv_chambolle(int32_t ndim, int32_t nx, int32_t ny, int32_t nz,
                      const float *g, float *q, float *v, float *u, float weight,
                      float tau, int32_t iters, float *dmax, void *stream);
 
+/* The iterations of vir_tv_chambolle (images of 2 or 3 axes, same bits) on two
+ * copies of q, several per pass over memory: *cur (0 or 1) says which of q0, q1
+ * holds q, on entry and on return.  q must be zero at each axis' last index, as
+ * from the start value 0 it stays.  dmax as above. */
+int vir_tv_chambolle_pair(int32_t ndim, int32_t nx, int32_t ny, int32_t nz,
+                          const float *g, float *q0, float *q1, int32_t *cur,
+                          float weight, float tau, int32_t iters, float *dmax,
+                          void *stream);
+
 /* Chambolle-Pock iteration for TV-regularised reconstruction (tv.py:229-294),
  * on volumes (nx, ny, nz) with periodic differences (tv.py:207-224); nz == 1
  * is 2-D.  z holds ndim (2 or 3) planes of the volume's size.

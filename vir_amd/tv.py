@@ -10,6 +10,8 @@ vir_tv_chambolle kernels.
 pdhg_tv: the Chambolle-Pock reconstruction of tv.py:229-294 over any
 projector.
 """
+import ctypes
+
 import numpy as np
 import torch
 
@@ -41,20 +43,36 @@ def denoise_tv_chambolle(image, weight=0.1, eps=2.0e-4, max_num_iter=200, tau=No
     dims = shape + (1,) * (3 - nd)
     tau = 1.0 / (4.0 * nd) if tau is None else float(tau)
     q = torch.zeros((nd,) + shape, dtype=torch.float32, device=g.device)
-    v = torch.empty_like(g)
     u = torch.empty_like(g)
+    # a second copy of q lets a pass over memory do several iterations; where
+    # there is no room for it, one residual image does
+    q2 = v = None
+    if nd > 1:
+        try:
+            q2 = torch.empty_like(q)
+        except torch.OutOfMemoryError:
+            pass
+    if q2 is None:
+        v = torch.empty_like(g)
+    cur = ctypes.c_int32(0)
     dmax = torch.empty(TV_WORK, dtype=torch.float32, device=g.device)
     L = _lib.lib()
     done = 0
     while done < max_num_iter:
         k = min(int(check_every), int(max_num_iter) - done)
-        _lib.check(L.vir_tv_chambolle(nd, dims[0], dims[1], dims[2], _lib.ptr(g), _lib.ptr(q), _lib.ptr(v),
-                                      None, float(weight), tau, k, _lib.ptr(dmax) if eps > 0 else None,
-                                      stream()), "vir_tv_chambolle")
+        dm = _lib.ptr(dmax) if eps > 0 else None
+        if q2 is not None:
+            _lib.check(L.vir_tv_chambolle_pair(nd, dims[0], dims[1], dims[2], _lib.ptr(g), _lib.ptr(q), _lib.ptr(q2),
+                                               ctypes.addressof(cur), float(weight), tau, k, dm, stream()),
+                       "vir_tv_chambolle_pair")
+        else:
+            _lib.check(L.vir_tv_chambolle(nd, dims[0], dims[1], dims[2], _lib.ptr(g), _lib.ptr(q), _lib.ptr(v),
+                                          None, float(weight), tau, k, dm, stream()), "vir_tv_chambolle")
         done += k
         if eps > 0 and float(dmax[0]) <= eps * weight:
             break
-    _lib.check(L.vir_tv_chambolle(nd, dims[0], dims[1], dims[2], _lib.ptr(g), _lib.ptr(q), _lib.ptr(v),
+    q = q2 if cur.value else q
+    _lib.check(L.vir_tv_chambolle(nd, dims[0], dims[1], dims[2], _lib.ptr(g), _lib.ptr(q), None,
                                   _lib.ptr(u), float(weight), tau, 0, None, stream()), "vir_tv_chambolle")
     return u if torch_in else u.cpu().numpy()
 
