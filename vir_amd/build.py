@@ -8,6 +8,9 @@ Every HIP translation unit is compiled with:
                                must round exactly as numpy's separate ops
   -Xclang -target-feature -Xclang -packed-fp32-ops
                                keep the compiler from emitting packed FP32 ops
+  -mllvm -amdgpu-mfma-vgpr-form=1
+                               matrix accumulators stay in VGPRs (copies to and
+                               from AGPRs cost a float64 product 60 % more time)
 """
 import os
 import subprocess
@@ -24,6 +27,7 @@ SOURCES = ["vir_common.hip", "siddon.hip", "csr.hip", "sirt_ops.hip", "dd.hip", 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["-O3", "-std=c++17", "--offload-arch=gfx950", "-fPIC", "-ffp-contract=off",
          "-fno-fast-math", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+         "-mllvm", "-amdgpu-mfma-vgpr-form=1",
          "-Wall", "-Wno-unused-function", "-Wno-unused-variable",
          "-I" + os.path.join(HERE, "..", "include")]
 

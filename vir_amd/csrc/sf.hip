@@ -392,7 +392,7 @@ __global__ __launch_bounds__(256) void k_sf_fp(SFGeo G, const float* __restrict_
 #pragma unroll
                 for (int q = 0; q < kSlabs; ++q)
                     if (SW.w[q] > 0.0f) sv_ += col[SW.first + q] * SW.w[q];
-                acc += (double)(wu * sv_);
+                acc = __builtin_fma((double)wu, (double)sv_, acc);
             } else {
                 // slabs whose magnified z interval meets [vl, vr]
                 float z0f = fminf(vl, vr) / f.cm * inv_d + 0.5f * (float)G.nz;
@@ -678,12 +678,12 @@ __global__ __launch_bounds__(64 * kVG) __attribute__((amdgpu_waves_per_eu(6))) v
                             const int2 e0 = wl[j], e1 = wl[j + 1];
                             const float p0 = R[e0.x + lane];
                             const float p1 = R[e1.x + lane];
-                            acc[i] += (double)(__int_as_float(e0.y) * p0);
-                            acc[i] += (double)(__int_as_float(e1.y) * p1);
+                            acc[i] = __builtin_fma((double)__int_as_float(e0.y), (double)p0, acc[i]);
+                            acc[i] = __builtin_fma((double)__int_as_float(e1.y), (double)p1, acc[i]);
                         }
                         if (j < cnt) {
                             const int2 e0 = wl[j];
-                            acc[i] += (double)(__int_as_float(e0.y) * R[e0.x + lane]);
+                            acc[i] = __builtin_fma((double)__int_as_float(e0.y), (double)R[e0.x + lane], acc[i]);
                         }
                     }
                 }
@@ -842,7 +842,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
                         for (int q = 0; q < kSlabs; ++q)
                             if (q < nzr) sv_ += row[rq[q]] * rw[q];
                     }
-                    acc += (double)(wu * sv_);
+                    acc = __builtin_fma((double)wu, (double)sv_, acc);
                 }
             }
         }
@@ -856,6 +856,196 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
     float res = (float)acc * G.out_scale;
     if (accumulate) res += img[o];
     img[o] = res;
+}
+
+// ------------------------------- parallel 3-D backward on the matrix cores
+//
+// Rows aligned with the slabs (slab z meets row z + shift only): a block of 4 x
+// 4 pixels backprojects a view as the product of its 16 x 4 KS footprint
+// weights and 4 KS sinogram rows, in float64 (v_mfma_f64_16x16x4_f64: exact
+// products of the float32 weights and values, float64 sums).  A lane evaluates
+// the weights that its operand slot needs -- pixel lane % 16, bin jb + 4 kk +
+// lane / 16 -- so there are no lists and no broadcasts, and a row is read once
+// for sixteen pixels.  Four accumulators cover 64 slabs.  The column kernel
+// above spends 184 cycles a pixel column and view on broadcasts, loads and sums
+// (7.0 ms for 8 x 256 x 256 x 64, 180 views of 384); this one 55 (2.1 ms), of
+// which 36 are the product's, a third of it on non-zero weights.
+//
+// Zero weights times infinite values make NaNs: where a sum is not finite, the
+// wave's pixels are done again bin by bin.
+typedef double sf_d4 __attribute__((ext_vector_type(4)));
+
+// One voxel (pixel (ix, iy), row m, weight rw of its slab) by the gather.
+__device__ double sf_bp_par3_one(const SFGeo& G, const float* __restrict__ cs, const float* __restrict__ sn,
+                                 const float* __restrict__ sb, int ix, int iy, int m, float rw) {
+    double acc = 0.0;
+    if (!(rw > 0.0f)) return acc;
+    const float u0 = sf_det(G.nu, G.du, G.su, 0), inv_du = 1.0f / G.du;
+    for (int ia = 0; ia < G.na; ++ia) {
+        const SFView V = sf_view(G, cs[ia], sn[ia], 0.0f);
+        const SFFoot f = sf_foot<SF_PAR3>(G, V, ix, iy);
+        if (!(f.u1 > u0 - G.du) || !((f.u0 - u0) * inv_du < (float)G.nu + 1.0f)) continue;
+        const int j0 = (int)fmaxf(floorf((f.u0 - u0) * inv_du) - 1.0f, 0.0f);
+        const int j1 = (int)fminf(floorf((f.u1 - u0) * inv_du) + 1.0f, (float)(G.nu - 1));
+        for (int j = j0; j <= j1; ++j) {
+            const float ou = ovl(f.u0, f.u1, sf_det(G.nu, G.du, G.su, j), sf_det(G.nu, G.du, G.su, j + 1));
+            if (ou > 0.0f)
+                acc = __builtin_fma((double)((ou * inv_du) * f.amp),
+                                    (double)(sb[((int64_t)ia * G.nu + j) * G.nv + m] * rw), acc);
+        }
+    }
+    return acc;
+}
+
+// SPLIT: the four waves of a block share one pixel block's views (few blocks)
+// and add their sums in wave order; else each takes a block of its own.
+template <int KS, bool SPLIT>
+__global__ __launch_bounds__(256) void k_sf_bp_par3_mfma(SFGeo G, const float* __restrict__ cs,
+                                                        const float* __restrict__ sn,
+                                                        const float* __restrict__ sino, float* __restrict__ img,
+                                                        int accumulate, int nby, int nbx, int nzt, int shift,
+                                                        int64_t nblk) {
+    __shared__ double red[SPLIT ? 4 : 1][SPLIT ? 1024 : 1];
+    const int lane = threadIdx.x & 63, lo = lane & 15, hi = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t blk = xcd_remap(blockIdx.x, gridDim.x);
+    int64_t wid = SPLIT ? blk : blk * 4 + wave;
+    if (wid >= nblk) return;  // whole wave (SPLIT: whole block)
+    const int zb = (int)(wid % nzt) * 64;
+    wid /= nzt;
+    const int by = (int)(wid % nby) * 4;
+    wid /= nby;
+    const int bx = (int)(wid % nbx) * 4;
+    const int b = (int)(wid / nbx);
+    const float* __restrict__ sb = sino + (int64_t)b * G.na * G.nu * G.nv;
+    const float inv_du = 1.0f / G.du, inv_dv = 1.0f / G.dv, half = 0.5f * (float)G.nu;
+    // slabs z = zb + 16 zg + lo: their row and its weight
+    const int nzg = min(4, (G.nz - zb + 15) / 16);
+    int off[4];
+    float rw[4];
+#pragma unroll
+    for (int zg = 0; zg < 4; ++zg) {
+        const int z = zb + 16 * zg + lo, m = z + shift;
+        off[zg] = hi * G.nv + min(max(m, 0), G.nv - 1);
+        const float ov = sf_bnd(G.nz, G.d, z + 1) - sf_bnd(G.nz, G.d, z);
+        rw[zg] = z < G.nz && m >= 0 && m < G.nv ? ov * inv_dv : 0.0f;
+    }
+    // weights: pixel (bx + lo / 4, by + lo % 4)
+    const float xc = G.d * (((float)(bx + (lo >> 2)) + 0.5f) - 0.5f * (float)G.nx);
+    const float yc = G.d * (((float)(by + (lo & 3)) + 0.5f) - 0.5f * (float)G.ny);
+    const float xm = G.d * ((float)(bx + 2) - 0.5f * (float)G.nx), ym = G.d * ((float)(by + 2) - 0.5f * (float)G.ny);
+    const float eps = 0.01f + 1e-6f * (float)G.nu;
+    sf_d4 acc[4];
+#pragma unroll
+    for (int zg = 0; zg < 4; ++zg) acc[zg] = sf_d4{0.0, 0.0, 0.0, 0.0};
+    const int vstep = SPLIT ? 4 : 1, vfirst = SPLIT ? wave : 0;
+    for (int g = vfirst; g < G.na; g += 64 * vstep) {
+        // lane = view g + vstep lane: its constants and the block's first bin
+        const int il = min(g + vstep * lane, G.na - 1);
+        const SFView L = sf_view(G, cs[il], sn[il], 0.0f);
+        const float lf = (-L.s * xm + L.c * ym - 4.0f * L.h) * inv_du - G.su + half;
+        const int jl = (int)fminf(fmaxf(floorf(lf - eps), 0.0f), (float)(G.nu - 4 * KS));
+        const int nl = min(64, (G.na - g + vstep - 1) / vstep);
+        struct View {
+            float x[KS][4];
+            double w[KS];
+        };
+        const auto load = [&](int l, View& T) {
+            const float c = ct_lane(L.c, l), s = ct_lane(L.s, l), amp = ct_lane(L.amp, l), h = ct_lane(L.h, l);
+            const int jb = __builtin_amdgcn_readlane(jl, l);
+            const float* __restrict__ p = sb + ((int64_t)(g + vstep * l) * G.nu + jb) * G.nv;
+#pragma unroll
+            for (int kk = 0; kk < KS; ++kk)
+#pragma unroll
+                for (int zg = 0; zg < 4; ++zg)
+                    if (zg < nzg) T.x[kk][zg] = p[(int64_t)4 * kk * G.nv + off[zg]];
+            const float pc = -s * xc + c * yc, u0 = pc - h, u1 = pc + h;
+#pragma unroll
+            for (int kk = 0; kk < KS; ++kk) {
+                const int j = jb + 4 * kk + hi;
+                const float ou = ovl(u0, u1, sf_det(G.nu, G.du, G.su, j), sf_det(G.nu, G.du, G.su, j + 1));
+                T.w[kk] = ou > 0.0f ? (double)((ou * inv_du) * amp) : 0.0;
+            }
+        };
+        const auto use = [&](const View& T) {
+#pragma unroll
+            for (int kk = 0; kk < KS; ++kk)
+#pragma unroll
+                for (int zg = 0; zg < 4; ++zg)
+                    if (zg < nzg)
+                        acc[zg] = __builtin_amdgcn_mfma_f64_16x16x4f64(T.w[kk], (double)(T.x[kk][zg] * rw[zg]), acc[zg],
+                                                                       0, 0, 0);
+        };
+        // the next view's rows are on their way while a view is multiplied
+        View A, B;
+        load(0, A);
+        for (int l = 0; l < nl; l += 2) {
+            if (l + 1 < nl) load(l + 1, B);
+            use(A);
+            if (l + 1 >= nl) break;
+            if (l + 2 < nl) load(l + 2, A);
+            use(B);
+        }
+    }
+    // element r of acc[zg]: pixel (bx + r, by + hi), slab zb + 16 zg + lo
+    if (SPLIT) {
+#pragma unroll
+        for (int zg = 0; zg < 4; ++zg)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) red[wave][256 * zg + 64 * r + lane] = acc[zg][r];
+        __syncthreads();
+    }
+#pragma unroll
+    for (int zg = 0; zg < 4; ++zg) {
+        if (zg >= nzg || (SPLIT && zg != wave)) continue;
+        sf_d4 v = acc[zg];
+        if (SPLIT) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int e = 256 * zg + 64 * r + lane;
+                v[r] = ((red[0][e] + red[1][e]) + red[2][e]) + red[3][e];
+            }
+        }
+        const int z = zb + 16 * zg + lo;
+        const bool bad = !(fabs(v[0]) + fabs(v[1]) + fabs(v[2]) + fabs(v[3]) < (double)VIR_INF);
+        const bool again = __any(bad);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int ix = bx + r, iy = by + hi;
+            if (ix >= G.nx || iy >= G.ny || z >= G.nz) continue;
+            if (again) v[r] = sf_bp_par3_one(G, cs, sn, sb, ix, iy, min(max(z + shift, 0), G.nv - 1), rw[zg]);
+            const int64_t o = (((int64_t)b * G.nx + ix) * G.ny + iy) * G.nz + z;
+            float res = (float)v[r] * G.out_scale;
+            if (accumulate) res += img[o];
+            img[o] = res;
+        }
+    }
+}
+
+// K-steps of the matrix backprojector for the geometry (a 4 x 4 pixel block is
+// at most 4 sqrt(2) d wide on the detector: that many bins and two), or 0 where
+// it does not apply: rows not aligned with the slabs, footprints too wide, a
+// detector narrower than a block's window.
+static int sf_par3_bp_ksteps(const SFGeo& G, int& shift) {
+    const double t = 0.5 * ((double)G.nv - G.nz) - (double)G.sv;
+    if (G.dv != G.d || t != std::floor(t) || std::fabs(t) > 1e6 || G.nu > 15000) return 0;  // (eps: 0.025 bin)
+    shift = (int)t;
+    const int ks = ((int)std::floor(4.0 * 1.41422 * (double)G.d / (double)G.du + 0.05) + 2 + 3) / 4;
+    return ks <= 4 && G.nu >= 4 * ks ? ks : 0;
+}
+
+template <int KS>
+static int sf_par3_bp_mfma(const SFGeo& G, const float* cosv, const float* sinv, const float* sino, float* img, int acc,
+                           int shift, hipStream_t st) {
+    const int nbx = (G.nx + 3) / 4, nby = (G.ny + 3) / 4, nzt = (G.nz + 63) / 64;
+    const int64_t n = (int64_t)G.nb * nbx * nby * nzt;
+    if (n < 8192)
+        hipLaunchKernelGGL((k_sf_bp_par3_mfma<KS, true>), dim3((unsigned)n), dim3(256), 0, st, G, cosv, sinv, sino, img,
+                           acc, nby, nbx, nzt, shift, n);
+    else
+        hipLaunchKernelGGL((k_sf_bp_par3_mfma<KS, false>), dim3((unsigned)((n + 3) / 4)), dim3(256), 0, st, G, cosv, sinv,
+                           sino, img, acc, nby, nbx, nzt, shift, n);
+    return check_hip(hipGetLastError(), "vir_sf_bp launch");
 }
 
 // True when the column backprojector applies: a slab meets at most kSlabs
@@ -933,7 +1123,7 @@ __global__ __launch_bounds__(256) void k_sf_bp(SFGeo G, const float* __restrict_
 #pragma unroll
                 for (int q = 0; q < kSlabs; ++q)
                     if (SW.w[q] > 0.0f) sv_ += rowp[q] * SW.w[q];
-                acc += (double)(wu * sv_);
+                acc = __builtin_fma((double)wu, (double)sv_, acc);
             }
             continue;
         }
@@ -1090,6 +1280,13 @@ int vir_sf_bp(const vir_sf_geom* geom, const float* ang, const float* cosv, cons
                 return ct_bp<SFCone>(G, G.nb, ns, ang, cosv, sinv, sino, img, acc, st, "vir_sf_bp launch");
             hipLaunchKernelGGL(k_sf_bp<SF_CONE3>, grd, dim3(256), 0, st, G, ang, cosv, sinv, sino, img, acc); break;
         default:
+            if (int shift = 0; !(flags & VIR_PER_OUTPUT)) {
+                const int ks = sf_par3_bp_ksteps(G, shift);
+                if (ks == 1) return sf_par3_bp_mfma<1>(G, cosv, sinv, sino, img, acc, shift, st);
+                if (ks == 2) return sf_par3_bp_mfma<2>(G, cosv, sinv, sino, img, acc, shift, st);
+                if (ks == 3) return sf_par3_bp_mfma<3>(G, cosv, sinv, sino, img, acc, shift, st);
+                if (ks == 4) return sf_par3_bp_mfma<4>(G, cosv, sinv, sino, img, acc, shift, st);
+            }
             if (sf_par3_bp_col_ok(G) && !(flags & VIR_PER_OUTPUT)) {
                 const int nzt = (G.nz + 63) / 64;
                 const int64_t nw = (int64_t)G.nb * G.nx * G.ny * nzt;
