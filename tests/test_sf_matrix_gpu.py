@@ -22,6 +22,10 @@ CASES = [
     dict(shape=(11, 9, 40), nu=30, nv=40, na=12, d_pix=0.7, dv=0.7, du=0.8),
     dict(shape=(256, 255, 3), nu=370, nv=3, na=5, batch=2),    # a wave a block
     dict(shape=(150, 20, 70), nu=100, nv=70, na=6),            # a narrow detector
+    dict(shape=(20, 90, 7), nu=140, nv=7, na=260),             # many blocks an item: one wave group
+    dict(shape=(20, 90, 7), nu=140, nv=7, na=260, sv=0.3),
+    dict(shape=(50, 47, 40), nu=40, nv=67, na=22, sv=0.4, dv=0.6, du=2.3, batch=2),  # chunks of a line
+    dict(shape=(50, 47, 8), nu=140, nv=8, na=22, du=0.4),
 ]
 
 

@@ -413,292 +413,336 @@ __global__ __launch_bounds__(256) void k_sf_fp(SFGeo G, const float* __restrict_
 
 // ------------------------------------------ tiled parallel 3-D forward
 //
-// One workgroup computes a tile of kTUB bins x kTV detector rows of kVG
-// neighbouring views of one batch item, one view per wave; lane m of every
-// wave owns detector row m_lo + m.  For every orthogonal line, over the
-// pixels whose footprints can meet the tile in any of the views (the union
-// of the per-bin ranges of k_sf_fp):
+// A block computes 16 bins x 64 detector rows of four neighbouring views of one
+// batch item, one view per wave.  For every orthogonal line the rows' slab sums
 //   P[k][m] = sum over the row's slabs q of w_q(m) * vox[k][first(m) + q]
-// read straight from the volume (lane m reads z = first(m) + q: consecutive
-// lanes, consecutive z) into LDS -- P depends on the line and the pixel
-// only, so the views share it -- while each wave lists, for its view's
-// bins, the pixels whose footprints meet the bin and their weights; then
-//   acc[u][m] += wu(k, u) * P[k][m].
-// Views whose driving axis differs from the first view's are done in a
-// second pass over the lines.  Weights, pixel order and arithmetic are those
-// of k_sf_fp, so both give the same bits.
-constexpr int kTUB = 16;         // detector bins per tile and view
-constexpr int kVG = 4;           // views per workgroup (one per wave)
-constexpr int kTU = kTUB * kVG;  // footprint lists per workgroup
-constexpr int kTV = 64;          // detector rows per tile (one per lane)
-constexpr int kKMax = 80;        // pixels of one line handled at once (LDS: 5-6 workgroups per CU)
-constexpr int kWMax = 12;        // pixels whose footprint meets one bin (checked on the host)
-// WPER candidate pixels per lane, 4 lanes per bin: 4 WPER <= kWMax pixels per
-// bin and line (the host picks the smallest WPER its bound allows)
-constexpr int kZW = 66;          // slabs a tile's 64 rows can meet (rows no taller than a voxel: 65)
+// of the pixels whose footprints can meet the tile in any of the views are
+// brought into LDS (P depends on the line and the pixel only, so the views
+// share it), and each wave adds its view's footprint weights times P as
+// float64 matrix products (v_mfma_f64_4x4x4_4b_f64: exact products of the
+// float32 factors, float64 sums).  Its four blocks take four groups of four
+// bins, each with the pixel window its group meets: 4 du plus a footprint, six
+// to eight pixels, so two K-steps of four pixels for pixels as wide as bins,
+// and a third of the products count.  A lane evaluates the weight its operand
+// slot needs and reads the same pixel's rows: no lists, no broadcasts.
+//
+// Each of NG wave groups takes every NG-th chunk of a line's pixels; their sums
+// are added at the end in group order.
+//
+// Rows that meet exactly one slab with weight 1 (UNIT) need no slab sums: the
+// voxel rows go straight from memory into the LDS operand, the next line's
+// while a line is multiplied, with one barrier a line.  Otherwise each wave
+// replaces its share of the staged rows by their slab sums in place.
+//
+// The matrix and vector operations of the waves take turns: 16 products a K-step
+// (294 cycles of about 500, with the 16 conversions, one weight and the reads).
+// Staging more lines ahead changed nothing; more than five waves a SIMD were not
+// to be had (16 float64 sums a lane).  8 x 256 x 256 x 64, 180 views of 384 x 64:
+// 8.2 -> 3.0 ms against a form that listed each bin's pixels with cross-lane
+// prefix sums and accumulated row by row; 1 x 256 x 256 x 64, 64 views, 2.79 -> 0.50.
+constexpr int kTUB = 16;  // detector bins per tile and view
+constexpr int kVG = 4;    // views per workgroup (one per wave)
+constexpr int kTV = 64;   // detector rows per tile
+constexpr int kMK = 40;   // pixels of one line staged at once
+constexpr int kMP = 68;   // LDS row pitch: 16-byte reads of four windows of rows meet different banks
+constexpr int kZW = 66;   // slabs a tile's 64 rows can meet (rows no taller than a voxel: 65)
 
-template <int WPER>
-__global__ __launch_bounds__(64 * kVG) __attribute__((amdgpu_waves_per_eu(6))) void k_sf_fp_par3_tile(SFGeo G, const float* __restrict__ ang,
-                                                        const float* __restrict__ cs,
-                                                        const float* __restrict__ sn,
-                                                        const float* __restrict__ img, float* __restrict__ sino,
-                                                        int accumulate, int nut, int nmt, int nvg) {
-    // row kk of the chunk: the voxels vox[k][zb + z] of pixel k = kc + kk,
-    // then, in place, its slab sums P[k][m] for the tile's rows m
-    __shared__ float R[kKMax * kZW];
-    // footprint list per bin: (LDS offset (k - kc) * kTV of the j-th pixel,
-    // its weight overlap/du * amplitude as bits), read as one 64-bit word
-    constexpr int kWSlot = 4 * WPER;  // footprint list stride per bin
-    __shared__ int2 wlist[kTU * kWSlot];
-    __shared__ int wcnt[kTU];
+// One bin and row by the gather.
+__device__ double sf_fp_par3_one(const SFGeo& G, const SFView& V, const float* __restrict__ vol, int iu, int iv) {
+    const bool xd = fabsf(V.s) >= fabsf(V.c);
+    const int nd = xd ? G.nx : G.ny, no = xd ? G.ny : G.nx;
+    const float ul = sf_det(G.nu, G.du, G.su, iu), ur = sf_det(G.nu, G.du, G.su, iu + 1);
+    const float inv_d = 1.0f / G.d, inv_du = 1.0f / G.du;
+    SlabWeights SW;
+    par3_row_slabs(G, iv, SW);
+    double acc = 0.0;
+    for (int io = 0; io < no; ++io) {
+        const float oc = (sf_bnd(no, G.d, io) + sf_bnd(no, G.d, io + 1)) * 0.5f;
+        const float x0 = sf_invert<SF_PAR3>(G, xd, V.c, V.s, ul - G.wmax, oc);
+        const float x1 = sf_invert<SF_PAR3>(G, xd, V.c, V.s, ur + G.wmax, oc);
+        const float k0f = fminf(x0, x1) * inv_d + 0.5f * (float)nd - 0.5f;
+        const float k1f = fmaxf(x0, x1) * inv_d + 0.5f * (float)nd - 0.5f;
+        if (!(k0f < (float)nd + 1.0f) || !(k1f > -2.0f)) continue;
+        const int k0 = (int)fmaxf(floorf(k0f) - 1.0f, 0.0f), k1 = (int)fminf(floorf(k1f) + 2.0f, (float)(nd - 1));
+        for (int k = k0; k <= k1; ++k) {
+            const int ix = xd ? k : io, iy = xd ? io : k;
+            const SFFoot f = sf_foot<SF_PAR3>(G, V, ix, iy);
+            const float ou = ovl(f.u0, f.u1, ul, ur);
+            if (!(ou > 0.0f)) continue;
+            const float* col = vol + ((int64_t)ix * G.ny + iy) * G.nz;
+            float sv = 0.0f;
+#pragma unroll
+            for (int q = 0; q < kSlabs; ++q)
+                if (SW.w[q] > 0.0f) sv += col[SW.first + q] * SW.w[q];
+            acc = __builtin_fma((double)((ou * inv_du) * f.amp), (double)sv, acc);
+        }
+    }
+    return acc;
+}
+
+template <bool UNIT, int NG>
+__global__ __launch_bounds__(64 * kVG * NG) __attribute__((amdgpu_waves_per_eu(4))) void k_sf_fp_par3_mfma(SFGeo G, const float* __restrict__ cs,
+                                                             const float* __restrict__ sn,
+                                                             const float* __restrict__ img, float* __restrict__ sino,
+                                                             int accumulate, int nut, int nmt, int nvg, int shift) {
+    // two objects, so that reads of one need not wait for loads into the other
+    __shared__ __attribute__((aligned(16))) float R0[NG * kMK * kMP], R1[NG * kMK * kMP];
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform: scalar
-    int blk = blockIdx.x;
-    const int mt = blk % nmt;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) % kVG;
+    const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) / kVG;
+    // operand slots: group (matrix block) mid; weights: bin lo, pixel hi; rows:
+    // row quad lo, pixel hi; sums: bin hi, row quad lo
+    const int lo = lane & 3, mid = (lane >> 2) & 3, hi = lane >> 4;
+    int blk = (int)xcd_remap(blockIdx.x, gridDim.x);
+    const int m_lo = (blk % nmt) * kTV;
     blk /= nmt;
-    const int ut = blk % nut;
+    const int u_lo = (blk % nut) * kTUB;
     blk /= nut;
-    const int vg = blk % nvg;
+    const int a0 = (blk % nvg) * kVG, nva = min(kVG, G.na - a0);
     const int b = blk / nvg;
-    const int u_lo = ut * kTUB, u_n = min(kTUB, G.nu - u_lo);
-    const int m_lo = mt * kTV, m_n = min(kTV, G.nv - m_lo);
-    const int a0 = vg * kVG, nva = min(kVG, G.na - a0);
-
-    // this wave's view
-    const int ia = a0 + wave;
+    const int ia = a0 + min(wave, nva - 1);
     const bool vwave = wave < nva;
-    const int iav = vwave ? ia : a0;
-    const SFView V = sf_view(G, cs[iav], sn[iav], ang[iav]);
-    const float c = V.c, s = V.s;
-    const bool xd = fabsf(s) >= fabsf(c);
+    const SFView V = sf_view(G, cs[ia], sn[ia], 0.0f);
+    const bool xd = fabsf(V.s) >= fabsf(V.c);
     const float inv_d = 1.0f / G.d, inv_du = 1.0f / G.du;
     const float* vol = img + (int64_t)b * G.nx * G.ny * G.nz;
 
-    // this lane's detector row: its slabs with non-zero weight, in slab
-    // order (the k_sf_fp sum skips the zero weights)
-    const bool mrow = lane < m_n;
-    SlabWeights SW;
-    par3_row_slabs(G, m_lo + (mrow ? lane : 0), SW);
-    int nzs = 0, sz[kSlabs];
+    // staging lanes: row m_lo + lane.  UNIT: its slab; else the slabs of
+    // non-zero weight in slab order, and the tile's slab range zb, span
+    const int m = m_lo + lane;
+    bool zin = false;
+    int zb = 0, span = 64, nzs = 0, zo[kSlabs];
     float swt[kSlabs];
+    if (UNIT) {
+        zb = m_lo - shift;
+        zin = m < G.nv && zb + lane >= 0 && zb + lane < G.nz;
+    } else {
+        SlabWeights SW;
+        par3_row_slabs(G, min(m, G.nv - 1), SW);
+        int sz[kSlabs];
 #pragma unroll
-    for (int q = 0; q < kSlabs; ++q) {
-        sz[q] = 0;
-        swt[q] = 0.0f;
-    }
+        for (int q = 0; q < kSlabs; ++q) {
+            sz[q] = 0;
+            swt[q] = 0.0f;
+        }
 #pragma unroll
-    for (int q = 0; q < kSlabs; ++q) {
-        if (SW.w[q] > 0.0f) {
+        for (int q = 0; q < kSlabs; ++q) {
+            if (SW.w[q] > 0.0f) {
 #pragma unroll
-            for (int r = 0; r < kSlabs; ++r) {  // slot nzs, without dynamic register indexing
-                if (r == nzs) {
-                    sz[r] = SW.first + q;
-                    swt[r] = SW.w[q];
+                for (int r = 0; r < kSlabs; ++r) {  // slot nzs, without dynamic register indexing
+                    if (r == nzs) {
+                        sz[r] = SW.first + q;
+                        swt[r] = SW.w[q];
+                    }
                 }
+                ++nzs;
             }
-            ++nzs;
         }
-    }
-    if (!mrow) nzs = 0;
-    // slabs any lane of the wave needs (wave-uniform): the staging loads
-    // are bounded by it, not masked per lane
-    int nzs_max = nzs;
+        if (m >= G.nv) nzs = 0;
+        int zlo = 0x7fffffff, zhi = -1;
 #pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) nzs_max = max(nzs_max, __shfl_xor(nzs_max, m));
-    const int nzs_u = __builtin_amdgcn_readfirstlane(nzs_max);
-    // the slabs of all the tile's rows: zb .. zb + span - 1 (the same in every wave)
-    int zlo = 0x7fffffff, zhi = -1;
+        for (int q = 0; q < kSlabs; ++q)
+            if (q < nzs) {
+                zlo = min(zlo, sz[q]);
+                zhi = max(zhi, sz[q]);
+            }
 #pragma unroll
-    for (int q = 0; q < kSlabs; ++q)
-        if (q < nzs) {
-            zlo = min(zlo, sz[q]);
-            zhi = max(zhi, sz[q]);
+        for (int t = 32; t >= 1; t >>= 1) {
+            zlo = min(zlo, __shfl_xor(zlo, t));
+            zhi = max(zhi, __shfl_xor(zhi, t));
         }
+        zb = __builtin_amdgcn_readfirstlane(zhi >= 0 ? zlo : 0);
+        span = min(__builtin_amdgcn_readfirstlane(zhi >= 0 ? zhi - zlo + 1 : 0), kZW);
 #pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) {
-        zlo = min(zlo, __shfl_xor(zlo, m));
-        zhi = max(zhi, __shfl_xor(zhi, m));
+        for (int q = 0; q < kSlabs; ++q) zo[q] = min(max(sz[q] - zb, 0), kZW - 1);
     }
-    const int zb = __builtin_amdgcn_readfirstlane(zhi >= 0 ? zlo : 0);
-    const int span = min(__builtin_amdgcn_readfirstlane(zhi >= 0 ? zhi - zlo + 1 : 0), kZW);
-    // this lane's slabs as offsets into an LDS row
-    int zo[kSlabs];
-#pragma unroll
-    for (int q = 0; q < kSlabs; ++q) zo[q] = min(max(sz[q] - zb, 0), kZW - 1);
 
-    // footprint-list lanes: bin u_lo + (lane & 15) of this wave's view (list
-    // slot tu_w), candidate group grp
-    const int tu_w = wave * kTUB + (lane & 15), grp = lane >> 4;
-    const int iu_w = u_lo + (lane & 15);
-    const bool ubin = vwave && (lane & 15) < u_n;
-    const float ul = sf_det(G.nu, G.du, G.su, iu_w), ur = sf_det(G.nu, G.du, G.su, iu_w + 1);
+    // this lane's weight: bin u_lo + 4 mid + lo; its group's pixel window
+    // starts at the first centre that projects past the group's left edge less
+    // a half footprint (x = A - oc B in pixels, widened by its rounding)
+    const int iu = u_lo + 4 * mid + lo;
+    const float ul = sf_det(G.nu, G.du, G.su, iu), ur = sf_det(G.nu, G.du, G.su, iu + 1);
+    const float pd = xd ? -V.s : V.c, po = xd ? V.c : -V.s;
+    const int nd = xd ? G.nx : G.ny;
+    const float eps = 2e-3f + 2e-6f * (float)(G.nx + G.ny);
+    const float rp = inv_d / pd, gB = po * rp, gc = 0.5f * (float)nd - 0.5f - eps;
+    const float ge0 = (sf_det(G.nu, G.du, G.su, u_lo + 4 * mid) - V.h) * rp;
+    const float ge1 = (sf_det(G.nu, G.du, G.su, u_lo + 4 * mid + 4) + V.h) * rp;
+    const float gA = fminf(ge0, ge1) + gc;
+    const int nks = __builtin_amdgcn_readfirstlane(((int)floorf(fabsf(ge1 - ge0) + 2.0f * eps) + 4) >> 2);
 
-    // the tile's bin edges (footprint margin included)
-    const float ut0 = sf_det(G.nu, G.du, G.su, u_lo) - G.wmax;
-    const float ut1 = sf_det(G.nu, G.du, G.su, u_lo + u_n) + G.wmax;
-    // sf_invert<SF_PAR3>(u, oc) = (u - po oc) / pd as u/pd - oc po/pd: one
-    // FMA per line.  The inverse only bounds pixel ranges that are widened
-    // by a pixel or more (|pd| >= 1/sqrt 2, rounding moves it by ~1e-4
-    // pixel), and pixels of zero overlap add nothing, so the sums are those
-    // of k_sf_fp.
-    const float pd = xd ? -s : c, po = xd ? c : -s;
-    const float inv_pd = 1.0f / pd, lin_b = po * inv_pd;
-    const float al = (ul - G.wmax) * inv_pd, ar = (ur + G.wmax) * inv_pd;
-    // every view of the group (wave-uniform): driving axis and the tile's
-    // band as at0 - oc lin_b .. at1 - oc lin_b
-    bool gxd[kVG];
+    // the tile's edges, and the views' bands x = at0 - oc lin .. at1 - oc lin
+    const float ut0 = sf_det(G.nu, G.du, G.su, u_lo), ut1 = sf_det(G.nu, G.du, G.su, min(u_lo + kTUB, G.nu));
+    bool gxd[kVG], mixed = false;
     float glin[kVG], gat0[kVG], gat1[kVG];
-    bool mixed = false;
 #pragma unroll
     for (int w = 0; w < kVG; ++w) {
         const int aw = a0 + min(w, nva - 1);
-        const float cw = cs[aw], sw = sn[aw];
-        gxd[w] = fabsf(sw) >= fabsf(cw);
-        const float pdw = gxd[w] ? -sw : cw, pow_ = gxd[w] ? cw : -sw;
-        const float ipd = 1.0f / pdw;
-        glin[w] = pow_ * ipd;
-        gat0[w] = ut0 * ipd;
-        gat1[w] = ut1 * ipd;
+        const SFView W = sf_view(G, cs[aw], sn[aw], 0.0f);
+        gxd[w] = fabsf(W.s) >= fabsf(W.c);
+        const float ipd = inv_d / (gxd[w] ? -W.s : W.c);
+        glin[w] = (gxd[w] ? W.c : -W.s) * ipd;
+        const float e0 = (ut0 - W.h) * ipd, e1 = (ut1 + W.h) * ipd;
+        gat0[w] = fminf(e0, e1) - eps;
+        gat1[w] = fmaxf(e0, e1) + eps;
         mixed |= w < nva && gxd[w] != gxd[0];
     }
 
-    double acc[kTUB];
+    double acc[16];  // bin u_lo + 4 mid + hi, rows 16 c + 4 lo + e at 4 c + e
 #pragma unroll
-    for (int i = 0; i < kTUB; ++i) acc[i] = 0.0;
+    for (int i = 0; i < 16; ++i) acc[i] = 0.0;
 
     // views whose driving axis is that of the first view, then the others
     for (int pass = 0; pass < (mixed ? 2 : 1); ++pass) {
         const bool pxd = pass == 0 ? gxd[0] : !gxd[0];
         const bool active = vwave && xd == pxd;
-        const int nd = pxd ? G.nx : G.ny, no = pxd ? G.ny : G.nx;
-        for (int io = 0; io < no; ++io) {
-            const float oc = (sf_bnd(no, G.d, io) + sf_bnd(no, G.d, io + 1)) * 0.5f;
-            // the union of the pass's views' pixel bands on this line
-            int k0t = nd, k1t = -1;
+        const int pnd = pxd ? G.nx : G.ny, pno = pxd ? G.ny : G.nx;
+        const int64_t kstride = (int64_t)(pxd ? G.ny : 1) * G.nz, lstride = (int64_t)(pxd ? 1 : G.ny) * G.nz;
+        for (int lb = 0; lb < pno; lb += 64) {
+            // lane = line lb + lane: the union of the pass's views' pixel bands
+            const int iol = lb + lane;
+            const float ocl = (sf_bnd(pno, G.d, iol) + sf_bnd(pno, G.d, iol + 1)) * 0.5f;
+            int k0l = pnd, k1l = -1;
 #pragma unroll
             for (int w = 0; w < kVG; ++w) {
                 if (w >= nva || gxd[w] != pxd) continue;
-                const float x0 = __builtin_fmaf(-oc, glin[w], gat0[w]);
-                const float x1 = __builtin_fmaf(-oc, glin[w], gat1[w]);
-                const float k0f = fminf(x0, x1) * inv_d + 0.5f * (float)nd - 0.5f;
-                const float k1f = fmaxf(x0, x1) * inv_d + 0.5f * (float)nd - 0.5f;
-                if (!(k0f < (float)nd + 1.0f) || !(k1f > -2.0f)) continue;
-                k0t = min(k0t, (int)fmaxf(floorf(k0f) - 1.0f, 0.0f));
-                k1t = max(k1t, (int)fminf(floorf(k1f) + 2.0f, (float)(nd - 1)));
+                const float c0 = 0.5f * (float)pnd - 0.5f;
+                k0l = min(k0l, (int)fmaxf(ceilf(__builtin_fmaf(-ocl, glin[w], gat0[w]) + c0), 0.0f));
+                k1l = max(k1l, (int)fminf(floorf(__builtin_fmaf(-ocl, glin[w], gat1[w]) + c0), (float)(pnd - 1)));
             }
-            if (k0t > k1t) continue;
-            // this lane's bin: its candidate pixel range (as k_sf_fp)
-            int kb0 = 0, kb1 = -1;
-            if (ubin && active) {
-                const float y0 = __builtin_fmaf(-oc, lin_b, al);
-                const float y1 = __builtin_fmaf(-oc, lin_b, ar);
-                const float b0f = fminf(y0, y1) * inv_d + 0.5f * (float)nd - 0.5f;
-                const float b1f = fmaxf(y0, y1) * inv_d + 0.5f * (float)nd - 0.5f;
-                if (b0f < (float)nd + 1.0f && b1f > -2.0f) {
-                    kb0 = (int)fmaxf(floorf(b0f) - 1.0f, 0.0f);
-                    kb1 = (int)fminf(floorf(b1f) + 2.0f, (float)(nd - 1));
+            if (iol >= pno) k1l = -1;
+            // this group's chunk (line cl, pixels ck .., nk of them; of every
+            // NG the group's own): all groups walk the same list
+            int l = -1, kc = 0, ke = -1, cl = 0, ck = 0, nk = 0;
+            const auto stage = [&](float* dst) {
+                bool any = false;
+                nk = 0;
+#pragma unroll
+                for (int s = 0; s < NG; ++s) {
+                    kc += kMK;
+                    while (kc > ke && l < 64) {
+                        if (++l >= 64 || lb + l >= pno) {
+                            l = 64;
+                            break;
+                        }
+                        kc = __builtin_amdgcn_readlane(k0l, l);
+                        ke = __builtin_amdgcn_readlane(k1l, l);
+                    }
+                    any |= l < 64;
+                    if (s == grp && l < 64) {
+                        cl = l;
+                        ck = kc;
+                        nk = min(kMK, ke - kc + 1);
+                    }
                 }
-            }
-            for (int kc = k0t; kc <= k1t; kc += kKMax) {
-                const int nk = min(kKMax, k1t - kc + 1);
-                __syncthreads();  // the previous chunk's reads are done
-                // the chunk's voxel rows, straight from the volume into LDS
-                // (consecutive lanes, consecutive z; no registers held): all of
-                // a wave's rows are in flight together, while the footprint
-                // lists below are built
+                const float* p = vol + (int64_t)(lb + cl) * lstride + (int64_t)ck * kstride + zb + lane;
                 for (int kk = wave; kk < nk; kk += kVG) {
-                    const int k = kc + kk;
-                    const int ix = pxd ? k : io, iy = pxd ? io : k;
-                    const float* col = vol + ((int64_t)ix * G.ny + iy) * G.nz + zb;
-                    float* row = R + kk * kZW;
-                    if (lane < span)
-                        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(col + lane),
+                    float* row = dst + (grp * kMK + kk) * kMP;
+                    if (UNIT ? zin : lane < span)
+                        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(p + kk * kstride),
                                                          (__attribute__((address_space(3))) void*)row, 4, 0, 0);
-                    if (lane < span - 64)
+                    if (!UNIT && lane < span - 64)
                         __builtin_amdgcn_global_load_lds(
-                            (const __attribute__((address_space(1))) void*)(col + 64 + lane),
+                            (const __attribute__((address_space(1))) void*)(p + kk * kstride + 64),
                             (__attribute__((address_space(3))) void*)(row + 64), 4, 0, 0);
                 }
-                // footprint lists of this wave's bins over the chunk, in pixel
-                // order: lane group grp tests candidates ka + WPER grp .. ka + WPER grp + WPER - 1
-                {
-                    const int ka = max(kb0, kc), kz = min(kb1, kc + nk - 1);
-                    float wv[WPER];
-                    int nzc = 0;
+                return any;
+            };
+            __syncthreads();  // the last chunk's readers are done
+            bool more = stage(R0);
+            const auto step = [&](float* Rp, float* Rn) {
+                const int dl = cl, dk = ck, dn = nk;
+                Rp += grp * kMK * kMP;
+                __syncthreads();  // these chunks have landed; the other buffer is no longer read
+                more = stage(Rn);
+                if (!UNIT) {
+                    // slab sums of this wave's rows, in place: each row is read
+                    // and rewritten by one wave, reads before writes
+                    for (int kk = wave; kk < dn; kk += kVG) {
+                        float sv = 0.0f;
 #pragma unroll
-                    for (int j = 0; j < WPER; ++j) {
-                        const int k = ka + grp * WPER + j;
-                        float w = 0.0f;
-                        if (k <= kz) {
-                            const int ix = xd ? k : io, iy = xd ? io : k;
-                            const SFFoot f = sf_foot<SF_PAR3>(G, V, ix, iy);
-                            const float ou = ovl(f.u0, f.u1, ul, ur);
-                            if (ou > 0.0f) w = (ou * inv_du) * f.amp;
-                        }
-                        wv[j] = w;
-                        nzc += (k <= kz && w != 0.0f) ? 1 : 0;
+                        for (int q = 0; q < kSlabs; ++q)
+                            if (q < nzs) sv += Rp[kk * kMP + zo[q]] * swt[q];
+                        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                        Rp[kk * kMP + lane] = sv;
                     }
-                    // exclusive prefix of the group counts of this bin (lanes l, l+16, l+32, l+48)
-                    const int c1 = __shfl_up(nzc, 16), c2 = __shfl_up(nzc, 32), c3 = __shfl_up(nzc, 48);
-                    int pos = (grp >= 1 ? c1 : 0) + (grp >= 2 ? c2 : 0) + (grp >= 3 ? c3 : 0);
-                    const int total = __shfl(pos + nzc, (lane & 15) + 48);
-#pragma unroll
-                    for (int j = 0; j < WPER; ++j) {
-                        const int k = ka + grp * WPER + j;
-                        if (k <= kz && wv[j] != 0.0f) {
-                            wlist[tu_w * kWSlot + pos] = make_int2((k - kc) * kZW, __float_as_int(wv[j]));
-                            ++pos;
-                        }
-                    }
-                    if (grp == 0) wcnt[tu_w] = ubin ? total : 0;
+                    __syncthreads();
                 }
-                __syncthreads();  // the voxel rows have landed
-                // slab sums of this wave's rows, in place: each row is read
-                // and rewritten by one wave, reads before writes
-                for (int kk = wave; kk < nk; kk += kVG) {
-                    float x[kSlabs];
+                if (!active || dn == 0) return;
+                const float oc = ct_lane(ocl, dl);
+                const float xl = G.d * (((float)(lb + dl) + 0.5f) - 0.5f * (float)pno);
+                const int win = (int)ceilf(__builtin_fmaf(-oc, gB, gA)) + hi;
+                for (int kk = 0; kk < nks; ++kk) {
+                    const int k = win + 4 * kk, kr = k - dk;
+                    const float xk = G.d * (((float)k + 0.5f) - 0.5f * (float)nd);
+                    const float pc = pd * xk + po * xl;
+                    const float ou = ovl(pc - V.h, pc + V.h, ul, ur);
+                    const bool in = ou > 0.0f && (unsigned)kr < (unsigned)dn;
+                    if (!__any(in)) continue;  // another view's pixels, or another chunk's
+                    const double w = in ? (double)((ou * inv_du) * V.amp) : 0.0;
+                    const float4* row = (const float4*)(Rp + min(max(kr, 0), dn - 1) * kMP + 4 * lo);
+                    float4 x[4];
 #pragma unroll
-                    for (int q = 0; q < kSlabs; ++q) x[q] = q < nzs_u ? R[kk * kZW + zo[q]] : 0.0f;
-                    float sv_ = 0.0f;
+                    for (int c = 0; c < 4; ++c) x[c] = row[4 * c];
 #pragma unroll
-                    for (int q = 0; q < kSlabs; ++q)
-                        if (q < nzs) sv_ += x[q] * swt[q];
-                    R[kk * kZW + lane] = sv_;
-                }
-                __syncthreads();
-                if (mrow && active) {
-#pragma unroll
-                    for (int i = 0; i < kTUB; ++i) {
-                        const int tu = wave * kTUB + i;
-                        const int cnt = wcnt[tu];  // wave-uniform
-                        const int2* wl = wlist + tu * kWSlot;
-                        int j = 0;
-                        // offsets (k - kc) * kZW with 0 <= k - kc < nk <= kKMax
-                        for (; j + 1 < cnt; j += 2) {
-                            const int2 e0 = wl[j], e1 = wl[j + 1];
-                            const float p0 = R[e0.x + lane];
-                            const float p1 = R[e1.x + lane];
-                            acc[i] = __builtin_fma((double)__int_as_float(e0.y), (double)p0, acc[i]);
-                            acc[i] = __builtin_fma((double)__int_as_float(e1.y), (double)p1, acc[i]);
-                        }
-                        if (j < cnt) {
-                            const int2 e0 = wl[j];
-                            acc[i] = __builtin_fma((double)__int_as_float(e0.y), (double)R[e0.x + lane], acc[i]);
-                        }
+                    for (int c = 0; c < 4; ++c) {
+                        acc[4 * c] = __builtin_amdgcn_mfma_f64_4x4x4f64(w, (double)x[c].x, acc[4 * c], 0, 0, 0);
+                        acc[4 * c + 1] = __builtin_amdgcn_mfma_f64_4x4x4f64(w, (double)x[c].y, acc[4 * c + 1], 0, 0, 0);
+                        acc[4 * c + 2] = __builtin_amdgcn_mfma_f64_4x4x4f64(w, (double)x[c].z, acc[4 * c + 2], 0, 0, 0);
+                        acc[4 * c + 3] = __builtin_amdgcn_mfma_f64_4x4x4f64(w, (double)x[c].w, acc[4 * c + 3], 0, 0, 0);
                     }
                 }
+            };
+            while (more) {
+                step(R0, R1);
+                if (more) step(R1, R0);
             }
         }
     }
-    if (!mrow || !vwave) return;
-    const int64_t base = (((int64_t)b * G.na + ia) * G.nu) * G.nv + m_lo + lane;
+    // the groups' sums, in group order
+    static_assert(NG == 1 || kVG * 64 * 8 * 2 <= NG * kMK * kMP, "eight sums a lane fit a buffer");
 #pragma unroll
-    for (int i = 0; i < kTUB; ++i) {
-        if (i >= u_n) continue;
-        const int64_t o = base + (int64_t)(u_lo + i) * G.nv;
-        float res = (float)acc[i] * G.out_scale;
-        if (accumulate) res += sino[o];
-        sino[o] = res;
+    for (int g = 1; g < NG; ++g) {
+        double *S0 = (double*)R0 + wave * 512 + lane, *S1 = (double*)R1 + wave * 512 + lane;
+        __syncthreads();
+        if (grp == g) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                S0[64 * i] = acc[i];
+                S1[64 * i] = acc[8 + i];
+            }
+        }
+        __syncthreads();
+        if (grp == 0) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                acc[i] += S0[64 * i];
+                acc[8 + i] += S1[64 * i];
+            }
+        }
+    }
+    if (grp != 0) return;
+    const int ob = u_lo + 4 * mid + hi;
+    if (!vwave || ob >= G.nu) return;
+    float* out = sino + (((int64_t)b * G.na + ia) * G.nu + ob) * G.nv;
+    const auto put = [&](int mr, double v) {
+        const float res = (float)v * G.out_scale;
+        out[mr] = accumulate ? out[mr] + res : res;
+    };
+    unsigned odd = 0;  // sums with zero weights times infinities: by the gather
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int mr = m_lo + 16 * (i >> 2) + 4 * lo + (i & 3);
+        if (mr >= G.nv) continue;
+        if (UNIT && (mr - shift < 0 || mr - shift >= G.nz)) put(mr, 0.0);  // a row without a slab
+        else if (fabs(acc[i]) < (double)VIR_INF) put(mr, acc[i]);
+        else odd |= 1u << i;
+    }
+    while (odd) {
+        const int i = __ffs((int)odd) - 1;
+        odd &= odd - 1;
+        const int mr = m_lo + 16 * (i >> 2) + 4 * lo + (i & 3);
+        put(mr, sf_fp_par3_one(G, V, vol, ob, mr));
     }
 }
 
@@ -999,7 +1043,7 @@ __global__ __launch_bounds__(256) void k_sf_bp_par3_mfma(SFGeo G, const float* _
     for (int zg = 0; zg < 4; ++zg) {
         if (zg >= nzg || (SPLIT && zg != wave)) continue;
         sf_d4 v = acc[zg];
-        if (SPLIT) {
+        if constexpr (SPLIT) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int e = 256 * zg + 64 * r + lane;
@@ -1056,20 +1100,29 @@ static bool sf_par3_bp_col_ok(const SFGeo& G) {
     return 1.4143 * (double)G.d / (double)G.du + 4.0 <= (double)kJMax;
 }
 
-// Bound on the candidate pixels of one bin along a line: a bin's pixel range
-// is floor(b1) - floor(b0) + 4 long, b1 - b0 = (du + 2 wmax) / (|pd| d) with
-// |pd| >= 1/sqrt 2, so it is at most floor(X) + 5 for X that ratio's bound;
-// per_bin = X + 5 keeps a margin for rounding.
-static double sf_par3_per_bin(const SFGeo& G) {
-    return ((double)G.du + 2.0 * (double)G.wmax) / (0.70710678 * (double)G.d) + 5.0;
-}
+// True when the tiled parallel 3-D forward kernel takes the call: detector rows
+// no taller than a voxel (each row meets at most kSlabs slabs), and where it is
+// faster than the gather.  256 x 256, 1.5 x 256 bins, tile | gather in us:
+// 8 items, 180 views, 64 rows, du = d: 2930 | 28500, 2 d: 2980 | 17600, 2.8 d:
+// 3990 | 16400; 1 item, 64 views: 500 | 1635, 1140 | 1230, 1510 | 1170 (wide bins
+// have long pixel windows).  8 items with 4 rows 2910 | 2225, with 8: 2910 |
+// 3910; 1 item, 64 views, 4 rows 500 | 480.
+static bool sf_par3_tiled_ok(const SFGeo& G) { return G.dv <= G.d && G.du <= 2.5f * G.d && G.nv >= 6; }
 
-// True when the tiled parallel 3-D forward kernel applies: detector rows no
-// taller than a voxel (each row meets at most kSlabs slabs) and at most
-// kWMax - 1 pixels per bin along a line.
-static bool sf_par3_tiled_ok(const SFGeo& G) {
-    if (!(G.dv <= G.d)) return false;
-    return sf_par3_per_bin(G) <= (double)(kWMax - 1);
+// An item with at most this many blocks (two a CU) takes two wave groups a
+// block: they wait for their own chain of operands, not for the matrix cores.
+// 256 x 256 x 64, 64 views (384 blocks) 682 -> 500 us; with 8 items and 180 views
+// (8640 blocks) one group is the faster one, 2940 against 3660 us.
+constexpr int kParBlocks2 = 512;
+
+// True when every row m meets slab m - shift alone with weight 1: rows aligned
+// with the slabs, and a power-of-two spacing, so that overlap / dv is exact.
+static bool sf_par3_unit_rows(const SFGeo& G, int& shift) {
+    const double t = 0.5 * ((double)G.nv - G.nz) - (double)G.sv;
+    int e;
+    if (G.dv != G.d || t != std::floor(t) || std::fabs(t) > 1e6 || std::frexp(G.d, &e) != 0.5f) return false;
+    shift = (int)t;
+    return true;
 }
 
 template <int MODE>
@@ -1238,15 +1291,15 @@ int vir_sf_fp(const vir_sf_geom* geom, const float* ang, const float* cosv, cons
             if (sf_par3_tiled_ok(G) && !(flags & VIR_PER_OUTPUT)) {
                 const int nut = (G.nu + kTUB - 1) / kTUB, nmt = (G.nv + kTV - 1) / kTV;
                 const int nvg = (G.na + kVG - 1) / kVG;
-                const int64_t nblk = (int64_t)G.nb * nvg * nut * nmt;
-                // two candidates per lane when a bin's range is at most 8 pixels
-                // (X <= 3.9 < 4), else three (X <= 6: at most 11 of 12)
-                if (sf_par3_per_bin(G) <= 8.9)
-                    hipLaunchKernelGGL(k_sf_fp_par3_tile<2>, dim3((unsigned)nblk), dim3(64 * kVG), 0, st, G, ang, cosv,
-                                       sinv, img, sino, acc, nut, nmt, nvg);
-                else
-                    hipLaunchKernelGGL(k_sf_fp_par3_tile<3>, dim3((unsigned)nblk), dim3(64 * kVG), 0, st, G, ang, cosv,
-                                       sinv, img, sino, acc, nut, nmt, nvg);
+                const dim3 tg((unsigned)((int64_t)G.nb * nvg * nut * nmt));
+                int shift = 0;
+                const bool unit = sf_par3_unit_rows(G, shift);
+                // by one item's blocks, so that an item's bits don't depend on the batch
+                const bool two = nvg * nut * nmt <= kParBlocks2;
+                const auto kern = unit ? (two ? k_sf_fp_par3_mfma<true, 2> : k_sf_fp_par3_mfma<true, 1>)
+                                       : (two ? k_sf_fp_par3_mfma<false, 2> : k_sf_fp_par3_mfma<false, 1>);
+                hipLaunchKernelGGL(kern, tg, dim3(64 * kVG * (two ? 2 : 1)), 0, st, G, cosv, sinv, img, sino, acc, nut,
+                                   nmt, nvg, shift);
             } else {
                 hipLaunchKernelGGL(k_sf_fp<SF_PAR3>, grd, dim3(256), 0, st, G, ang, cosv, sinv, img, sino, acc);
             }
