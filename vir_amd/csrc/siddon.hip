@@ -17,6 +17,7 @@
 namespace vir {
 
 constexpr int kRayThreads = 256;
+constexpr int kFpSplit = 8;  // waves that share a ray's walk, at most
 
 // ---------------------------------------------------------------- trace
 
@@ -208,6 +209,96 @@ __global__ __launch_bounds__(kRayThreads) __attribute__((amdgpu_waves_per_eu(NB 
     if (bad && err) atomicAdd(err, bad);
 }
 
+// k_siddon_fp with each ray's walk divided among the S waves of a workgroup of
+// 64 rays: wave i takes the pairs whose left element lies in (T_i, T_i+1],
+// T_i = amin + i/S (amax - amin), entering at T_i with walker_seek, which
+// recomputes the same plane alphas.  A walk that ends past T_i+1 has also
+// visited the pair across it, the next wave's first; that one is taken back
+// (it is still pending).  The parts are summed in float64 in order.
+// FLAT: grids one voxel thick; waves whose rays all lie in the plane walk two
+// streams, with the third index fixed.  What bounds it: issue, two thirds of it
+// float64 (no form of the index but the float64 midpoint gives the same entries).
+template <bool P2, bool FLAT, int NB>
+__global__ __launch_bounds__(64 * kFpSplit) void k_siddon_fp_split(
+    GridK g, const float* __restrict__ src, const float* __restrict__ trg, const float* __restrict__ rec,
+    int64_t nrays, const float* __restrict__ vol, float* __restrict__ sino, int accumulate,
+    int32_t* __restrict__ err, SirtEpi E, int64_t vstride, int S) {
+    __shared__ double part[kFpSplit * NB * 64];
+    const int lane = threadIdx.x & 63;
+    const int seg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t r = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * 64 + lane;
+    double sum[NB];
+    float pv[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+        sum[j] = 0.0;
+        pv[j] = 0.0f;
+    }
+    int bad = 0;
+    if (r < nrays) {
+        Ray R;
+        if (NB > 1 || rec) ray_load_record(rec + (size_t)kRayRec * r, R);
+        else ray_setup<false>(g, src + 3 * r, trg + 3 * r, R);
+        if (R.hit) {
+            const float span = (R.amax - R.amin) / (float)S;
+            const float t0 = R.amin + (float)seg * span;
+            const float t1 = seg + 1 < S ? R.amin + (float)(seg + 1) * span : VIR_INF;
+            const unsigned nyz = (unsigned)(g.n[1] * g.n[2]);
+            float pl = 0.0f;
+            bool pin = false, pbad = false;
+            auto visit = [&](int ix, int iy, int iz, float len, bool keep) {
+                bool in = (unsigned)ix < (unsigned)g.n[0] && (unsigned)iy < (unsigned)g.n[1] &&
+                          (unsigned)iz < (unsigned)g.n[2];
+                bad += pbad ? 1 : 0;
+                pbad = keep && !in;
+                bool use = keep && in;
+                unsigned vi = (unsigned)ix * nyz + __umul24((unsigned)iy, (unsigned)g.n[2]) + (unsigned)iz;
+                const unsigned gi = use ? vi : 0u;
+#pragma unroll
+                for (int j = 0; j < NB; ++j) {
+                    sum[j] += (double)((pin ? pv[j] : 0.0f) * pl);
+                    pv[j] = vol[j * vstride + gi];
+                }
+                pin = use;
+                pl = use ? len : 0.0f;
+            };
+            bool across = false;
+            const auto walk = [&](auto fast, auto flat) {
+                constexpr bool F = decltype(fast)::value, D = decltype(flat)::value;
+                Walker W;
+                if (seg == 0) walker_begin(g, R, W);
+                else walker_seek<F>(g, R, W, t0);
+                walk_entries<P2, false, false, F, true, false, D>(g, R, W, t1, visit);
+                across = W.prev > t1;
+            };
+            if constexpr (FLAT) {
+                if (__ballot(R.dST[2] != 0.0f) == 0) walk(Fast<false>{}, Fast<true>{});
+                else walk(Fast<false>{}, Fast<false>{});  // (a third walk would take the ray to scratch memory)
+            } else {
+                walk_dispatch(g, R, [&](auto fast) { walk(fast, Fast<false>{}); });
+            }
+            if (!across) {
+                bad += pbad ? 1 : 0;
+#pragma unroll
+                for (int j = 0; j < NB; ++j) sum[j] += (double)((pin ? pv[j] : 0.0f) * pl);
+            }
+        }
+        if (bad && err) atomicAdd(err, bad);
+    }
+#pragma unroll
+    for (int j = 0; j < NB; ++j) part[(seg * NB + j) * 64 + lane] = sum[j];
+    __syncthreads();
+    if (seg != 0 || r >= nrays) return;
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+        for (int i = 1; i < S; ++i) sum[j] += part[(i * NB + j) * 64 + lane];
+        float res = (float)sum[j];
+        float* sj = sino + j * nrays;
+        if (accumulate) res += sj[r];
+        sirt_store(sirt_item(E, j * nrays), sj, r, res);
+    }
+}
+
 // ------------------------------------------------------------ backward
 
 // Brick geometry shared by all threads of a workgroup for one view.
@@ -361,6 +452,9 @@ __global__ __launch_bounds__(64 * WX * WY) __attribute__((amdgpu_waves_per_eu(NB
     // sub-brick (copies summed in slot order at the end), so rays of
     // different views never meet in one accumulator
     constexpr int LPQ = 64 / NS;
+    // rays in the plane (float64 lists): their own walk of two streams, 512^2,
+    // 720 views 1720 -> 1240 us
+    constexpr bool FLAT = SBZ == 1 && !UNG;
     __shared__ float acc_all[WX * WY * NB * NS * kVox];
     const int wave = threadIdx.x >> 6;
     const int lane = threadIdx.x & 63;
@@ -508,20 +602,28 @@ __global__ __launch_bounds__(64 * WX * WY) __attribute__((amdgpu_waves_per_eu(NB
                     const bool mid = UNG && window_mid(g, R, alo, ahi);
                     if (UNIT) unit_ray(g, R);
                     const GridK& gw = UNIT ? gu : g;
+                    auto visit = [&](int ix, int iy, int iz, float len) {
+                        int lx = ix - b0[0], ly = iy - b0[1], lz = iz - b0[2];
+                        if ((unsigned)lx < (unsigned)(b1[0] - b0[0]) &&
+                            (unsigned)ly < (unsigned)(b1[1] - b0[1]) &&
+                            (unsigned)lz < (unsigned)(b1[2] - b0[2])) {
+                            const int li = (lx * SBY + ly) * SBZ + lz;
+#pragma unroll
+                            for (int j = 0; j < NB; ++j) acc[j * NS * kVox + li] += wgt[j] * len;
+                        }
+                    };
+                    if constexpr (FLAT) {
+                        if (__ballot(R.dST[2] != 0.0f) == 0) {
+                            Walker W;
+                            walker_seek(gw, R, W, alo);
+                            walk_entries<P2, ISO, false, false, false, false, true>(gw, R, W, ahi, visit);
+                            continue;
+                        }
+                    }
                     walk_dispatch<UNG>(gw, R, [&](auto fast) {
                         constexpr bool F = decltype(fast)::value;
                         Walker W;
                         walker_seek<F>(gw, R, W, alo);
-                        auto visit = [&](int ix, int iy, int iz, float len) {
-                            int lx = ix - b0[0], ly = iy - b0[1], lz = iz - b0[2];
-                            if ((unsigned)lx < (unsigned)(b1[0] - b0[0]) &&
-                                (unsigned)ly < (unsigned)(b1[1] - b0[1]) &&
-                                (unsigned)lz < (unsigned)(b1[2] - b0[2])) {
-                                const int li = (lx * SBY + ly) * SBZ + lz;
-#pragma unroll
-                                for (int j = 0; j < NB; ++j) acc[j * NS * kVox + li] += wgt[j] * len;
-                            }
-                        };
                         // windows away from the rays' ends: the walk without
                         // the special values (same entries) when every
                         // walking lane's window qualifies (in the kernels
@@ -601,29 +703,47 @@ struct BpShape {
 // on four views at once, each into its own accumulator copy
 using BpShape3 = BpShape<16, 8, 8, 2, 2, 4, 2>;
 using BpShape2 = BpShape<32, 16, 1, 2, 2, 4, 4>;
+// small 2-D grids: a wave's serial walk bounds the call, so shorter walks
+using BpShape2S = BpShape<16, 16, 1, 1, 1, 4, 4>;
 
 struct BpPlan {
-    int kind;  // 0: 3D sub-bricks, 1: 2D sub-bricks
+    int kind;  // 0: 3D sub-bricks, 1: 2D sub-bricks, 2: the same for small grids
     int sbx, sby, sbz, wx, wy;
     int nbx, nby, nbz;  // workgroup regions (wx*sbx x wy*sby x sbz)
     int nchunks, views_per_chunk;
 };
 
-static BpPlan plan_bp(const GridK& g, int nviews) {
-    BpPlan p;
-    if (g.n[2] == 1) {
-        p.kind = 1; p.sbx = BpShape2::sbx; p.sby = BpShape2::sby; p.sbz = BpShape2::sbz;
-        p.wx = BpShape2::wx; p.wy = BpShape2::wy;
-    } else {
-        p.kind = 0; p.sbx = BpShape3::sbx; p.sby = BpShape3::sby; p.sbz = BpShape3::sbz;
-        p.wx = BpShape3::wx; p.wy = BpShape3::wy;
-    }
+template <class S>
+static void bp_regions(BpPlan& p, const GridK& g) {
+    p.sbx = S::sbx; p.sby = S::sby; p.sbz = S::sbz;
+    p.wx = S::wx; p.wy = S::wy;
     p.nbx = (g.n[0] + p.wx * p.sbx - 1) / (p.wx * p.sbx);
     p.nby = (g.n[1] + p.wy * p.sby - 1) / (p.wy * p.sby);
     p.nbz = (g.n[2] + p.sbz - 1) / p.sbz;
+}
+
+// 2-D grids of fewer than 32 workgroup regions (64 x 32 voxels) take the small
+// shape with as many chunks as there are passes of NS views, up to 4096 waves:
+// n^2, 180 views of 1.45 n bins, small | large in us: 128 60 | 84, 200 93 | 143;
+// 256 (360 views) 242 | 189, 512 812 | 660.
+static BpPlan plan_bp(const GridK& g, int nviews) {
+    BpPlan p;
+    int target = 1024, most = nviews;
+    if (g.n[2] == 1) {
+        p.kind = 1;
+        bp_regions<BpShape2>(p, g);
+        if ((int64_t)p.nbx * p.nby < 32) {
+            p.kind = 2;
+            bp_regions<BpShape2S>(p, g);
+            target = 4096;
+            most = (nviews + 3) / 4;
+        }
+    } else {
+        p.kind = 0;
+        bp_regions<BpShape3>(p, g);
+    }
     int64_t nb = (int64_t)p.nbx * p.nby * p.nbz;
-    const int target = 1024;
-    int nch = (int)std::min<int64_t>(nviews, std::max<int64_t>(1, (target + nb - 1) / nb));
+    int nch = (int)std::min<int64_t>(most, std::max<int64_t>(1, (target + nb - 1) / nb));
     p.views_per_chunk = (nviews + nch - 1) / nch;
     p.nchunks = (nviews + p.views_per_chunk - 1) / p.views_per_chunk;
     return p;
@@ -686,6 +806,21 @@ int vir_siddon_fill(const float* src, const float* trg, int64_t nrays, const vir
     return check_hip(hipGetLastError(), "vir_siddon_fill launch");
 }
 
+// Waves that share a ray's walk.  A wave's walk is a serial chain, so few rays
+// leave the chip idle; from 4096 waves of records in 3-D on, one wave a ray with
+// its special-value-free middle is faster.  Flat sets (rays in the plane have
+// float64 lists and no such middle) always take the split kernel, for its walk
+// of two streams.  One | 4 | 8 waves a ray, us: flat 128^2, 520 waves of rays
+// 105 | 34 | 32, 200^2, 815 159 | 63 | 47, 256^2, 2086 277 | 120 | 118, 512^2, 8347
+// 1030 | 789 | 795, 1024^2, 33390 6650 | 6320 | 6340; 48^3, 1336 31 | 23 | 31, 4010
+// 43 | 46 | 68.  The count depends on the rays alone, so every form of a call
+// (records, batch, fused step) sums alike.
+static int fp_split(int64_t nrays, bool flat) {
+    const int64_t waves = (nrays + 63) / 64;
+    if (flat) return waves < 1024 ? 8 : 4;
+    return waves < 2048 ? 4 : 1;
+}
+
 // The forward projector from endpoints (rec == NULL) or from per-ray
 // records (src == trg == NULL).
 // Largest number of volumes one FP launch traces together; larger batches
@@ -697,6 +832,14 @@ template <int NB>
 static void siddon_fp_launch(const GridK& g, const float* src, const float* trg, const float* rec, int64_t nrays,
                              const float* vol, float* sino, int acc, int32_t* err_count, hipStream_t st,
                              const SirtEpi& E, int64_t nvox, bool p2, bool iso, bool ung) {
+    const bool flat = g.n[2] == 1 && !ung;
+    if (const int S = fp_split(nrays, flat); S > 1) {
+        const auto kern = flat ? (all_pow2(g) ? k_siddon_fp_split<true, true, NB> : k_siddon_fp_split<false, true, NB>)
+                               : (all_pow2(g) ? k_siddon_fp_split<true, false, NB> : k_siddon_fp_split<false, false, NB>);
+        hipLaunchKernelGGL(kern, dim3((unsigned)((nrays + 63) / 64)), dim3(64 * S), 0, st, g, src, trg, rec, nrays, vol,
+                           sino, acc, err_count, E, nvox, S);
+        return;
+    }
     const int64_t nb = (nrays + kRayThreads - 1) / kRayThreads;
 #define VIR_FP_LAUNCH(P2_, ISO_, UNG_)                                                                       \
     hipLaunchKernelGGL((k_siddon_fp<P2_, ISO_, UNG_, NB>), dim3((unsigned)nb), dim3(kRayThreads), 0, st, g,  \
@@ -865,16 +1008,23 @@ static int siddon_bp(const float* src, const float* trg, const float* rec, int32
 #define BP3_WX BpShape3::wx
 #define BP3_WY BpShape3::wy
 #define BP2_ARGS 32, 16, 1, 2, 2, 4, 4
-#define BP2_WX 2
-#define BP2_WY 2
+#define BP2_WX BpShape2::wx
+#define BP2_WY BpShape2::wy
+#define BP2S_ARGS 16, 16, 1, 1, 1, 4, 4
+#define BP2S_WX BpShape2S::wx
+#define BP2S_WY BpShape2S::wy
         if (p.kind == 0) VIR_BP_LAUNCH(BP3);
-        else VIR_BP_LAUNCH(BP2);
+        else if (p.kind == 1) VIR_BP_LAUNCH(BP2);
+        else VIR_BP_LAUNCH(BP2S);
 #undef BP3_ARGS
 #undef BP3_WX
 #undef BP3_WY
 #undef BP2_ARGS
 #undef BP2_WX
 #undef BP2_WY
+#undef BP2S_ARGS
+#undef BP2S_WX
+#undef BP2S_WY
 #undef VIR_BP_ARGS
 #undef VIR_BP_LAUNCH
 #undef VIR_BP_LAUNCH1

@@ -424,12 +424,13 @@ __device__ __forceinline__ void walker_begin(const GridK& g, const Ray& R, Walke
 // Branch-free in the stream choice: one division per step whichever axis
 // advances.  ISO: all three axes share (n, d, origin), so the plane
 // coordinate needs no per-axis selection.
-template <bool ISO, bool FAST, bool UNIT = false>
+// FLAT: every lane's ray has dST = 0 on axis 2 (its stream is empty).
+template <bool ISO, bool FAST, bool UNIT = false, bool FLAT = false>
 __device__ __forceinline__ float walker_pop(const GridK& g, const Ray& R, Walker& W) {
     float h0 = W.h0, h1 = W.h1, h2 = W.h2;
     bool c1 = h1 < h0;
     float hm = c1 ? h1 : h0;
-    bool c2 = h2 < hm;
+    bool c2 = !FLAT && h2 < hm;
     hm = c2 ? h2 : hm;
     W.remaining -= 1;
     // the special value goes first on ties.  Once both are consumed sp is
@@ -562,20 +563,24 @@ __device__ __forceinline__ void walker_seek(const GridK& g, const Ray& R, Walker
 // siddon.py:796-809.  Returns false when the reference drops the entry
 // (length not > 0).  idx holds the truncated index per axis.  P2: every
 // voxel size is a power of two, so dividing by it is a multiplication.
-template <bool P2, bool EXACT, bool FAST = false, bool UNIT = false>
+// FLAT: a float64 list with dST = 0 on axis 2, whose index is the same for
+// every pair (m dST is a zero).
+template <bool P2, bool EXACT, bool FAST = false, bool UNIT = false, bool FLAT = false>
 __device__ __forceinline__ bool segment(const GridK& g, const Ray& R, float a0, float a1,
                                         int idx[3], float& len) {
     // idx: truncated index per axis.  EXACT maps values outside int32 to
     // INT32_MIN as numpy does on x86-64 (needed only where raw indices are
     // returned); otherwise they saturate, which is equally outside the grid
     // (NaN cannot occur: rays with NaN endpoints fail the gate).
-    if (!FAST && R.f64) {
+    if (FLAT || (!FAST && R.f64)) {
         double A0 = (double)a0, A1 = (double)a1;
         double dA = A1 - A0;
         double m = 0.5 * (A1 + A0);
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-            double pos = ((double)R.s[a] + m * (double)R.dST[a]) - (double)g.p0[a];
+            double at = (double)R.s[a];
+            if (!(FLAT && a == 2)) at += m * (double)R.dST[a];
+            double pos = at - (double)g.p0[a];
             double v = P2 ? pos * (double)g.inv_d[a] : pos / (double)g.d[a];
             idx[a] = EXACT ? to_i32_d(v) : (int)v;
         }
@@ -596,9 +601,9 @@ __device__ __forceinline__ bool segment(const GridK& g, const Ray& R, float a0, 
 }
 
 // End-trim tests, siddon.py:789-793 (np.isclose default atol=1e-8).
-template <bool FAST = false>
+template <bool FAST = false, bool FLAT = false>
 __device__ __forceinline__ bool trim_close(const Ray& R, float x, float y) {
-    return (!FAST && R.f64) ? isclose_d((double)x, (double)y, 1e-8) : isclose_f(x, y, 1e-8f);
+    return (FLAT || (!FAST && R.f64)) ? isclose_d((double)x, (double)y, 1e-8) : isclose_f(x, y, 1e-8f);
 }
 
 // Walk the merged list from the current walker state and call
@@ -617,36 +622,36 @@ __device__ __forceinline__ void visit_pair(Visit& visit, const int idx[3], float
 }
 
 template <bool P2, bool ISO, bool EXACT = false, bool FAST = false, bool ALL = false, bool UNIT = false,
-          class Visit>
+          bool FLAT = false, class Visit>
 __device__ __forceinline__ void walk_entries(const GridK& g, const Ray& R, Walker& W,
                                              float a_stop, Visit&& visit) {
     int idx[3];
     float len;
     if (W.consumed == 0) {
         if (W.remaining == 0) return;
-        W.prev = walker_pop<ISO, FAST, UNIT>(g, R, W);
+        W.prev = walker_pop<ISO, FAST, UNIT, FLAT>(g, R, W);
         W.consumed = 1;
     }
     if (W.consumed == 1) {
         if (W.remaining == 0 || W.prev > a_stop) return;
-        float b = walker_pop<ISO, FAST, UNIT>(g, R, W);
-        bool skip = trim_close<FAST>(R, W.prev, b);                   // drop A[0]
-        if (W.remaining == 0) skip |= trim_close<FAST>(R, b, W.prev);  // drop A[-1]
-        bool keep = segment<P2, EXACT, FAST, UNIT>(g, R, W.prev, b, idx, len);
+        float b = walker_pop<ISO, FAST, UNIT, FLAT>(g, R, W);
+        bool skip = trim_close<FAST, FLAT>(R, W.prev, b);                   // drop A[0]
+        if (W.remaining == 0) skip |= trim_close<FAST, FLAT>(R, b, W.prev);  // drop A[-1]
+        bool keep = segment<P2, EXACT, FAST, UNIT, FLAT>(g, R, W.prev, b, idx, len);
         visit_pair<ALL>(visit, idx, len, keep && !skip);
         W.prev = b;
         W.consumed = 2;
     }
     while (W.remaining > 1 && !(W.prev > a_stop)) {
-        float b = walker_pop<ISO, FAST, UNIT>(g, R, W);
-        bool keep = segment<P2, EXACT, FAST, UNIT>(g, R, W.prev, b, idx, len);
+        float b = walker_pop<ISO, FAST, UNIT, FLAT>(g, R, W);
+        bool keep = segment<P2, EXACT, FAST, UNIT, FLAT>(g, R, W.prev, b, idx, len);
         visit_pair<ALL>(visit, idx, len, keep);
         W.prev = b;
     }
     if (W.remaining == 1 && !(W.prev > a_stop)) {
-        float b = walker_pop<ISO, FAST, UNIT>(g, R, W);
-        bool skip = trim_close<FAST>(R, b, W.prev);                    // drop A[-1]
-        bool keep = segment<P2, EXACT, FAST, UNIT>(g, R, W.prev, b, idx, len);
+        float b = walker_pop<ISO, FAST, UNIT, FLAT>(g, R, W);
+        bool skip = trim_close<FAST, FLAT>(R, b, W.prev);                    // drop A[-1]
+        bool keep = segment<P2, EXACT, FAST, UNIT, FLAT>(g, R, W.prev, b, idx, len);
         visit_pair<ALL>(visit, idx, len, keep && !skip);
         W.prev = b;
     }
