@@ -713,6 +713,14 @@ struct BpPlan {
     int nchunks, views_per_chunk;
 };
 
+// Workgroups aimed at for 3-D grids: eight a CU, two rounds of the four that
+// are resident, so that a round's last blocks overlap the next one's; 1024 left
+// the slowest block to bound the call.  Only while the partial volumes fit
+// VIR_SIDDON_BP_SCRATCH_BYTES (a plan that needed more for 1024 keeps those).
+// Projection pair, 100 views of 1.45 n x 1.3 n, 1024 | 2048 in us: 48^3 220 | 185,
+// 64^3 552 | 458, 96^3 784 | 762, 128^3 1790 | 1540; 160^3 has the same plan.
+constexpr int64_t kBp3Target = 2048;
+
 template <class S>
 static void bp_regions(BpPlan& p, const GridK& g) {
     p.sbx = S::sbx; p.sby = S::sby; p.sbz = S::sbz;
@@ -743,8 +751,13 @@ static BpPlan plan_bp(const GridK& g, int nviews) {
         bp_regions<BpShape3>(p, g);
     }
     int64_t nb = (int64_t)p.nbx * p.nby * p.nbz;
-    int nch = (int)std::min<int64_t>(most, std::max<int64_t>(1, (target + nb - 1) / nb));
-    p.views_per_chunk = (nviews + nch - 1) / nch;
+    int64_t nch = (target + nb - 1) / nb;
+    if (p.kind == 0) {
+        const int64_t fit = (int64_t)VIR_SIDDON_BP_SCRATCH_BYTES / ((int64_t)g.n[0] * g.n[1] * g.n[2] * (int64_t)sizeof(float));
+        nch = std::max(nch, std::min((kBp3Target + nb - 1) / nb, fit));
+    }
+    nch = std::min<int64_t>(most, std::max<int64_t>(1, nch));
+    p.views_per_chunk = (int)((nviews + nch - 1) / nch);
     p.nchunks = (nviews + p.views_per_chunk - 1) / p.views_per_chunk;
     return p;
 }
