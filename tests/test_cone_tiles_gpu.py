@@ -92,3 +92,25 @@ def test_infinite_values_stay_where_they_are(kind):
         b = _per_output(P, kind, fp, v, shape)
         assert not torch.isnan(a).any() and torch.isinf(b).any()
         assert torch.equal(torch.isinf(a), torch.isinf(b))
+
+
+@pytest.mark.parametrize("kind", ["dd", "sf"])
+@pytest.mark.parametrize("k", [3, 4, 7, 8])
+def test_infinite_and_nan_voxels_reach_only_their_bins(k, kind):
+    """A voxel's value counts where its weight is not zero, and nowhere else:
+    the bins a unit voxel projects on are the ones an infinite one spoils."""
+    import torch
+    P = _pair(kind, CASES[k])
+    vshape = P.vol_shape if kind == "sf" else P.img_shape
+    x = torch.from_numpy(np.random.default_rng(k).uniform(0.2, 1.0, vshape).astype(np.float32)).cuda()
+    at = [x.numel() // 2 + 3, x.numel() // 3]
+    ones, bad, none = torch.zeros_like(x), x.clone(), x.clone()
+    ones.view(-1)[at] = 1.0
+    none.view(-1)[at] = 0.0
+    bad.view(-1)[at[0]] = float("inf")
+    bad.view(-1)[at[1]] = float("nan")
+    hit, got, ref = P.fp(ones) > 0, P.fp(bad), P.fp(none)
+    assert hit.any() and not hit.all()
+    assert torch.equal(~torch.isfinite(got), hit)
+    # (without its voxel a sum's float64 additions group alike: one rounding)
+    assert torch.allclose(got[~hit], ref[~hit], rtol=3e-7, atol=0)

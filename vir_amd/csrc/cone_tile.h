@@ -23,9 +23,9 @@
 // and bin.  Here a weight is evaluated once per (line, bin) or (view, column)
 // by one lane and read by the wave, lanes run along v (z), and a bin costs
 // one multiply-add in float64 per pixel and row.  Measured, forward /
-// backward: distance driven 128^3, 180 views of 192^2: 5.5 -> 1.5 ms / 2.7 ->
+// backward: distance driven 128^3, 180 views of 192^2: 5.5 -> 0.74 ms / 2.7 ->
 // 0.60 ms; separable footprint 120 x 132 x 101, 150 views of 187 x 150: 8.3 ->
-// 1.6 ms / 2.1 -> 0.53 ms.
+// 1.14 ms / 2.1 -> 0.53 ms.
 #pragma once
 #include "vir_common.h"
 
@@ -35,7 +35,8 @@ constexpr int kCtBins = 16;   // bins of a forward tile, accumulated in register
 constexpr int kCtWaves = 4;   // waves of a forward block: they share a tile's lines
 constexpr int kCtLines = 4;   // lines whose lists a wave builds at once (16 bins x 4 lines = 64 lanes)
 constexpr int kCtPix = 24;    // pixels of a line whose row sums are staged at once
-constexpr int kCtList = 4;    // pixels of a line one bin's list holds
+constexpr int kCtList = 8;    // pixels of a line one bin's list holds
+constexpr int kCtPitch = 68;  // of the row sums in LDS: 16-byte reads of four pixels' rows meet different banks
 constexpr int kCtFoot = 6;    // bins a column's footprint list holds
 
 __device__ __forceinline__ int ct_uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
@@ -80,12 +81,45 @@ __device__ __forceinline__ float ct_sum(const float* __restrict__ p, const float
 // four lines in turn and add their float64 sums in wave order at the end, so
 // the line loop has no barrier.  Per group a lane lists one (line, bin)'s
 // pixels; per line the wave sums each pixel's slabs for its 64 rows into LDS
-// (lane = row; consecutive lanes read consecutive z) and every bin then adds
-// weight * sum for its pixels.
+// (lane = row; consecutive lanes read consecutive z) and multiplies weights
+// and sums on the matrix cores: v_mfma_f64_4x4x4_4b_f64, exact products of
+// float32 factors added in float64, one block for each group of four bins with
+// the pixels that group meets, four a step (two or three steps for pixels about
+// as wide as bins, two fifths of the products of non-zero weight).  Adding bin by
+// bin, with scalar branches and LDS reads in a chain, took 1.50 ms where this takes
+// 0.74 (distance driven, 128^3, 180 views of 192^2; separable footprint, 120 x 132
+// x 101, 150 views of 187 x 150: 1.58 and 1.14).  What bounds it now: vector
+// issue, most of it in the rows' slab sums and, with footprints, the weights.
 struct CtWaveLds {
-    float P[kCtPix * 64];
-    double w[kCtLines * kCtBins * kCtList];
+    float P[kCtPix * kCtPitch];
+    float w[kCtLines * kCtBins * kCtList];
 };
+
+// One bin and row, pixel by pixel.
+template <class M, class Geo, int NS>
+__device__ double ct_fp_one(const Geo& G, const M& V, const float* __restrict__ vol, int iu, int iv) {
+    const float vl = G.dv * (((float)iv - 0.5f * (float)G.nv) + G.sv);
+    const float vr = G.dv * (((float)(iv + 1) - 0.5f * (float)G.nv) + G.sv);
+    const float ul = G.du * (((float)iu - 0.5f * (float)G.nu) + G.su);
+    const float ur = G.du * (((float)(iu + 1) - 0.5f * (float)G.nu) + G.su);
+    const float fu = M::fp_unit(G);
+    double acc = 0.0;
+    for (int io = 0; io < V.no; ++io) {
+        int k0 = 0, k1 = -1;
+        if (!V.range(ul, ur, io, k0, k1)) continue;
+        for (int k = k0; k <= k1; ++k) {
+            const float w = V.weight(k, io, ul, ur);
+            if (!(w > 0.0f)) continue;
+            const float zm = V.zmag(k, io), r = 1.0f / ((M::kLineMag ? V.zmag(0, io) : zm) * G.d);
+            float ws[NS];
+            const int z0 = ct_cells<NS>(vl * r, vr * r, G.nz, ws);
+            const int ix = V.xd ? k : io, iy = V.xd ? io : k;
+            const float p = ct_sum<NS>(vol + ((int64_t)ix * G.ny + iy) * G.nz + z0, ws);
+            acc = __builtin_fma((double)(w * (zm * fu)), (double)p, acc);
+        }
+    }
+    return acc;
+}
 
 template <class M, class Geo, int NS>
 __global__ __launch_bounds__(64 * kCtWaves) __attribute__((amdgpu_waves_per_eu(4))) void k_cone_fp_tile(Geo G, const float* __restrict__ ang,
@@ -94,13 +128,16 @@ __global__ __launch_bounds__(64 * kCtWaves) __attribute__((amdgpu_waves_per_eu(4
                                                                const float* __restrict__ vol,
                                                                float* __restrict__ sino, int accumulate, int nut,
                                                                int nvt) {
-    __shared__ union {
+    __shared__ __attribute__((aligned(16))) union {
         CtWaveLds wave[kCtWaves];
         double red[kCtWaves][kCtBins * 64];
     } lds;
     const int lane = threadIdx.x & 63;
     const int wave = ct_uni(threadIdx.x >> 6);
     CtWaveLds& L = lds.wave[wave];
+    // operand slots: group (matrix block) mid; weights: bin lo, pixel hi; sums:
+    // pixel hi, row quad lo; results: bin hi, row quad lo
+    const int lo = lane & 3, mid = (lane >> 2) & 3, hi = lane >> 4;
     int blk = (int)xcd_remap(blockIdx.x, gridDim.x);
     const int v_lo = (blk % nvt) * 64;
     blk /= nvt;
@@ -118,7 +155,8 @@ __global__ __launch_bounds__(64 * kCtWaves) __attribute__((amdgpu_waves_per_eu(4
     const float ul = G.du * (((float)iul - 0.5f * (float)G.nu) + G.su);
     const float ur = G.du * (((float)(iul + 1) - 0.5f * (float)G.nu) + G.su);
     const float fu = M::fp_unit(G);
-    double acc[kCtBins];
+    const int64_t kstride = (int64_t)(V.xd ? G.ny : 1) * G.nz, lstride = (int64_t)(V.xd ? 1 : G.ny) * G.nz;
+    double acc[kCtBins];  // bin 4 mid + hi, rows 16 c + 4 lo + e at 4 c + e
 #pragma unroll
     for (int i = 0; i < kCtBins; ++i) acc[i] = 0.0;
 
@@ -136,23 +174,37 @@ __global__ __launch_bounds__(64 * kCtWaves) __attribute__((amdgpu_waves_per_eu(4
                     continue;
                 }
                 if (!cnt) kf = k;
-                if (cnt < kCtList) L.w[lane * kCtList + cnt] = (double)(w * (V.zmag(k, io) * fu));
+                if (cnt < kCtList) L.w[lane * kCtList + cnt] = w * (V.zmag(k, io) * fu);
                 ++cnt;
             }
         }
         // more pixels a bin than a list holds (bins much wider than pixels):
         // the line is done in chunks of that many, each listed anew
         const bool over = __any(cnt > kCtList);
+        // the pixels of a group of bins and of the line, and the line's steps
         int b0 = cnt ? kf : 0x7fffffff, b1 = cnt ? kf + cnt - 1 : -1;
 #pragma unroll
-        for (int m = 8; m >= 1; m >>= 1) {
+        for (int m = 2; m >= 1; m >>= 1) {
             b0 = min(b0, __shfl_xor(b0, m));
             b1 = max(b1, __shfl_xor(b1, m));
+        }
+        const int gb = b1 >= 0 ? b0 : 0;
+        int steps = b1 >= 0 ? (b1 - b0 + 4) >> 2 : 0;
+#pragma unroll
+        for (int m = 8; m >= 4; m >>= 1) {
+            b0 = min(b0, __shfl_xor(b0, m));
+            b1 = max(b1, __shfl_xor(b1, m));
+            steps = max(steps, __shfl_xor(steps, m));
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // a wave's LDS accesses are in order
         for (int l = 0; l < kCtLines && g + l < V.no; ++l) {
             const int io = g + l;
             const int kb = __builtin_amdgcn_readlane(b0, 16 * l), ke = __builtin_amdgcn_readlane(b1, 16 * l);
+            if (ke < 0) continue;
+            const int nks = __builtin_amdgcn_readlane(steps, 16 * l);
+            // this operand slot's list
+            const int e = 16 * l + (lane & 15);
+            const int kfe = __shfl(kf, e), cne = __shfl(cnt, e), win = __shfl(gb, e) + hi;
             float ws[NS];
             int z0 = 0;
             if (M::kLineMag) {
@@ -164,49 +216,43 @@ __global__ __launch_bounds__(64 * kCtWaves) __attribute__((amdgpu_waves_per_eu(4
                 const int nk = min(step, ke - kc + 1);
                 if (over && (lane >> 4) == l)
                     for (int k = max(kf, kc); k < min(kf + cnt, kc + nk); ++k)
-                        L.w[lane * kCtList + k - kc] = (double)(V.weight(k, io, ul, ur) * (V.zmag(k, io) * fu));
+                        L.w[lane * kCtList + k - kc] = V.weight(k, io, ul, ur) * (V.zmag(k, io) * fu);
                 float rk = 0.0f;  // lane = pixel
                 if (!M::kLineMag) rk = 1.0f / (V.zmag(min(kc + lane, V.nd - 1), io) * G.d);
-                auto stage = [&](int kk) {
-                    const int k = kc + kk;
-                    const int ix = V.xd ? k : io, iy = V.xd ? io : k;
-                    const float* col = vol + ((int64_t)ix * G.ny + iy) * G.nz;
+                const float* col = vol + (int64_t)io * lstride + (int64_t)kc * kstride;
+                auto stage = [&](int kk, const float* p) {
                     if (!M::kLineMag) {
                         const float r = ct_lane(rk, kk);
                         z0 = ct_cells<NS>(vl * r, vr * r, G.nz, ws);
                     }
-                    return ct_sum<NS>(col + z0, ws);
+                    return ct_sum<NS>(p + z0, ws);
                 };
                 int kk = 0;
-                for (; kk + 3 < nk; kk += 4) {
+                for (; kk + 3 < nk; kk += 4, col += 4 * kstride) {
                     float p[4];
 #pragma unroll
-                    for (int t = 0; t < 4; ++t) p[t] = stage(kk + t);
+                    for (int t = 0; t < 4; ++t) p[t] = stage(kk + t, col + t * kstride);
 #pragma unroll
-                    for (int t = 0; t < 4; ++t) L.P[(kk + t) * 64 + lane] = p[t];
+                    for (int t = 0; t < 4; ++t) L.P[(kk + t) * kCtPitch + lane] = p[t];
                 }
-                for (; kk < nk; ++kk) L.P[kk * 64 + lane] = stage(kk);
+                for (; kk < nk; ++kk, col += kstride) L.P[kk * kCtPitch + lane] = stage(kk, col);
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                const int k0 = over ? kc + hi : win, ns = over ? (nk + 3) >> 2 : nks, wb = over ? kc : kfe;
+                for (int t = 0; t < ns; ++t) {
+                    const int k = k0 + 4 * t, kr = k - kc;
+                    const bool in = (unsigned)(k - kfe) < (unsigned)cne && (unsigned)kr < (unsigned)nk;
+                    if (!__any(in)) continue;  // another chunk's pixels
+                    const double w = in ? (double)L.w[e * kCtList + (k - wb)] : 0.0;
+                    const float4* row = (const float4*)(L.P + min(max(kr, 0), nk - 1) * kCtPitch + 4 * lo);
+                    float4 x[4];
 #pragma unroll
-                for (int i = 0; i < kCtBins; ++i) {
-                    const int e = l * kCtBins + i;
-                    const int f = __builtin_amdgcn_readlane(kf, e) - kc, n = __builtin_amdgcn_readlane(cnt, e);
-                    const int j0 = max(0, -f), j1 = min(n, nk - f);
-                    const float* p = L.P + f * 64 + lane;
-                    const double* w = L.w + e * kCtList + (over ? f : 0);
-                    if (j0 == 0 && j1 == 2) {
-                        const float p0 = p[0], p1 = p[64];
-                        const double w0 = w[0], w1 = w[1];
-                        acc[i] = __builtin_fma(w0, (double)p0, acc[i]);
-                        acc[i] = __builtin_fma(w1, (double)p1, acc[i]);
-                    } else if (j0 == 0 && j1 == 3) {
-                        const float p0 = p[0], p1 = p[64], p2 = p[128];
-                        const double w0 = w[0], w1 = w[1], w2 = w[2];
-                        acc[i] = __builtin_fma(w0, (double)p0, acc[i]);
-                        acc[i] = __builtin_fma(w1, (double)p1, acc[i]);
-                        acc[i] = __builtin_fma(w2, (double)p2, acc[i]);
-                    } else {
-                        for (int j = j0; j < j1; ++j) acc[i] = __builtin_fma(w[j], (double)p[j * 64], acc[i]);
+                    for (int c = 0; c < 4; ++c) x[c] = row[4 * c];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        acc[4 * c] = __builtin_amdgcn_mfma_f64_4x4x4f64(w, (double)x[c].x, acc[4 * c], 0, 0, 0);
+                        acc[4 * c + 1] = __builtin_amdgcn_mfma_f64_4x4x4f64(w, (double)x[c].y, acc[4 * c + 1], 0, 0, 0);
+                        acc[4 * c + 2] = __builtin_amdgcn_mfma_f64_4x4x4f64(w, (double)x[c].z, acc[4 * c + 2], 0, 0, 0);
+                        acc[4 * c + 3] = __builtin_amdgcn_mfma_f64_4x4x4f64(w, (double)x[c].w, acc[4 * c + 3], 0, 0, 0);
                     }
                 }
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -221,9 +267,12 @@ __global__ __launch_bounds__(64 * kCtWaves) __attribute__((amdgpu_waves_per_eu(4
     for (int i = wave; i < kCtBins; i += kCtWaves) {
         const int iu = u_lo + i;
         if (iu >= G.nu) break;
-        double s = lds.red[0][i * 64 + lane];
+        // bin i, row lane: sum 4 (lane / 16) + lane % 4 of slot mid = i / 4, hi = i % 4
+        const int e = (4 * (lane >> 4) + lo) * 64 + 16 * (i & 3) + 4 * (i >> 2) + mid;
+        double s = lds.red[0][e];
 #pragma unroll
-        for (int w = 1; w < kCtWaves; ++w) s += lds.red[w][i * 64 + lane];
+        for (int w = 1; w < kCtWaves; ++w) s += lds.red[w][e];
+        if (!(fabs(s) < (double)VIR_INF)) s = ct_fp_one<M, Geo, NS>(G, V, vol, iu, iv);  // zero weights times infinities
         const int64_t o = ((int64_t)ia * G.nu + iu) * G.nv + iv;
         float r = (float)s * G.out_scale;
         if (accumulate) r += sino[o];
