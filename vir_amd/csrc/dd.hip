@@ -167,7 +167,7 @@ __global__ __launch_bounds__(256) void k_dd2d_fp(DDGeo G, const float* __restric
 template <int MODE>
 struct DDFlat {
     static constexpr int kFixed = 3;
-    static constexpr bool kShared = true, kCentre = false;
+    static constexpr bool kShared = true, kCentre = false, kCorners = false;
     struct Trig {
         float c, s;
         __device__ Trig(float c_, float s_, float) : c(c_), s(s_) {}

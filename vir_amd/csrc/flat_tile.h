@@ -17,6 +17,8 @@
 //   pixel(k, io, u0, u1)    interval of pixel k, returns its own factor (the
 //                           other models)
 //   bp_unit(G)              factor of the quad's factors for overlaps in bins
+//   grid(k, io), amp(k, io) its interval spans the corners grid() of its two
+//                           ends and edges, its factor is amp() (kCorners)
 //   quad(ix, iy, ...)       intervals and factors of a 2 x 2 pixel block
 //
 // The one-thread-per-output kernels repeat the interval of a pixel for every
@@ -27,7 +29,7 @@
 // sums in wave order.  Measured, forward / backward: distance-driven fan 512^2,
 // 720 views of 888 bins: 1.88 -> 0.85 ms / 1.18 -> 0.64 ms (the forward was a
 // tile of 256 bins with two barriers a line pair and waited in 62 % of its
-// cycles); separable-footprint fan 256^2, 360 views of 444: 2.01 -> 0.41 ms /
+// cycles); separable-footprint fan 256^2, 360 views of 444: 2.01 -> 0.37 ms /
 // 0.43 -> 0.10 ms.  VALU work bounds both directions.
 #pragma once
 #include "vir_common.h"
@@ -187,10 +189,41 @@ __global__ __launch_bounds__(64 * NW) void k_fp2d_tile(Geo G, const float* __res
                         if constexpr (M::kShared) {
                             L.e[h][k] = V.edge(min(kc[h] + k, kc[h] + nk[h]), oc[h]);
                             L.v[h][k] = x[h][t];
-                        } else {
+                        } else if constexpr (!M::kCorners) {
                             float u0, u1;
                             const float f = V.pixel(min(kc[h] + k, nd - 1), min(io, no - 1), u0, u1);
                             L.p[h][k] = make_float4(u0, k < nk[h] ? u1 : u0, x[h][t], f);
+                        }
+                    }
+                    if constexpr (M::kCorners) {
+                        // the corners at pixel k's lower end, the line's two
+                        // edges; the next lane's are those at its upper end
+                        // (four divisions a pixel for six: 0.41 -> 0.39 ms)
+                        const int il = min(io, no - 1);
+                        if (nk[h] + kFtPad <= 0) continue;     // whole wave
+                        const bool two = nk[h] + kFtPad > 64;  // whole wave
+                        float lo[2], hi[2];
+#pragma unroll
+                        for (int t = 0; t < 2; ++t) {
+                            lo[t] = hi[t] = 0.0f;
+                            if (t && !two) continue;
+                            const float c0 = V.grid(min(kc[h] + 64 * t + lane, nd), il);
+                            const float c1 = V.grid(min(kc[h] + 64 * t + lane, nd), il + 1);
+                            lo[t] = fminf(c0, c1);
+                            hi[t] = fmaxf(c0, c1);
+                        }
+#pragma unroll
+                        for (int t = 0; t < 2; ++t) {
+                            if (t && !two) continue;
+                            const int k = 64 * t + lane;
+                            float ln = __shfl_down(lo[t], 1), hn = __shfl_down(hi[t], 1);
+                            if (t == 0) {  // (slots 63, if there is no second half, and 127 are empty)
+                                ln = lane == 63 ? ft_lane(lo[1], 0) : ln;
+                                hn = lane == 63 ? ft_lane(hi[1], 0) : hn;
+                            }
+                            const float u0 = fminf(lo[t], ln), u1 = fmaxf(hi[t], hn);
+                            L.p[h][k] = make_float4(u0, k < nk[h] ? u1 : u0, x[h][t],
+                                                    V.amp(min(kc[h] + k, nd - 1), il));
                         }
                     }
                 }
@@ -295,13 +328,17 @@ __global__ __launch_bounds__(64 * NW) void k_bp2d_tile(Geo G, const float* __res
 }
 
 // Waves that share a tile: four, or sixteen (eight forward) where the tiles
-// alone would leave CUs without work.
+// alone would leave CUs without work (forward: in less than about two rounds of
+// resident waves, the edge tiles' short bands leave some idle; four | eight
+// waves, footprint fan pair at 256^2, 360 views, 1440 tiles: 454 | 437 us,
+// distance-driven arc pair with 2 iterations 557 | 541; 400^2, 1800: 819 | 799,
+// 1043 | 1035; 600^2, 2880: no difference).
 template <class M, class Geo>
 int ft_fp(const Geo& G, int nb, const float* ang, const float* cosv, const float* sinv, const float* img,
           float* sino, int acc, hipStream_t st, const SirtEpi& E, const char* what) {
     const int nut = (G.nu + kFtBins - 1) / kFtBins;
     const int64_t n = (int64_t)nb * G.na * nut;
-    if (n >= 1024)
+    if (n >= 2048)
         hipLaunchKernelGGL((k_fp2d_tile<M, Geo, 4>), dim3((unsigned)n), dim3(256), 0, st, G, ang, cosv, sinv, img,
                            sino, acc, nut, E);
     else

@@ -216,7 +216,7 @@ __device__ __forceinline__ float sf_invert(const SFGeo& G, bool xd, float c, flo
 template <int MODE>
 struct SFFlat {
     static constexpr int kFixed = 4;
-    static constexpr bool kShared = false, kCentre = true;
+    static constexpr bool kShared = false, kCentre = true, kCorners = MODE == SF_FAN2;
     struct Trig {
         SFView V;
         __device__ Trig(float c, float s, float ang) {
@@ -262,6 +262,8 @@ struct SFFlat {
         u1 = f.u1;
         return f.amp;
     }
+    __device__ float amp(int k, int io) const { return sf_fan_amp(G, V, xd ? k : io, xd ? io : k, xd ? io : k); }
+    __device__ float grid(int k, int io) const { return xd ? corner(k, io) : corner(io, k); }
     __device__ float corner(int ix, int iy) const {
         const float x = sf_bnd(G.nx, G.d, ix), y = sf_bnd(G.ny, G.d, iy);
         return G.DSD * (-V.s * x + V.c * y) / (G.DSO - (V.c * x + V.s * y));
