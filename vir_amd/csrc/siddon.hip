@@ -820,7 +820,7 @@ int vir_siddon_fill(const float* src, const float* trg, int64_t nrays, const vir
 }
 
 // Waves that share a ray's walk.  A wave's walk is a serial chain, so few rays
-// leave the chip idle; from 4096 waves of records in 3-D on, one wave a ray with
+// leave the chip idle; from about 2048 waves in 3-D on, one wave a ray with
 // its special-value-free middle is faster.  Flat sets (rays in the plane have
 // float64 lists and no such middle) always take the split kernel, for its walk
 // of two streams.  One | 4 | 8 waves a ray, us: flat 128^2, 520 waves of rays
