@@ -83,11 +83,13 @@ __device__ __forceinline__ float dd_scale(const DDGeo& G, const DDView& V, float
 }
 
 // detector coordinate u as the slope t = p / (DSO - o) of its ray (fan), or
-// u itself (parallel): the per-bin part of dd_invert, hoisted out of loops
+// u itself (parallel): the per-bin part of dd_invert, hoisted out of loops.
+// Arc angles end short of 90 degrees, where the slope turns over; pixels lie
+// in front of the source, so no bin edge past that meets one.
 template <int MODE>
 __device__ __forceinline__ float dd_slope(const DDGeo& G, float u) {
     if (MODE == DD_PAR) return u;
-    return MODE == DD_FAN_FLAT ? u / G.DSD : tanf(u / G.DSD);
+    return MODE == DD_FAN_FLAT ? u / G.DSD : tanf(fminf(fmaxf(u / G.DSD, -1.57f), 1.57f));
 }
 
 // inverse of dd_bound along the driving axis: the drive coordinate whose
@@ -100,19 +102,40 @@ __device__ __forceinline__ float dd_invert(const DDGeo& G, const DDView& V, floa
     return (t * (G.DSO - oo) - po) / (V.pd + t * V.od);
 }
 
-// dd_invert as x = A - oc B for a fixed slope t (the tiled forward's range).
-// The inverse only bounds pixel ranges, which are widened by its rounding.
+// dd_invert's denominator, zero for rays along the driving axis: such a ray
+// makes 45 degrees or more with the central one
 template <int MODE>
-__device__ __forceinline__ void dd_invert_lin(const DDGeo& G, const DDView& V, float t, float& A, float& B) {
-    if (MODE == DD_PAR) {
-        const float r = 1.0f / V.pd;
-        A = t * r;
-        B = V.po * r;
-    } else {
-        const float r = 1.0f / (V.pd + t * V.od);
-        A = t * G.DSO * r;
-        B = (t * V.oo + V.po) * r;
-    }
+__device__ __forceinline__ float dd_den(const DDView& V, float t) {
+    return MODE == DD_PAR ? V.pd : V.pd + t * V.od;
+}
+
+// dd_invert as x = A - oc B for a fixed slope t (the tiled forward's range);
+// returns dd_den.
+template <int MODE>
+__device__ __forceinline__ float dd_invert_lin(const DDGeo& G, const DDView& V, float t, float& A, float& B) {
+    const float den = dd_den<MODE>(V, t), r = 1.0f / den;
+    A = MODE == DD_PAR ? t * r : t * G.DSO * r;
+    B = MODE == DD_PAR ? V.po * r : (t * V.oo + V.po) * r;
+    return den;
+}
+
+// Pixels [k0, k1] of line oc whose boundaries can project between the slopes
+// tl and tr of a bin, widened by one for rounding (false: none).  A bin with
+// a ray along the driving axis between its edges (or about there) takes the
+// whole line: the inverse runs through infinity inside it.
+template <int MODE>
+__device__ __forceinline__ bool dd_pixels(const DDGeo& G, const DDView& V, float tl, float tr, float oc, int nd,
+                                          int& k0, int& k1) {
+    k0 = 0;
+    k1 = nd - 1;
+    if (MODE != DD_PAR && !(dd_den<MODE>(V, tl) * dd_den<MODE>(V, tr) > 1e-6f)) return true;
+    const float inv_d = 1.0f / G.d;
+    const float x0 = dd_invert<MODE>(G, V, tl, oc), x1 = dd_invert<MODE>(G, V, tr, oc);
+    const float k0f = fminf(x0, x1) * inv_d + 0.5f * (float)nd, k1f = fmaxf(x0, x1) * inv_d + 0.5f * (float)nd;
+    if (!(k0f < (float)nd + 2.0f) || !(k1f > -2.0f)) return false;
+    k0 = (int)fmaxf(floorf(k0f) - 1.0f, 0.0f);
+    k1 = (int)fminf(floorf(k1f) + 1.0f, (float)(nd - 1));
+    return true;
 }
 
 __device__ __forceinline__ float overlap(float a0, float a1, float b0, float b1) {
@@ -134,16 +157,11 @@ __global__ __launch_bounds__(256) void k_dd2d_fp(DDGeo G, const float* __restric
     const int nd = V.xd ? G.nx : G.ny, no = V.xd ? G.ny : G.nx;
     const float ul = det_bnd(G.nu, G.du, G.su, iu), ur = det_bnd(G.nu, G.du, G.su, iu + 1);
     const float tl = dd_slope<MODE>(G, ul), tr = dd_slope<MODE>(G, ur);
-    const float inv_d = 1.0f / G.d;
     double acc = 0.0;
     for (int io = 0; io < no; ++io) {
         const float oc = cell_cen(no, G.d, io);
-        float x0 = dd_invert<MODE>(G, V, tl, oc), x1 = dd_invert<MODE>(G, V, tr, oc);
-        float k0f = fminf(x0, x1) * inv_d + 0.5f * (float)nd;
-        float k1f = fmaxf(x0, x1) * inv_d + 0.5f * (float)nd;
-        int k0 = (int)fmaxf(floorf(k0f) - 1.0f, 0.0f);
-        int k1 = (int)fminf(floorf(k1f) + 1.0f, (float)(nd - 1));
-        if (!(k0f < (float)nd + 2.0f) || !(k1f > -2.0f)) continue;
+        int k0, k1;
+        if (!dd_pixels<MODE>(G, V, tl, tr, oc, nd, k0, k1)) continue;
         const float sc = dd_scale<MODE>(G, V, oc);
         float pb = dd_bound<MODE>(G, V, cell_bnd(nd, G.d, k0), oc);
         for (int k = k0; k <= k1; ++k) {
@@ -188,13 +206,11 @@ struct DDFlat {
         }
     }
     __device__ float centre(int io) const { return cell_cen(no, G.d, io); }
-    // bins past the grid's shadow are inverted at its rim (the inverse turns
-    // over at 45 degrees, and they meet no pixel)
-    __device__ void lin(float u, float& A, float& B) const {
+    // bins past the grid's shadow, which meet no pixel, are inverted at its rim
+    __device__ float lin(float u, float& A, float& B) const {
         float t = dd_slope<MODE>(G, u);
-        if (MODE == DD_FAN_ARC && fabsf(u) > 1.5f * G.DSD) t = u > 0.0f ? tmax : -tmax;
         if (MODE != DD_PAR) t = fminf(fmaxf(t, -tmax), tmax);
-        dd_invert_lin<MODE>(G, V, t, A, B);
+        return dd_invert_lin<MODE>(G, V, t, A, B);
     }
     __device__ float margin() const { return 0.0f; }
     __device__ float line_factor(float oc) const { return dd_scale<MODE>(G, V, oc); }
@@ -284,14 +300,8 @@ struct DDCone {
         no = xd ? G.ny : G.nx;
     }
     __device__ bool range(float ul, float ur, int io, int& k0, int& k1) const {
-        const float oc = cell_cen(no, G.d, io), inv_d = 1.0f / G.d;
-        const float x0 = dd_invert<DD_FAN_FLAT>(G, V, dd_slope<DD_FAN_FLAT>(G, ul), oc);
-        const float x1 = dd_invert<DD_FAN_FLAT>(G, V, dd_slope<DD_FAN_FLAT>(G, ur), oc);
-        const float k0f = fminf(x0, x1) * inv_d + 0.5f * (float)nd, k1f = fmaxf(x0, x1) * inv_d + 0.5f * (float)nd;
-        if (!(k0f < (float)nd + 2.0f) || !(k1f > -2.0f)) return false;
-        k0 = (int)fmaxf(floorf(k0f) - 1.0f, 0.0f);
-        k1 = (int)fminf(floorf(k1f) + 1.0f, (float)(nd - 1));
-        return true;
+        return dd_pixels<DD_FAN_FLAT>(G, V, dd_slope<DD_FAN_FLAT>(G, ul), dd_slope<DD_FAN_FLAT>(G, ur),
+                                      cell_cen(no, G.d, io), nd, k0, k1);
     }
     __device__ void foot(int k, int io, float& lo, float& hi) const {
         const float oc = cell_cen(no, G.d, io);
@@ -328,15 +338,11 @@ __global__ __launch_bounds__(256) void k_ddcone_fp(DDGeo G, const float* __restr
     double acc = 0.0;
     for (int io = 0; io < no; ++io) {
         const float oc = cell_cen(no, G.d, io);
-        float x0 = dd_invert<DD_FAN_FLAT>(G, V, tl, oc), x1 = dd_invert<DD_FAN_FLAT>(G, V, tr, oc);
-        float k0f = fminf(x0, x1) * inv_d + 0.5f * (float)nd;
-        float k1f = fmaxf(x0, x1) * inv_d + 0.5f * (float)nd;
-        if (!(k0f < (float)nd + 2.0f) || !(k1f > -2.0f)) continue;
+        int k0, k1;
+        if (!dd_pixels<DD_FAN_FLAT>(G, V, tl, tr, oc, nd, k0, k1)) continue;
         const float zm = cone_zmag(G, V, oc);
         float z0f = vl / zm * inv_d + 0.5f * (float)G.nz, z1f = vr / zm * inv_d + 0.5f * (float)G.nz;
         if (!(z0f < (float)G.nz + 2.0f) || !(z1f > -2.0f)) continue;
-        int k0 = (int)fmaxf(floorf(k0f) - 1.0f, 0.0f);
-        int k1 = (int)fminf(floorf(k1f) + 1.0f, (float)(nd - 1));
         int z0 = (int)fmaxf(floorf(z0f) - 1.0f, 0.0f);
         int z1 = (int)fminf(floorf(z1f) + 1.0f, (float)(G.nz - 1));
         const float sc = dd_scale<DD_FAN_FLAT>(G, V, oc);
@@ -381,7 +387,7 @@ __global__ __launch_bounds__(256) void k_ddcone_fp_compat(DDGeo G, const float* 
     const float u0 = det_bnd(G.nu, G.du, G.su, 0), v0 = det_bnd(G.nv, G.dv, G.sv, 0);
     const float ul = det_bnd(G.nu, G.du, G.su, iu), ur = det_bnd(G.nu, G.du, G.su, iu + 1);
     const float tl = dd_slope<DD_FAN_FLAT>(G, ul), tr = dd_slope<DD_FAN_FLAT>(G, ur);
-    const float inv_d = 1.0f / G.d, inv_du = 1.0f / G.du, inv_dv = 1.0f / G.dv;
+    const float inv_du = 1.0f / G.du, inv_dv = 1.0f / G.dv;
     float* row = sino + t * G.nv;
     if (!accumulate)
         for (int iv = 0; iv < G.nv; ++iv) row[iv] = 0.0f;
@@ -399,11 +405,8 @@ __global__ __launch_bounds__(256) void k_ddcone_fp_compat(DDGeo G, const float* 
         const float zm = cone_zmag(G, V, oc);
         const float sc = dd_scale<DD_FAN_FLAT>(G, V, oc);
         // pixels of this line whose shadows can meet the bin
-        float x0 = dd_invert<DD_FAN_FLAT>(G, V, tl, oc), x1 = dd_invert<DD_FAN_FLAT>(G, V, tr, oc);
-        const float k0f = fminf(fmaxf(fminf(x0, x1) * inv_d + 0.5f * (float)nd, -4.0f), (float)nd + 4.0f);
-        const float k1f = fminf(fmaxf(fmaxf(x0, x1) * inv_d + 0.5f * (float)nd, -4.0f), (float)nd + 4.0f);
-        const int k0 = (int)fmaxf(floorf(k0f) - 1.0f, 0.0f);
-        const int k1 = (int)fminf(floorf(k1f) + 1.0f, (float)(nd - 1));
+        int k0, k1;
+        if (!dd_pixels<DD_FAN_FLAT>(G, V, tl, tr, oc, nd, k0, k1)) k1 = -1;
         for (int iz = 0; iz < G.nz; ++iz) {
             const float zl = zm * cell_bnd(G.nz, G.d, iz), zr = zm * cell_bnd(G.nz, G.d, iz + 1);
             const float ga = fminf(fmaxf((zl - v0) * inv_dv, -1.0f), (float)G.nv + 1.0f);

@@ -7,7 +7,8 @@
 //   xd, nd, no              driving axis, pixels a line, lines
 //   centre(io)              orthogonal coordinate of line io
 //   lin(u, A, B)            detector coordinate u inverted along a line with
-//                           coordinate oc: pixel position A - oc B
+//                           coordinate oc: pixel position A - oc B; returns
+//                           the denominator, zero for rays along the line
 //   margin()                largest distance of a pixel's interval end from
 //                           the position lin() inverts (kCentre models: of
 //                           its centre; others invert pixel edges, margin 0)
@@ -75,26 +76,29 @@ __global__ __launch_bounds__(64 * NW) void k_fp2d_tile(Geo G, const float* __res
     const M V(G, typename M::Trig(cs[ia], sn[ia], ang ? ang[ia] : 0.0f));
     const int nd = V.nd, no = V.no;
     const float half = 0.5f * (float)nd, inv_d = 1.0f / G.d;
-    // rounding of a pixel position (a sum of terms as large as the image)
-    const float eps = 2e-3f + 2e-6f * (float)(nd + no);
     const auto edge = [&](int j) { return G.du * (((float)j - 0.5f * (float)G.nu) + G.su); };
-    // pixel range of the interval [u0, u1]: position p0 - oc q0 .. p1 - oc q1
-    struct Inv { float p0, q0, p1, q1; };
+    // pixel range of the interval [u0, u1]: position p0 - oc q0 .. p1 - oc q1,
+    // widened by eps for the rounding of a position (a sum of such terms).  An
+    // interval with a ray along the line inside, where positions run through
+    // infinity, takes the whole line.
+    struct Inv { float p0, q0, p1, q1, eps; };
     const auto invert = [&](float u0, float u1) {
         Inv r;
-        V.lin(u0 - V.margin(), r.p0, r.q0);
-        V.lin(u1 + V.margin(), r.p1, r.q1);
+        const float e0 = V.lin(u0 - V.margin(), r.p0, r.q0), e1 = V.lin(u1 + V.margin(), r.p1, r.q1);
+        if (!(e0 * e1 > 1e-6f)) return Inv{-1e9f, 0.0f, 1e9f, 0.0f, 0.0f};
         const float c = M::kCentre ? half - 0.5f : half;
         r.p0 = __builtin_fmaf(r.p0, inv_d, c);
         r.p1 = __builtin_fmaf(r.p1, inv_d, c);
         r.q0 *= inv_d;
         r.q1 *= inv_d;
+        r.eps = 2e-3f + 2e-6f * (float)(nd + no) +
+                4e-7f * (fmaxf(fabsf(r.p0), fabsf(r.p1)) + 0.5f * (float)no * fmaxf(fabsf(r.q0), fabsf(r.q1)));
         return r;
     };
     const auto range = [&](const Inv& r, float oc, float& a, float& b) {
         const float x0 = __builtin_fmaf(-oc, r.q0, r.p0), x1 = __builtin_fmaf(-oc, r.q1, r.p1);
-        a = fminf(x0, x1) - eps;
-        b = floorf(fmaxf(x0, x1) + eps);
+        a = fminf(x0, x1) - r.eps;
+        b = floorf(fmaxf(x0, x1) + r.eps);
         a = M::kCentre ? ceilf(a) : floorf(a);
     };
     float ul[2], ur[2];

@@ -247,12 +247,13 @@ struct SFFlat {
         no = xd ? G.ny : G.nx;
     }
     __device__ float centre(int io) const { return (sf_bnd(no, G.d, io) + sf_bnd(no, G.d, io + 1)) * 0.5f; }
-    __device__ void lin(float u, float& A, float& B) const {
+    __device__ float lin(float u, float& A, float& B) const {
         const float pd = xd ? -V.s : V.c, po = xd ? V.c : -V.s;
         const float od = xd ? V.c : V.s, oo = xd ? V.s : V.c;
-        const float t = MODE == SF_PAR2 ? u : u / G.DSD, r = 1.0f / (MODE == SF_PAR2 ? pd : pd + t * od);
+        const float t = MODE == SF_PAR2 ? u : u / G.DSD, den = MODE == SF_PAR2 ? pd : pd + t * od, r = 1.0f / den;
         A = MODE == SF_PAR2 ? t * r : t * G.DSO * r;
         B = MODE == SF_PAR2 ? po * r : (t * oo + po) * r;
+        return den;
     }
     __device__ float margin() const { return G.wmax; }
     __device__ float line_factor(float) const { return 1.0f / G.du; }
