@@ -242,7 +242,7 @@ struct DDFlat {
                 f[2 * i + j] = xd ? sc[j] : sc[i];
             }
     }
-    __host__ __device__ static float bp_unit(const DDGeo& g) { return g.du; }
+    __host__ __device__ static float bp_unit(const DDGeo&) { return 1.0f; }
 };
 
 // One thread per pixel.

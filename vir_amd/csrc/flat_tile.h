@@ -17,7 +17,7 @@
 //                           line share their edges)
 //   pixel(k, io, u0, u1)    interval of pixel k, returns its own factor (the
 //                           other models)
-//   bp_unit(G)              factor of the quad's factors for overlaps in bins
+//   bp_unit(G)              factor of the quad's factors (backward)
 //   grid(k, io), amp(k, io) its interval spans the corners grid() of its two
 //                           ends and edges, its factor is amp() (kCorners)
 //   quad(ix, iy, ...)       intervals and factors of a 2 x 2 pixel block
@@ -259,8 +259,7 @@ __global__ __launch_bounds__(64 * NW) void k_fp2d_tile(Geo G, const float* __res
 // --------------------------------------------------------------- backward
 //
 // A block takes 16 x 16 pixels, a 2 x 2 block a lane; wave w of its NW takes
-// views w, w + NW, ...  Overlaps are formed in bins from the detector's
-// centre.
+// views w, w + NW, ...
 template <class M, class Geo, int NW>
 __global__ __launch_bounds__(64 * NW) void k_bp2d_tile(Geo G, const float* __restrict__ ang,
                                                       const float* __restrict__ cs, const float* __restrict__ sn,
@@ -275,6 +274,9 @@ __global__ __launch_bounds__(64 * NW) void k_bp2d_tile(Geo G, const float* __res
     const int bx = (tile / nty) * 16, by = (tile % nty) * 16;
     const int ix = bx + 2 * (lane >> 3), iy = by + 2 * (lane & 7);
     const float inv_du = 1.0f / G.du, half = 0.5f * (float)G.nu;
+    // u in bins from the first one's edge, and its rounding
+    const float off = half - G.su, mar = 1e-4f + 1e-6f * ((float)G.nu + fabsf(G.su));
+    const float uend = G.du * (half + G.su);
     double acc[4] = {0.0, 0.0, 0.0, 0.0};
     for (int g = 0; g < G.na; g += 64 * NW) {
         const int il = min(g + NW * lane + wave, G.na - 1);
@@ -289,33 +291,36 @@ __global__ __launch_bounds__(64 * NW) void k_bp2d_tile(Geo G, const float* __res
             float y[4][3];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                lo[q] = __builtin_fmaf(lo[q], inv_du, -G.su);
-                hi[q] = fminf(__builtin_fmaf(hi[q], inv_du, -G.su), half);
-                const float j = fminf(fmaxf(floorf(lo[q] + half), 0.0f), (float)(G.nu - 1));
+                hi[q] = fminf(hi[q], uend);
+                const float j = fminf(fmaxf(floorf(__builtin_fmaf(lo[q], inv_du, off) - mar), 0.0f), (float)(G.nu - 1));
                 j0[q] = (int)j;
-                n[q] = (int)fminf(hi[q] + half, (float)(G.nu - 1)) - j0[q];  // bins past the first
+                n[q] = (int)fminf(__builtin_fmaf(hi[q], inv_du, off) + mar, (float)(G.nu - 1)) - j0[q];  // bins past the first
 #pragma unroll
                 for (int t = 0; t < 3; ++t) y[q][t] = row[min(j0[q] + t, G.nu - 1)];
             }
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                float s = 0.0f, e = (float)j0[q] - half;
+                double s = 0.0;
+                // neighbouring bins share the rounded edge between them, so a
+                // pixel's overlaps add up to its interval
+                float k = ((float)j0[q] - half) + G.su, e = G.du * k;
                 const auto term = [&](float v) {
-                    const float ov = fminf(hi[q], e + 1.0f) - fmaxf(lo[q], e);
-                    s = __builtin_fmaf(ov > 0.0f ? v : 0.0f, fmaxf(ov, 0.0f), s);
-                    e += 1.0f;
+                    k += 1.0f;
+                    const float e1 = G.du * k, ov = fminf(hi[q], e1) - fmaxf(lo[q], e);
+                    s += (double)(ov > 0.0f ? v * ov : 0.0f);
+                    e = e1;
                 };
 #pragma unroll
                 for (int t = 0; t < 3; ++t) term(y[q][t]);
                 for (int t = 3; t <= n[q]; ++t) term(row[j0[q] + t]);
-                acc[q] = __builtin_fma((double)s, (double)f[q], acc[q]);
+                acc[q] = __builtin_fma(s, (double)f[q], acc[q]);
             }
         }
     }
 #pragma unroll
     for (int q = 0; q < 4; ++q) red[wave][64 * q + lane] = acc[q];
     __syncthreads();
-    const float unit = G.out_scale * M::bp_unit(G);
+    const double unit = (double)M::bp_unit(G);
     for (int i = threadIdx.x; i < 256; i += 64 * NW) {
         // consecutive threads, consecutive pixels: px (i / 16, i % 16)
         const int x = i >> 4, y = i & 15;
@@ -325,7 +330,7 @@ __global__ __launch_bounds__(64 * NW) void k_bp2d_tile(Geo G, const float* __res
 #pragma unroll
         for (int w = 1; w < NW; ++w) s += red[w][slot];
         const int64_t o = (item * G.nx + bx + x) * G.ny + by + y;
-        float r = (float)s * unit;
+        float r = (float)(s * unit) * G.out_scale;
         if (accumulate) r += img[o];
         sirt_store(E, img, o, r);
     }

@@ -293,7 +293,7 @@ struct SFFlat {
             f[q] = sf_fan_amp(G, V, ix + i, iy + j, iy + j);
         }
     }
-    __host__ __device__ static float bp_unit(const SFGeo&) { return 1.0f; }
+    __host__ __device__ static float bp_unit(const SFGeo& g) { return 1.0f / g.du; }
 };
 
 // One view of the cone geometry as cone_tile.h's model: weights and ranges of
