@@ -32,3 +32,35 @@ def test_backprojection_over_many_bins(per, su, kind):
     ref = sum((y[:, first + k:first + k + n * per:per].astype(np.float64) * w[k]).sum(0) for k in range(per + 1))
     out = P.bp(torch.from_numpy(y).cuda()).cpu().numpy()
     assert np.array_equal(out, np.broadcast_to(ref.astype(np.float32), (5, n)))
+
+
+def test_cone_rows_over_several_slabs():
+    """One line of pixels at magnification 2, each on one bin; a row meets half
+    a slab, a whole one and another half."""
+    import torch
+    from vir_amd.sys_mat.dd import DDProjector
+    n, nz, na = 24, 66, 2
+    P = DDProjector((1, n, nz), np.zeros(na), n, "cone", nv=33, DSO=4096.0, DSD=8192.0, du=2.0, dv=4.0, sv=0.25)
+    x = _values((1, n, nz), 1)
+    zb = np.arange(nz + 1) - nz / 2.0
+    vb = 2.0 * (np.arange(34) - 16.5 + 0.25)                 # row edges in slabs
+    W = np.clip(np.minimum(zb[1:, None], vb[None, 1:]) - np.maximum(zb[:-1, None], vb[None, :-1]), 0.0, None)
+    ref = x[0].astype(np.float64) @ W / 2.0                  # over the row's two slabs
+    out = P.fp(torch.from_numpy(x).cuda()).cpu().numpy()
+    assert np.array_equal(out, np.broadcast_to(ref.astype(np.float32), (na, n, 33)))
+
+
+def test_cone_slabs_over_several_rows():
+    """The same line backprojected: a slab meets half a row, a whole one and
+    another half."""
+    import torch
+    from vir_amd.sys_mat.dd import DDProjector
+    n, nz, na = 24, 40, 3
+    P = DDProjector((1, n, nz), np.zeros(na), n, "cone", nv=82, DSO=4096.0, DSD=8192.0, du=2.0, dv=1.0, sv=0.5)
+    y = _values(P.sino_shape, 2)
+    zb = 2.0 * (np.arange(nz + 1) - nz / 2.0)                # slab edges in rows
+    vb = np.arange(83) - 41.0 + 0.5
+    W = np.clip(np.minimum(zb[1:, None], vb[None, 1:]) - np.maximum(zb[:-1, None], vb[None, :-1]), 0.0, None)
+    ref = y.astype(np.float64).sum(0) @ W.T                  # (24, 82) x (82, 40)
+    out = P.bp(torch.from_numpy(y).cuda()).cpu().numpy()
+    assert np.array_equal(out, ref.astype(np.float32)[None])

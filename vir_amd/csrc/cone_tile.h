@@ -13,19 +13,20 @@
 //   weight(k, io, lo, hi)              w of pixel k for those edges, <= 0: none
 //   zmag(k, io)                        z magnification
 //   foot(k, io, lo, hi)                the pixel's interval along u
-//   fp_unit(G), bp_unit(G)             factors of w for v overlaps in slabs
-//                                      (times zmag) and in rows
+//   fp_unit(G), bp_unit(G)             factors of w for v overlaps in detector
+//                                      units and in rows
 // and G the sizes nx, ny, nz, nu, nv, na, spacings d, du, dv, offsets su, sv
 // and out_scale.
 //
 // The one-thread-per-output kernels evaluate every weight, v overlaps
 // included, for each (bin, voxel) pair: about 200 VALU instructions a pixel
 // and bin.  Here a weight is evaluated once per (line, bin) or (view, column)
-// by one lane and read by the wave, lanes run along v (z), and a bin costs
-// one multiply-add in float64 per pixel and row.  Measured, forward /
-// backward: distance driven 128^3, 180 views of 192^2: 5.5 -> 0.74 ms / 2.7 ->
-// 0.60 ms; separable footprint 120 x 132 x 101, 150 views of 187 x 150: 8.3 ->
-// 1.14 ms / 2.1 -> 0.53 ms.
+// by one lane and read by the wave, and lanes run along v (z): forward, a
+// pixel's slabs are summed once for each of its rows and the bins' sums are
+// matrix products; backward, a bin costs its rows' sum and one multiply-add.
+// All sums are held in float64.  Measured, forward / backward: distance driven
+// 128^3, 180 views of 192^2: 5.5 -> 0.82 ms / 2.7 -> 0.59 ms; separable footprint
+// 120 x 132 x 101, 150 views of 187 x 150: 8.3 -> 0.98 ms / 2.1 -> 0.55 ms.
 #pragma once
 #include "vir_common.h"
 
@@ -34,7 +35,7 @@ namespace vir {
 constexpr int kCtBins = 16;   // bins of a forward tile, accumulated in registers
 constexpr int kCtWaves = 4;   // waves of a forward block: they share a tile's lines
 constexpr int kCtLines = 4;   // lines whose lists a wave builds at once (16 bins x 4 lines = 64 lanes)
-constexpr int kCtPix = 24;    // pixels of a line whose row sums are staged at once
+constexpr int kCtPix = 20;    // pixels of a line whose row sums are staged at once
 constexpr int kCtList = 8;    // pixels of a line one bin's list holds
 constexpr int kCtPitch = 68;  // of the row sums in LDS: 16-byte reads of four pixels' rows meet different banks
 constexpr int kCtFoot = 6;    // bins a column's footprint list holds
@@ -44,34 +45,64 @@ __device__ __forceinline__ float ct_lane(float x, int l) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
 }
 
-// Overlaps w[0 .. NS-1] of [a, b] with the unit cells first, first + 1, ... of
-// n >= NS cells whose edges lie at k - n/2.  Covers every cell of positive
-// overlap when b - a <= NS - 1.01 (the launch checks that): an interval of
-// length L meets at most floor(L) + 2 cells.
+// First of the NS cells, of n >= NS, that an interval of at most NS - 1.01 cells
+// (the launch checks that) from cell coordinate a on can meet: an interval of
+// length L meets at most floor(L) + 2 cells.  a may be rounded.
 template <int NS>
-__device__ __forceinline__ int ct_cells(float a, float b, int n, float (&w)[NS]) {
-    const float half = 0.5f * (float)n;
-    const float f = fminf(fmaxf(floorf(a + half), 0.0f), (float)(n - NS));
+__device__ __forceinline__ float ct_first(float a, int n) {
+    return fminf(fmaxf(floorf(a - (1e-3f + 4e-7f * (float)n)), 0.0f), (float)(n - NS));
+}
+
+// Overlaps w[0 .. NS-1] of [a, b] with the unit cells first, first + 1, ... of
+// n cells whose edges lie at k - n/2.
+template <int NS>
+__device__ __forceinline__ int ct_cells(float a, float b, int n, double (&w)[NS]) {
+    const float half = 0.5f * (float)n, f = ct_first<NS>(a + half, n);
     float e = f - half;
 #pragma unroll
     for (int q = 0; q < NS; ++q) {
         const float e1 = e + 1.0f;
-        w[q] = fmaxf(fminf(e1, b) - fmaxf(e, a), 0.0f);
+        w[q] = (double)fmaxf(fminf(e1, b) - fmaxf(e, a), 0.0f);
         e = e1;
     }
     return (int)f;
 }
 
-// Weighted sum of NS consecutive values; values of zero weight do not count
-// (they may be infinite).
+// The same of the detector interval [a, b] and cells of height h = 1/r on the
+// detector, with edges at h (k - n/2): neighbouring cells share the rounded
+// edge between them, so that the overlaps of an interval add up to its length.
 template <int NS>
-__device__ __forceinline__ float ct_sum(const float* __restrict__ p, const float (&w)[NS]) {
+__device__ __forceinline__ int ct_slabs(float a, float b, float h, float r, int n, double (&w)[NS]) {
+    const float half = 0.5f * (float)n, f = ct_first<NS>(__builtin_fmaf(a, r, half), n), k = f - half;
+    float e = h * k;
+#pragma unroll
+    for (int q = 0; q < NS; ++q) {
+        const float e1 = h * (k + (float)(q + 1));
+        w[q] = (double)fmaxf(fminf(e1, b) - fmaxf(e, a), 0.0f);
+        e = e1;
+    }
+    return (int)f;
+}
+
+// Weighted sum of NS consecutive values, in float64.
+template <int NS>
+__device__ __forceinline__ double ct_sum(const float* __restrict__ p, const double (&w)[NS]) {
     float x[NS];
 #pragma unroll
     for (int q = 0; q < NS; ++q) x[q] = p[q];
-    float s = 0.0f;
+    double s = (double)x[0] * w[0];
 #pragma unroll
-    for (int q = 0; q < NS; ++q) s = __builtin_fmaf(w[q] > 0.0f ? x[q] : 0.0f, w[q], s);
+    for (int q = 1; q < NS; ++q) s = __builtin_fma((double)x[q], w[q], s);
+    return s;
+}
+
+// The same where values of zero weight may be infinite: they do not count.
+template <int NS>
+__device__ __forceinline__ double ct_sum_some(const float* __restrict__ p, const double (&w)[NS]) {
+    double s = 0.0;
+#pragma unroll
+    for (int q = 0; q < NS; ++q)
+        if (w[q] > 0.0) s = __builtin_fma((double)p[q], w[q], s);
     return s;
 }
 
@@ -82,16 +113,18 @@ __device__ __forceinline__ float ct_sum(const float* __restrict__ p, const float
 // the line loop has no barrier.  Per group a lane lists one (line, bin)'s
 // pixels; per line the wave sums each pixel's slabs for its 64 rows into LDS
 // (lane = row; consecutive lanes read consecutive z) and multiplies weights
-// and sums on the matrix cores: v_mfma_f64_4x4x4_4b_f64, exact products of
-// float32 factors added in float64, one block for each group of four bins with
-// the pixels that group meets, four a step (two or three steps for pixels about
-// as wide as bins, two fifths of the products of non-zero weight).  Adding bin by
-// bin, with scalar branches and LDS reads in a chain, took 1.50 ms where this takes
-// 0.74 (distance driven, 128^3, 180 views of 192^2; separable footprint, 120 x 132
-// x 101, 150 views of 187 x 150: 1.58 and 1.14).  What bounds it now: vector
+// and sums on the matrix cores: v_mfma_f64_4x4x4_4b_f64, one block for each
+// group of four bins with the pixels that group meets, four a step (two or
+// three steps for pixels about as wide as bins, two fifths of the products of
+// non-zero weight).  The row sums lie in LDS in float64, which leaves room for
+// 20 pixels a wave with three blocks a CU; 16, 18 or 19 (pitch 72) and 24 (two
+// blocks) are slower: distance driven, 128^3, 180 views of 192^2: 909, 881, 867,
+// 1056 us against 821; separable footprint, 120 x 132 x 101, 150 views of 187 x
+// 150: 1083, 1037, 1013, 1135 against 981.  (Sums in float32: 702 and 1099, with
+// an error against float64 1.6 and 1.09 times as large.)  What bounds it: vector
 // issue, most of it in the rows' slab sums and, with footprints, the weights.
 struct CtWaveLds {
-    float P[kCtPix * kCtPitch];
+    double P[kCtPix * kCtPitch];
     float w[kCtLines * kCtBins * kCtList];
 };
 
@@ -110,19 +143,18 @@ __device__ double ct_fp_one(const Geo& G, const M& V, const float* __restrict__ 
         for (int k = k0; k <= k1; ++k) {
             const float w = V.weight(k, io, ul, ur);
             if (!(w > 0.0f)) continue;
-            const float zm = V.zmag(k, io), r = 1.0f / ((M::kLineMag ? V.zmag(0, io) : zm) * G.d);
-            float ws[NS];
-            const int z0 = ct_cells<NS>(vl * r, vr * r, G.nz, ws);
+            const float h = V.zmag(M::kLineMag ? 0 : k, io) * G.d;
+            double ws[NS];
+            const int z0 = ct_slabs<NS>(vl, vr, h, 1.0f / h, G.nz, ws);
             const int ix = V.xd ? k : io, iy = V.xd ? io : k;
-            const float p = ct_sum<NS>(vol + ((int64_t)ix * G.ny + iy) * G.nz + z0, ws);
-            acc = __builtin_fma((double)(w * (zm * fu)), (double)p, acc);
+            acc = __builtin_fma((double)(w * fu), ct_sum_some<NS>(vol + ((int64_t)ix * G.ny + iy) * G.nz + z0, ws), acc);
         }
     }
     return acc;
 }
 
 template <class M, class Geo, int NS>
-__global__ __launch_bounds__(64 * kCtWaves) __attribute__((amdgpu_waves_per_eu(4))) void k_cone_fp_tile(Geo G, const float* __restrict__ ang,
+__global__ __launch_bounds__(64 * kCtWaves) __attribute__((amdgpu_waves_per_eu(3))) void k_cone_fp_tile(Geo G, const float* __restrict__ ang,
                                                                const float* __restrict__ cs,
                                                                const float* __restrict__ sn,
                                                                const float* __restrict__ vol,
@@ -138,6 +170,9 @@ __global__ __launch_bounds__(64 * kCtWaves) __attribute__((amdgpu_waves_per_eu(4
     // operand slots: group (matrix block) mid; weights: bin lo, pixel hi; sums:
     // pixel hi, row quad lo; results: bin hi, row quad lo
     const int lo = lane & 3, mid = (lane >> 2) & 3, hi = lane >> 4;
+    // place of row lane's sum: rows 16 c + 4 lo + e at 8 (2 c + e / 2) + 2 lo + e % 2,
+    // so that the four row quads of a 16-byte read lie side by side
+    const int slot = 8 * (2 * hi + (lo >> 1)) + 2 * mid + (lo & 1);
     int blk = (int)xcd_remap(blockIdx.x, gridDim.x);
     const int v_lo = (blk % nvt) * 64;
     blk /= nvt;
@@ -174,7 +209,7 @@ __global__ __launch_bounds__(64 * kCtWaves) __attribute__((amdgpu_waves_per_eu(4
                     continue;
                 }
                 if (!cnt) kf = k;
-                if (cnt < kCtList) L.w[lane * kCtList + cnt] = w * (V.zmag(k, io) * fu);
+                if (cnt < kCtList) L.w[lane * kCtList + cnt] = w * fu;
                 ++cnt;
             }
         }
@@ -205,37 +240,37 @@ __global__ __launch_bounds__(64 * kCtWaves) __attribute__((amdgpu_waves_per_eu(4
             // this operand slot's list
             const int e = 16 * l + (lane & 15);
             const int kfe = __shfl(kf, e), cne = __shfl(cnt, e), win = __shfl(gb, e) + hi;
-            float ws[NS];
+            double ws[NS];
             int z0 = 0;
             if (M::kLineMag) {
-                const float r = 1.0f / (V.zmag(0, io) * G.d);
-                z0 = ct_cells<NS>(vl * r, vr * r, G.nz, ws);
+                const float h = V.zmag(0, io) * G.d;
+                z0 = ct_slabs<NS>(vl, vr, h, 1.0f / h, G.nz, ws);
             }
             const int step = over ? kCtList : kCtPix;
             for (int kc = kb; kc <= ke; kc += step) {
                 const int nk = min(step, ke - kc + 1);
                 if (over && (lane >> 4) == l)
                     for (int k = max(kf, kc); k < min(kf + cnt, kc + nk); ++k)
-                        L.w[lane * kCtList + k - kc] = V.weight(k, io, ul, ur) * (V.zmag(k, io) * fu);
-                float rk = 0.0f;  // lane = pixel
-                if (!M::kLineMag) rk = 1.0f / (V.zmag(min(kc + lane, V.nd - 1), io) * G.d);
+                        L.w[lane * kCtList + k - kc] = V.weight(k, io, ul, ur) * fu;
+                float hk = 0.0f, rk = 0.0f;  // lane = pixel
+                if (!M::kLineMag) {
+                    hk = V.zmag(min(kc + lane, V.nd - 1), io) * G.d;
+                    rk = 1.0f / hk;
+                }
                 const float* col = vol + (int64_t)io * lstride + (int64_t)kc * kstride;
                 auto stage = [&](int kk, const float* p) {
-                    if (!M::kLineMag) {
-                        const float r = ct_lane(rk, kk);
-                        z0 = ct_cells<NS>(vl * r, vr * r, G.nz, ws);
-                    }
+                    if (!M::kLineMag) z0 = ct_slabs<NS>(vl, vr, ct_lane(hk, kk), ct_lane(rk, kk), G.nz, ws);
                     return ct_sum<NS>(p + z0, ws);
                 };
                 int kk = 0;
                 for (; kk + 3 < nk; kk += 4, col += 4 * kstride) {
-                    float p[4];
+                    double p[4];
 #pragma unroll
                     for (int t = 0; t < 4; ++t) p[t] = stage(kk + t, col + t * kstride);
 #pragma unroll
-                    for (int t = 0; t < 4; ++t) L.P[(kk + t) * kCtPitch + lane] = p[t];
+                    for (int t = 0; t < 4; ++t) L.P[(kk + t) * kCtPitch + slot] = p[t];
                 }
-                for (; kk < nk; ++kk, col += kstride) L.P[kk * kCtPitch + lane] = stage(kk, col);
+                for (; kk < nk; ++kk, col += kstride) L.P[kk * kCtPitch + slot] = stage(kk, col);
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 const int k0 = over ? kc + hi : win, ns = over ? (nk + 3) >> 2 : nks, wb = over ? kc : kfe;
                 for (int t = 0; t < ns; ++t) {
@@ -243,16 +278,14 @@ __global__ __launch_bounds__(64 * kCtWaves) __attribute__((amdgpu_waves_per_eu(4
                     const bool in = (unsigned)(k - kfe) < (unsigned)cne && (unsigned)kr < (unsigned)nk;
                     if (!__any(in)) continue;  // another chunk's pixels
                     const double w = in ? (double)L.w[e * kCtList + (k - wb)] : 0.0;
-                    const float4* row = (const float4*)(L.P + min(max(kr, 0), nk - 1) * kCtPitch + 4 * lo);
-                    float4 x[4];
+                    const double2* row = (const double2*)(L.P + min(max(kr, 0), nk - 1) * kCtPitch + 2 * lo);
+                    double2 x[8];
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) x[c] = row[4 * c];
+                    for (int c = 0; c < 8; ++c) x[c] = row[4 * c];
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        acc[4 * c] = __builtin_amdgcn_mfma_f64_4x4x4f64(w, (double)x[c].x, acc[4 * c], 0, 0, 0);
-                        acc[4 * c + 1] = __builtin_amdgcn_mfma_f64_4x4x4f64(w, (double)x[c].y, acc[4 * c + 1], 0, 0, 0);
-                        acc[4 * c + 2] = __builtin_amdgcn_mfma_f64_4x4x4f64(w, (double)x[c].z, acc[4 * c + 2], 0, 0, 0);
-                        acc[4 * c + 3] = __builtin_amdgcn_mfma_f64_4x4x4f64(w, (double)x[c].w, acc[4 * c + 3], 0, 0, 0);
+                    for (int c = 0; c < 8; ++c) {
+                        acc[2 * c] = __builtin_amdgcn_mfma_f64_4x4x4f64(w, x[c].x, acc[2 * c], 0, 0, 0);
+                        acc[2 * c + 1] = __builtin_amdgcn_mfma_f64_4x4x4f64(w, x[c].y, acc[2 * c + 1], 0, 0, 0);
                     }
                 }
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -286,6 +319,45 @@ __global__ __launch_bounds__(64 * kCtWaves) __attribute__((amdgpu_waves_per_eu(4
 // = view lists the bins that the column's pixel meets; the view loop then
 // reads the list by readlane and each lane sums the NS rows its slab meets
 // of every bin.
+//
+// Zero weights times infinite values make NaNs: a sum that is not finite is
+// formed again without them.
+
+// Bins [j0, j1] that pixel k of line io can meet in view V.
+template <class M, class Geo>
+__device__ __forceinline__ void ct_bins(const Geo& G, const M& V, int k, int io, int& j0, int& j1) {
+    const float inv_du = 1.0f / G.du, u0 = G.du * (-0.5f * (float)G.nu + G.su);
+    const float mar = 0.01f + 1e-6f * (float)G.nu;  // rounding of the bin positions
+    float lo, hi;
+    V.foot(k, io, lo, hi);
+    j0 = (int)fmaxf(floorf((lo - u0) * inv_du - mar), 0.0f);
+    j1 = (int)fminf(floorf((hi - u0) * inv_du + mar), (float)(G.nu - 1));
+}
+
+// One voxel, bin by bin.
+template <class M, class Geo, int NS>
+__device__ double ct_bp_one(const Geo& G, const float* __restrict__ ang, const float* __restrict__ cs,
+                            const float* __restrict__ sn, const float* __restrict__ sino, int ix, int iy, int iz) {
+    const auto edge = [&](int j) { return G.du * (((float)j - 0.5f * (float)G.nu) + G.su); };
+    const float zl = G.d * ((float)iz - 0.5f * (float)G.nz), zr = G.d * ((float)(iz + 1) - 0.5f * (float)G.nz);
+    double acc = 0.0;
+    for (int ia = 0; ia < G.na; ++ia) {
+        const M V(G, cs[ia], sn[ia], ang ? ang[ia] : 0.0f);
+        const int k = V.xd ? ix : iy, io = V.xd ? iy : ix;
+        int j0, j1;
+        ct_bins(G, V, k, io, j0, j1);
+        const float m = V.zmag(k, io) / G.dv;
+        double ws[NS];
+        const int m0 = ct_cells<NS>(__builtin_fmaf(zl, m, -G.sv), __builtin_fmaf(zr, m, -G.sv), G.nv, ws);
+        for (int j = j0; j <= j1; ++j) {
+            const float w = V.weight(k, io, edge(j), edge(j + 1));
+            if (w > 0.0f)
+                acc = __builtin_fma((double)w, ct_sum_some<NS>(sino + ((int64_t)ia * G.nu + j) * G.nv + m0, ws), acc);
+        }
+    }
+    return acc;
+}
+
 template <class M, class Geo, int NS>
 __global__ __launch_bounds__(256) void k_cone_bp_col(Geo G, const float* __restrict__ ang,
                                                     const float* __restrict__ cs, const float* __restrict__ sn,
@@ -301,8 +373,6 @@ __global__ __launch_bounds__(256) void k_cone_bp_col(Geo G, const float* __restr
     const int ix = (int)(r % G.nx);
     vol += (r / G.nx) * G.nx * G.ny * G.nz;
     sino += (r / G.nx) * (int64_t)G.na * G.nu * G.nv;
-    const float inv_du = 1.0f / G.du, inv_dv = 1.0f / G.dv;
-    const float u0 = G.du * (-0.5f * (float)G.nu + G.su);
     const float zl = G.d * ((float)iz - 0.5f * (float)G.nz), zr = G.d * ((float)(iz + 1) - 0.5f * (float)G.nz);
     double acc = 0.0;
     for (int va = 0; va < G.na; va += 64) {
@@ -313,12 +383,10 @@ __global__ __launch_bounds__(256) void k_cone_bp_col(Geo G, const float* __restr
         const int ial = min(va + lane, G.na - 1);
         const M V(G, cs[ial], sn[ial], ang ? ang[ial] : 0.0f);
         const int k = V.xd ? ix : iy, io = V.xd ? iy : ix;
-        float lo, hi;
-        V.foot(k, io, lo, hi);
-        const float mar = 0.01f + 1e-6f * (float)G.nu;  // rounding of the bin positions
-        const int j1 = (int)fminf(floorf((hi - u0) * inv_du + mar), (float)(G.nu - 1));
+        int j0, j1;
+        ct_bins(G, V, k, io, j0, j1);
         const auto edge = [&](int j) { return G.du * (((float)j - 0.5f * (float)G.nu) + G.su); };
-        for (int j = (int)fmaxf(floorf((lo - u0) * inv_du - mar), 0.0f); j <= j1; ++j) {
+        for (int j = j0; j <= j1; ++j) {
             const float x = V.weight(k, io, edge(j), edge(j + 1));
             if (!(x > 0.0f)) {
                 if (cnt) break;
@@ -329,7 +397,7 @@ __global__ __launch_bounds__(256) void k_cone_bp_col(Geo G, const float* __restr
             for (int t = 0; t < kCtFoot; ++t) w[t] = t == cnt ? x : w[t];
             ++cnt;
         }
-        zs = V.zmag(k, io) * inv_dv;
+        zs = V.zmag(k, io) / G.dv;
         const bool over = __any(cnt > kCtFoot);  // bins much finer than pixels
         const int nvw = min(64, G.na - va);
         for (int v = 0; v < nvw; ++v) {
@@ -337,7 +405,7 @@ __global__ __launch_bounds__(256) void k_cone_bp_col(Geo G, const float* __restr
             if (n == 0) continue;
             const int j = __builtin_amdgcn_readlane(jf, v);
             const float m = ct_lane(zs, v);
-            float ws[NS];
+            double ws[NS];
             const int m0 = ct_cells<NS>(__builtin_fmaf(zl, m, -G.sv), __builtin_fmaf(zr, m, -G.sv), G.nv, ws);
             const float* row = sino + ((int64_t)(va + v) * G.nu + j) * G.nv + m0;
             if (over) {
@@ -345,36 +413,38 @@ __global__ __launch_bounds__(256) void k_cone_bp_col(Geo G, const float* __restr
                 const int kv = W.xd ? ix : iy, iov = W.xd ? iy : ix;
                 for (int t = 0; t < n; ++t)
                     acc = __builtin_fma((double)W.weight(kv, iov, edge(j + t), edge(j + t + 1)),
-                                        (double)ct_sum<NS>(row + (int64_t)t * G.nv, ws), acc);
+                                        ct_sum<NS>(row + (int64_t)t * G.nv, ws), acc);
                 continue;
             }
             if (n >= 2) {
-                const float s0 = ct_sum<NS>(row, ws), s1 = ct_sum<NS>(row + G.nv, ws);
-                acc = __builtin_fma((double)ct_lane(w[0], v), (double)s0, acc);
-                acc = __builtin_fma((double)ct_lane(w[1], v), (double)s1, acc);
+                const double s0 = ct_sum<NS>(row, ws), s1 = ct_sum<NS>(row + G.nv, ws);
+                acc = __builtin_fma((double)ct_lane(w[0], v), s0, acc);
+                acc = __builtin_fma((double)ct_lane(w[1], v), s1, acc);
             } else {
-                acc = __builtin_fma((double)ct_lane(w[0], v), (double)ct_sum<NS>(row, ws), acc);
+                acc = __builtin_fma((double)ct_lane(w[0], v), ct_sum<NS>(row, ws), acc);
             }
 #pragma unroll
             for (int t = 2; t < kCtFoot; ++t) {
                 if (t >= n) break;
-                acc = __builtin_fma((double)ct_lane(w[t], v), (double)ct_sum<NS>(row + (int64_t)t * G.nv, ws), acc);
+                acc = __builtin_fma((double)ct_lane(w[t], v), ct_sum<NS>(row + (int64_t)t * G.nv, ws), acc);
             }
         }
     }
     if (iz >= G.nz) return;
+    if (!(fabs(acc) < (double)VIR_INF)) acc = ct_bp_one<M, Geo, NS>(G, ang, cs, sn, sino, ix, iy, iz);
     const int64_t o = ((int64_t)ix * G.ny + iy) * G.nz + iz;
-    float res = (float)acc * (G.out_scale * M::bp_unit(G));
+    float res = (float)(acc * (double)M::bp_unit(G)) * G.out_scale;
     if (accumulate) res += vol[o];
     vol[o] = res;
 }
 
 // Cells a v (z) interval of at most `len` cells can meet, as the NS of the
 // kernels above, or 0 where they do not apply (intervals longer than 2.9
-// cells, or fewer than NS cells in all).
+// cells, fewer than NS cells in all, or so many that ct_first's margin would
+// not fit).
 inline int ct_slots(double len, int n) {
     const int ns = len <= 0.99 ? 2 : len <= 1.99 ? 3 : len <= 2.9 ? 4 : 0;
-    return n >= ns ? ns : 0;
+    return n >= ns && n <= 20000 ? ns : 0;
 }
 
 template <class M, class Geo>

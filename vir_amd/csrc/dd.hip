@@ -316,7 +316,7 @@ struct DDCone {
         return (fminf(hi, ur) - fmaxf(lo, ul)) * dd_scale<DD_FAN_FLAT>(G, V, cell_cen(no, G.d, io));
     }
     __device__ float zmag(int, int io) const { return cone_zmag(G, V, cell_cen(no, G.d, io)); }
-    __host__ __device__ static float fp_unit(const DDGeo& g) { return g.d; }
+    __host__ __device__ static float fp_unit(const DDGeo&) { return 1.0f; }
     __host__ __device__ static float bp_unit(const DDGeo& g) { return g.dv; }
 };
 

@@ -127,9 +127,10 @@ __device__ __forceinline__ SFFoot sf_foot(const SFGeo& G, const SFView& V, int i
     float u0 = fm * (pxl + pyl), u1 = fm * (pxr + pyl), u2 = fm * (pxl + pyr), u3 = fm * (pxr + pyr);
     f.u0 = fminf(fminf(u0, u1), fminf(u2, u3));
     f.u1 = fmaxf(fmaxf(u0, u1), fmaxf(u2, u3));
-    // 1/cos of the fan angle atan(t), t = uc/DSD
-    const float t = (pxc + pyc) / den_c;
-    f.cm = fm * __builtin_sqrtf(1.0f + t * t);
+    // over the cosine of the fan angle atan(t): sqrt(1 + t^2) as 1 + t^2 / (1 +
+    // sqrt(1 + t^2)), whose small term's rounding hardly counts
+    const float t = (pxc + pyc) / den_c, t2 = t * t;
+    f.cm = __builtin_fmaf(fm, t2 * __builtin_amdgcn_rcpf(1.0f + __builtin_sqrtf(1.0f + t2)), fm);
     return f;
 }
 
@@ -331,7 +332,7 @@ struct SFCone {
         return ((fminf(f.u1, ur) - fmaxf(f.u0, ul)) * (1.0f / G.du)) * f.amp;
     }
     __device__ float zmag(int k, int io) const { return at(k, io).cm; }
-    __host__ __device__ static float fp_unit(const SFGeo& g) { return g.d * (1.0f / g.dv); }
+    __host__ __device__ static float fp_unit(const SFGeo& g) { return 1.0f / g.dv; }
     __host__ __device__ static float bp_unit(const SFGeo&) { return 1.0f; }
 };
 
