@@ -42,11 +42,32 @@ __device__ __forceinline__ float ft_lane(float x, int l) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
 }
 
+// Sum of all chains, of which wave w of NW has added its own (w, w + NW, ..) up:
+// in the order of four waves.
+template <int NW, class Part>
+__device__ __forceinline__ double ft_chains(Part&& part) {
+    double s = 0.0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        double t = part(w);
+#pragma unroll
+        for (int c = w + 4; c < NW; c += 4) t += part(c);
+        s = w == 0 ? t : s + t;
+    }
+    return s;
+}
+
 constexpr int kFtBins = 128;   // bins of a forward tile, two a lane
 constexpr int kFtStage = 128;  // interval slots of a line staged at once
 constexpr int kFtPad = 6;      // of which empty ones past the last pixel, read but of no overlap
 
 // ---------------------------------------------------------------- forward
+//
+// A bin's lines are summed in kFtLines chains (line modulo kFtLines) and the
+// chains in one order, whatever the number of waves, so that an item's bits do
+// not depend on the batch it is in (at most 2 % of the time).
+constexpr int kFtLines = 8;
+
 template <bool SHARED>
 struct FtWaveLds {  // an edge and a value per pixel
     float e[2][kFtStage + 2];
@@ -111,7 +132,7 @@ __global__ __launch_bounds__(64 * NW) void k_fp2d_tile(Geo G, const float* __res
         I[q] = invert(ul[q], ur[q]);
     }
     const Inv T = invert(edge(u_lo), edge(min(u_lo + kFtBins, G.nu)));
-    double acc[2] = {0.0, 0.0};
+    double acc[2], sum[2] = {0.0, 0.0};
     // this bin's pixels of line slot h, pixels kc .. kc + nk - 1 staged
     const auto merge = [&](int h, float oc, float lf, int kc, int nk) {
 #pragma unroll
@@ -144,111 +165,115 @@ __global__ __launch_bounds__(64 * NW) void k_fp2d_tile(Geo G, const float* __res
         }
     };
     const int stride = V.xd ? G.ny : 1, lstride = V.xd ? 1 : G.ny;
-    for (int g = 0; g < no; g += 64 * NW) {
-        // lane = line g + NW lane + wave: its coordinate, pixel band and factor
-        const int iol = g + NW * lane + wave;
-        const float ocl = V.centre(min(iol, no - 1));
-        const float lfl = V.line_factor(ocl);
-        float a, b;
-        range(T, ocl, a, b);
-        const int kbl = (int)fmaxf(a - 1.0f, 0.0f);
-        const int kel = iol < no ? (int)fminf(b + 1.0f, (float)(nd - 1)) : -1;
-        const int nl = min(64, (no - g - wave + NW - 1) / NW);
-        for (int l = 0; l < nl; l += 2) {
-            int kb[2], ke[2];
-            float oc[2], lf[2];
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int t = min(l + h, 63);
-                kb[h] = __builtin_amdgcn_readlane(kbl, t);
-                ke[h] = l + h < nl ? __builtin_amdgcn_readlane(kel, t) : -1;
-                oc[h] = ft_lane(ocl, t);
-                lf[h] = ft_lane(lfl, t);
-            }
-            const int most = max(ke[0] - kb[0], ke[1] - kb[1]);
-            for (int c = 0; c <= most; c += kFtStage - kFtPad) {
-                int kc[2], nk[2];
-                float x[2][2];
+    constexpr int STEP = kFtLines / NW;  // chains of a wave: wave, wave + NW, ..
+    for (int ch = 0; ch < STEP; ++ch) {
+        acc[0] = acc[1] = 0.0;
+        for (int g = 0; g < no; g += 64 * NW) {
+            // lane = line g + NW lane + wave: its coordinate, pixel band and factor
+            const int iol = g + NW * lane + wave;
+            const float ocl = V.centre(min(iol, no - 1));
+            const float lfl = V.line_factor(ocl);
+            float a, b;
+            range(T, ocl, a, b);
+            const int kbl = (int)fmaxf(a - 1.0f, 0.0f);
+            const int kel = iol < no ? (int)fminf(b + 1.0f, (float)(nd - 1)) : -1;
+            const int nl = min(64, (no - g - wave + NW - 1) / NW);
+            for (int l = ch; l < nl; l += 2 * STEP) {
+                int kb[2], ke[2];
+                float oc[2], lf[2];
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
-                    kc[h] = kb[h] + c;
-                    nk[h] = min(kFtStage - kFtPad, ke[h] - kc[h] + 1);
-                    const int io = g + NW * (l + h) + wave;
-#pragma unroll
-                    for (int t = 0; t < 2; ++t) {
-                        const int k = 64 * t + lane;
-                        x[h][t] = 0.0f;
-                        if (k < nk[h]) x[h][t] = img[(int64_t)(kc[h] + k) * stride + (int64_t)io * lstride];
-                    }
+                    const int t = min(l + STEP * h, 63);
+                    kb[h] = __builtin_amdgcn_readlane(kbl, t);
+                    ke[h] = l + STEP * h < nl ? __builtin_amdgcn_readlane(kel, t) : -1;
+                    oc[h] = ft_lane(ocl, t);
+                    lf[h] = ft_lane(lfl, t);
                 }
+                const int most = max(ke[0] - kb[0], ke[1] - kb[1]);
+                for (int c = 0; c <= most; c += kFtStage - kFtPad) {
+                    int kc[2], nk[2];
+                    float x[2][2];
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const int io = g + NW * (l + h) + wave;
-#pragma unroll
-                    for (int t = 0; t < 2; ++t) {
-                        const int k = 64 * t + lane;
-                        if (64 * t >= nk[h] + kFtPad) continue;  // whole wave
-                        // slots past the last pixel are empty: both ends at
-                        // one place
-                        if constexpr (M::kShared) {
-                            L.e[h][k] = V.edge(min(kc[h] + k, kc[h] + nk[h]), oc[h]);
-                            L.v[h][k] = x[h][t];
-                        } else if constexpr (!M::kCorners) {
-                            float u0, u1;
-                            const float f = V.pixel(min(kc[h] + k, nd - 1), min(io, no - 1), u0, u1);
-                            L.p[h][k] = make_float4(u0, k < nk[h] ? u1 : u0, x[h][t], f);
-                        }
-                    }
-                    if constexpr (M::kCorners) {
-                        // the corners at pixel k's lower end, the line's two
-                        // edges; the next lane's are those at its upper end
-                        // (four divisions a pixel for six: 0.41 -> 0.39 ms)
-                        const int il = min(io, no - 1);
-                        if (nk[h] + kFtPad <= 0) continue;     // whole wave
-                        const bool two = nk[h] + kFtPad > 64;  // whole wave
-                        float lo[2], hi[2];
+                    for (int h = 0; h < 2; ++h) {
+                        kc[h] = kb[h] + c;
+                        nk[h] = min(kFtStage - kFtPad, ke[h] - kc[h] + 1);
+                        const int io = g + NW * (l + STEP * h) + wave;
 #pragma unroll
                         for (int t = 0; t < 2; ++t) {
-                            lo[t] = hi[t] = 0.0f;
-                            if (t && !two) continue;
-                            const float c0 = V.grid(min(kc[h] + 64 * t + lane, nd), il);
-                            const float c1 = V.grid(min(kc[h] + 64 * t + lane, nd), il + 1);
-                            lo[t] = fminf(c0, c1);
-                            hi[t] = fmaxf(c0, c1);
-                        }
-#pragma unroll
-                        for (int t = 0; t < 2; ++t) {
-                            if (t && !two) continue;
                             const int k = 64 * t + lane;
-                            float ln = __shfl_down(lo[t], 1), hn = __shfl_down(hi[t], 1);
-                            if (t == 0) {  // (slots 63, if there is no second half, and 127 are empty)
-                                ln = lane == 63 ? ft_lane(lo[1], 0) : ln;
-                                hn = lane == 63 ? ft_lane(hi[1], 0) : hn;
-                            }
-                            const float u0 = fminf(lo[t], ln), u1 = fmaxf(hi[t], hn);
-                            L.p[h][k] = make_float4(u0, k < nk[h] ? u1 : u0, x[h][t],
-                                                    V.amp(min(kc[h] + k, nd - 1), il));
+                            x[h][t] = 0.0f;
+                            if (k < nk[h]) x[h][t] = img[(int64_t)(kc[h] + k) * stride + (int64_t)io * lstride];
                         }
                     }
-                }
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // a wave's LDS accesses are in order
 #pragma unroll
-                for (int h = 0; h < 2; ++h)
-                    if (nk[h] > 0) merge(h, oc[h], lf[h], kc[h], nk[h]);
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    for (int h = 0; h < 2; ++h) {
+                        const int io = g + NW * (l + STEP * h) + wave;
+#pragma unroll
+                        for (int t = 0; t < 2; ++t) {
+                            const int k = 64 * t + lane;
+                            if (64 * t >= nk[h] + kFtPad) continue;  // whole wave
+                            // slots past the last pixel are empty: both ends at
+                            // one place
+                            if constexpr (M::kShared) {
+                                L.e[h][k] = V.edge(min(kc[h] + k, kc[h] + nk[h]), oc[h]);
+                                L.v[h][k] = x[h][t];
+                            } else if constexpr (!M::kCorners) {
+                                float u0, u1;
+                                const float f = V.pixel(min(kc[h] + k, nd - 1), min(io, no - 1), u0, u1);
+                                L.p[h][k] = make_float4(u0, k < nk[h] ? u1 : u0, x[h][t], f);
+                            }
+                        }
+                        if constexpr (M::kCorners) {
+                            // the corners at pixel k's lower end, the line's two
+                            // edges; the next lane's are those at its upper end
+                            // (four divisions a pixel for six: 0.41 -> 0.39 ms)
+                            const int il = min(io, no - 1);
+                            if (nk[h] + kFtPad <= 0) continue;     // whole wave
+                            const bool two = nk[h] + kFtPad > 64;  // whole wave
+                            float lo[2], hi[2];
+#pragma unroll
+                            for (int t = 0; t < 2; ++t) {
+                                lo[t] = hi[t] = 0.0f;
+                                if (t && !two) continue;
+                                const float c0 = V.grid(min(kc[h] + 64 * t + lane, nd), il);
+                                const float c1 = V.grid(min(kc[h] + 64 * t + lane, nd), il + 1);
+                                lo[t] = fminf(c0, c1);
+                                hi[t] = fmaxf(c0, c1);
+                            }
+#pragma unroll
+                            for (int t = 0; t < 2; ++t) {
+                                if (t && !two) continue;
+                                const int k = 64 * t + lane;
+                                float ln = __shfl_down(lo[t], 1), hn = __shfl_down(hi[t], 1);
+                                if (t == 0) {  // (slots 63, if there is no second half, and 127 are empty)
+                                    ln = lane == 63 ? ft_lane(lo[1], 0) : ln;
+                                    hn = lane == 63 ? ft_lane(hi[1], 0) : hn;
+                                }
+                                const float u0 = fminf(lo[t], ln), u1 = fmaxf(hi[t], hn);
+                                L.p[h][k] = make_float4(u0, k < nk[h] ? u1 : u0, x[h][t],
+                                                        V.amp(min(kc[h] + k, nd - 1), il));
+                            }
+                        }
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // a wave's LDS accesses are in order
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+                        if (nk[h] > 0) merge(h, oc[h], lf[h], kc[h], nk[h]);
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                }
             }
         }
+        sum[0] += acc[0];
+        sum[1] += acc[1];
     }
     __syncthreads();
-    lds.red[wave][lane] = acc[0];
-    lds.red[wave][64 + lane] = acc[1];
+    lds.red[wave][lane] = sum[0];
+    lds.red[wave][64 + lane] = sum[1];
     __syncthreads();
     for (int i = threadIdx.x; i < kFtBins; i += 64 * NW) {
         const int iu = u_lo + i;
         if (iu >= G.nu) continue;
-        double s = lds.red[0][i];
-#pragma unroll
-        for (int w = 1; w < NW; ++w) s += lds.red[w][i];
+        const double s = ft_chains<NW>([&](int w) { return lds.red[w][i]; });
         const int64_t o = row * G.nu + iu;
         float r = (float)s * G.out_scale;
         if (accumulate) r += sino[o];
@@ -259,7 +284,9 @@ __global__ __launch_bounds__(64 * NW) void k_fp2d_tile(Geo G, const float* __res
 // --------------------------------------------------------------- backward
 //
 // A block takes 16 x 16 pixels, a 2 x 2 block a lane; wave w of its NW takes
-// views w, w + NW, ...
+// views w, w + NW, ..., in chains (view modulo kFtViews) as the forward's lines.
+constexpr int kFtViews = 16;
+
 template <class M, class Geo, int NW>
 __global__ __launch_bounds__(64 * NW) void k_bp2d_tile(Geo G, const float* __restrict__ ang,
                                                       const float* __restrict__ cs, const float* __restrict__ sn,
@@ -277,48 +304,55 @@ __global__ __launch_bounds__(64 * NW) void k_bp2d_tile(Geo G, const float* __res
     // u in bins from the first one's edge, and its rounding
     const float off = half - G.su, mar = 1e-4f + 1e-6f * ((float)G.nu + fabsf(G.su));
     const float uend = G.du * (half + G.su);
-    double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int g = 0; g < G.na; g += 64 * NW) {
-        const int il = min(g + NW * lane + wave, G.na - 1);
-        const typename M::Trig tl(cs[il], sn[il], ang ? ang[il] : 0.0f);  // lane = view
-        const int nl = min(64, (G.na - g - wave + NW - 1) / NW);
-        for (int l = 0; l < nl; ++l) {
-            const M V(G, tl.lane(l));
-            const float* __restrict__ row = sino + (int64_t)(g + NW * l + wave) * G.nu;
-            float lo[4], hi[4], f[4];
-            V.quad(ix, iy, lo, hi, f);
-            int j0[4], n[4];
-            float y[4][3];
+    double acc[4], sum[4] = {0.0, 0.0, 0.0, 0.0};
+    constexpr int STEP = kFtViews / NW;  // chains of a wave: wave, wave + NW, ..
+    for (int ch = 0; ch < STEP; ++ch) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                hi[q] = fminf(hi[q], uend);
-                const float j = fminf(fmaxf(floorf(__builtin_fmaf(lo[q], inv_du, off) - mar), 0.0f), (float)(G.nu - 1));
-                j0[q] = (int)j;
-                n[q] = (int)fminf(__builtin_fmaf(hi[q], inv_du, off) + mar, (float)(G.nu - 1)) - j0[q];  // bins past the first
+        for (int q = 0; q < 4; ++q) acc[q] = 0.0;
+        for (int g = 0; g < G.na; g += 64 * NW) {
+            const int il = min(g + NW * lane + wave, G.na - 1);
+            const typename M::Trig tl(cs[il], sn[il], ang ? ang[il] : 0.0f);  // lane = view
+            const int nl = min(64, (G.na - g - wave + NW - 1) / NW);
+            for (int l = ch; l < nl; l += STEP) {
+                const M V(G, tl.lane(l));
+                const float* __restrict__ row = sino + (int64_t)(g + NW * l + wave) * G.nu;
+                float lo[4], hi[4], f[4];
+                V.quad(ix, iy, lo, hi, f);
+                int j0[4], n[4];
+                float y[4][3];
 #pragma unroll
-                for (int t = 0; t < 3; ++t) y[q][t] = row[min(j0[q] + t, G.nu - 1)];
-            }
+                for (int q = 0; q < 4; ++q) {
+                    hi[q] = fminf(hi[q], uend);
+                    const float j = fminf(fmaxf(floorf(__builtin_fmaf(lo[q], inv_du, off) - mar), 0.0f), (float)(G.nu - 1));
+                    j0[q] = (int)j;
+                    n[q] = (int)fminf(__builtin_fmaf(hi[q], inv_du, off) + mar, (float)(G.nu - 1)) - j0[q];  // bins past the first
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                double s = 0.0;
-                // neighbouring bins share the rounded edge between them, so a
-                // pixel's overlaps add up to its interval
-                float k = ((float)j0[q] - half) + G.su, e = G.du * k;
-                const auto term = [&](float v) {
-                    k += 1.0f;
-                    const float e1 = G.du * k, ov = fminf(hi[q], e1) - fmaxf(lo[q], e);
-                    s += (double)(ov > 0.0f ? v * ov : 0.0f);
-                    e = e1;
-                };
+                    for (int t = 0; t < 3; ++t) y[q][t] = row[min(j0[q] + t, G.nu - 1)];
+                }
 #pragma unroll
-                for (int t = 0; t < 3; ++t) term(y[q][t]);
-                for (int t = 3; t <= n[q]; ++t) term(row[j0[q] + t]);
-                acc[q] = __builtin_fma(s, (double)f[q], acc[q]);
+                for (int q = 0; q < 4; ++q) {
+                    double s = 0.0;
+                    // neighbouring bins share the rounded edge between them, so a
+                    // pixel's overlaps add up to its interval
+                    float k = ((float)j0[q] - half) + G.su, e = G.du * k;
+                    const auto term = [&](float v) {
+                        k += 1.0f;
+                        const float e1 = G.du * k, ov = fminf(hi[q], e1) - fmaxf(lo[q], e);
+                        s += (double)(ov > 0.0f ? v * ov : 0.0f);
+                        e = e1;
+                    };
+#pragma unroll
+                    for (int t = 0; t < 3; ++t) term(y[q][t]);
+                    for (int t = 3; t <= n[q]; ++t) term(row[j0[q] + t]);
+                    acc[q] = __builtin_fma(s, (double)f[q], acc[q]);
+                }
             }
         }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) sum[q] += acc[q];
     }
 #pragma unroll
-    for (int q = 0; q < 4; ++q) red[wave][64 * q + lane] = acc[q];
+    for (int q = 0; q < 4; ++q) red[wave][64 * q + lane] = sum[q];
     __syncthreads();
     const double unit = (double)M::bp_unit(G);
     for (int i = threadIdx.x; i < 256; i += 64 * NW) {
@@ -326,9 +360,7 @@ __global__ __launch_bounds__(64 * NW) void k_bp2d_tile(Geo G, const float* __res
         const int x = i >> 4, y = i & 15;
         const int slot = 64 * (2 * (x & 1) + (y & 1)) + 8 * (x >> 1) + (y >> 1);
         if (bx + x >= G.nx || by + y >= G.ny) continue;
-        double s = red[0][slot];
-#pragma unroll
-        for (int w = 1; w < NW; ++w) s += red[w][slot];
+        const double s = ft_chains<NW>([&](int w) { return red[w][slot]; });
         const int64_t o = (item * G.nx + bx + x) * G.ny + by + y;
         float r = (float)(s * unit) * G.out_scale;
         if (accumulate) r += img[o];

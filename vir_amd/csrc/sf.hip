@@ -1082,12 +1082,19 @@ static int sf_par3_bp_ksteps(const SFGeo& G, int& shift) {
     return ks <= 4 && G.nu >= 4 * ks ? ks : 0;
 }
 
+// Items of fewer pixel blocks split each one's views over four waves.  Split |
+// one wave a block, us: 256 x 256 x 64 (4096 blocks), 180 views, one item 277 | 294,
+// eight 2102 | 2038, 45 views 78 | 77, 583 | 527; 128 x 128 x 64 (1024 blocks), 180
+// views, 32 items 2135 | 2056, one 76 | (too few waves).
+constexpr int64_t kParSplit = 4096;
+
 template <int KS>
 static int sf_par3_bp_mfma(const SFGeo& G, const float* cosv, const float* sinv, const float* sino, float* img, int acc,
                            int shift, hipStream_t st) {
     const int nbx = (G.nx + 3) / 4, nby = (G.ny + 3) / 4, nzt = (G.nz + 63) / 64;
     const int64_t n = (int64_t)G.nb * nbx * nby * nzt;
-    if (n < 8192)
+    // by one item's blocks, so that an item's bits don't depend on the batch
+    if ((int64_t)nbx * nby * nzt < kParSplit)
         hipLaunchKernelGGL((k_sf_bp_par3_mfma<KS, true>), dim3((unsigned)n), dim3(256), 0, st, G, cosv, sinv, sino, img,
                            acc, nby, nbx, nzt, shift, n);
     else
