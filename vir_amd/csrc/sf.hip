@@ -1113,12 +1113,24 @@ static bool sf_par3_bp_col_ok(const SFGeo& G) {
 
 // True when the tiled parallel 3-D forward kernel takes the call: detector rows
 // no taller than a voxel (each row meets at most kSlabs slabs), and where it is
-// faster than the gather.  256 x 256, 1.5 x 256 bins, tile | gather in us:
-// 8 items, 180 views, 64 rows, du = d: 2930 | 28500, 2 d: 2980 | 17600, 2.8 d:
-// 3990 | 16400; 1 item, 64 views: 500 | 1635, 1140 | 1230, 1510 | 1170 (wide bins
-// have long pixel windows).  8 items with 4 rows 2910 | 2225, with 8: 2910 |
-// 3910; 1 item, 64 views, 4 rows 500 | 480.
-static bool sf_par3_tiled_ok(const SFGeo& G) { return G.dv <= G.d && G.du <= 2.5f * G.d && G.nv >= 6; }
+// faster than the gather, judged by one item so that an item's bits don't depend
+// on the batch.  256 x 256, 1.5 x 256 bins, tile | gather in us, 8 items, 180
+// views, 64 rows: du = d 2930 | 28500, 2 d 2980 | 17600; 1 item, 64 views: 500 |
+// 1635, 1140 | 1230.  8 items with 4 rows 2910 | 2225, with 8: 2910 | 3910; 1 item,
+// 64 views, 4 rows 500 | 480.
+// Bins wider than 2.5 pixels have long pixel windows, and a block takes its 1.5
+// ms at 256^2 however few there are.  An item needs blocks (counted by the rows
+// in use) to make up for it: below 2.75 pixels as many as let a batch fill
+// the chip, from 2.75 on as many as win alone.  2.6 | 2.8 | 3.2 | 4 pixels, gather
+// over tile, 64 rows: 405 blocks, one item 1.58 | 1.61 | 1.34 | 0.82, eight 4.4 | 4.0 |
+// 3.5 | 2.9; 144: 0.89 | 0.78 | 0.74 | 0.55, 2.9 | 2.6 | 2.2 | 1.8; 48: 0.66 | 0.65 | 0.69 |
+// 0.52, 1.8 | 1.5 | 1.6 | 1.1; 20: 0.51 | 0.52 | 0.51 | 0.40, 1.0 | 1.0 | 0.9 | 0.7.
+static bool sf_par3_tiled_ok(const SFGeo& G) {
+    if (!(G.dv <= G.d) || G.nv < 6) return false;
+    if (G.du <= 2.5f * G.d) return true;
+    const double full = (double)((G.na + kVG - 1) / kVG) * ((G.nu + kTUB - 1) / kTUB) * G.nv / kTV;
+    return G.du <= 2.75f * G.d ? full >= 48.0 : G.du <= 3.2f * G.d && full >= 400.0;
+}
 
 // An item with at most this many blocks (two a CU) takes two wave groups a
 // block: they wait for their own chain of operands, not for the matrix cores.
