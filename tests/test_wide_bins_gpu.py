@@ -17,6 +17,7 @@ CASES = [
     dict(shape=(60, 70, 40), nu=36, nv=50, na=150, du=2.76, sv=0.3),
     dict(shape=(130, 121, 64), nu=60, nv=64, na=397, du=3.2),                    # 400 blocks
     dict(shape=(130, 121, 60), nu=60, nv=60, na=397, du=3.2),                    # 375
+    dict(shape=(130, 121, 60), nu=60, nv=60, na=337, du=3.2, batch=2),           # 319
     dict(shape=(130, 121, 64), nu=60, nv=64, na=397, du=3.3),
     dict(shape=(130, 121, 100), nu=60, nv=100, na=397, du=3.0, sv=-0.4, dv=0.9),
 ]

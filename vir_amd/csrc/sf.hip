@@ -1122,14 +1122,15 @@ static bool sf_par3_bp_col_ok(const SFGeo& G) {
 // ms at 256^2 however few there are.  An item needs blocks (counted by the rows
 // in use) to make up for it: below 2.75 pixels as many as let a batch fill
 // the chip, from 2.75 on as many as win alone.  2.6 | 2.8 | 3.2 | 4 pixels, gather
-// over tile, 64 rows: 405 blocks, one item 1.58 | 1.61 | 1.34 | 0.82, eight 4.4 | 4.0 |
-// 3.5 | 2.9; 144: 0.89 | 0.78 | 0.74 | 0.55, 2.9 | 2.6 | 2.2 | 1.8; 48: 0.66 | 0.65 | 0.69 |
-// 0.52, 1.8 | 1.5 | 1.6 | 1.1; 20: 0.51 | 0.52 | 0.51 | 0.40, 1.0 | 1.0 | 0.9 | 0.7.
+// over tile, 64 rows: 450 | 405 | 360 | 270 blocks, one item 1.58 | 1.61 | 1.34 | 0.82,
+// eight 4.4 | 4.0 | 3.5 | 2.9; 160 | 144 | 128 | 96: 0.89 | 0.78 | 0.74 | 0.55, 2.9 | 2.6 |
+// 2.2 | 1.8; 48 | 48 | 32 | 32: 0.66 | 0.65 | 0.69 | 0.52, 1.8 | 1.5 | 1.6 | 1.1; 20 | 20 | 16 |
+// 12: 0.51 | 0.52 | 0.51 | 0.40, 1.0 | 1.0 | 0.9 | 0.7.
 static bool sf_par3_tiled_ok(const SFGeo& G) {
     if (!(G.dv <= G.d) || G.nv < 6) return false;
     if (G.du <= 2.5f * G.d) return true;
     const double full = (double)((G.na + kVG - 1) / kVG) * ((G.nu + kTUB - 1) / kTUB) * G.nv / kTV;
-    return G.du <= 2.75f * G.d ? full >= 48.0 : G.du <= 3.2f * G.d && full >= 400.0;
+    return G.du <= 2.75f * G.d ? full >= 48.0 : G.du <= 3.2f * G.d && full >= 350.0;
 }
 
 // An item with at most this many blocks (two a CU) takes two wave groups a
