@@ -1,0 +1,69 @@
+"""Cone-beam projections of volumes and detectors a few slabs (rows) thick, on
+both sides of the lines between the routes, against the one-thread-per-output
+kernels.
+
+Overlaps are formed in cells (rows) instead of detector units: as in
+test_cone_tiles_gpu a boundary of n cells rounds by up to 2^-24 n / 2 * 2, here
+below 6e-6 cell, random in sign over at least 8 views or lines: relative L2 below
+3e-6.  Bar 5e-6.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+BAR = 5e-6
+
+
+def _per_output(P, name, x, shape):
+    import torch
+    from vir_amd import _lib
+    from vir_amd.device import stream
+    out = torch.empty(shape, device="cuda")
+    trig = ([_lib.ptr(P.ang)] if name.startswith("vir_sf") else []) + [_lib.ptr(P.cos), _lib.ptr(P.sin)]
+    _lib.check(getattr(_lib.lib(), name)(P.g, *trig, _lib.ptr(x), _lib.ptr(out), getattr(P, "fp_scale", 1.0),
+                                         _lib.VIR_PER_OUTPUT, stream()), name)
+    return out
+
+
+def _rel(a, b):
+    assert float(b.abs().max()) > 0
+    return float((a.double() - b.double()).norm() / b.double().norm())
+
+
+@pytest.mark.parametrize("kind", ["dd", "sf"])
+@pytest.mark.parametrize("nx,ny,nz,nv,batch", [
+    (150, 149, 3, 3, 1), (150, 149, 5, 30, 1), (150, 149, 13, 12, 1), (150, 149, 18, 18, 1), (64, 66, 4, 5, 1),
+    (130, 131, 66, 9, 1), (45, 40, 7, 6, 30),
+])
+def test_backprojection_of_thin_volumes(nx, ny, nz, nv, batch, kind):
+    import torch
+    from vir_amd.sys_mat.dd import DDProjector
+    from vir_amd.sys_mat.pd import SFProjector
+    if batch > 1 and kind == "dd":
+        pytest.skip("no batch")
+    kw = dict(nv=nv, DSO=4.0 * nx, DSD=8.0 * nx, du=2.0, dv=2.0, su=0.25, sv=-0.2)
+    ang = np.arange(9) * (2 * np.pi / 9)
+    nu = int(1.3 * nx)
+    P = DDProjector((nx, ny, nz), ang, nu, "cone", **kw) if kind == "dd" else \
+        SFProjector((nx, ny, nz), ang, nu, "cone", batch=batch, **kw)
+    y = torch.from_numpy(np.random.default_rng(nz).uniform(0.2, 1.0, P.sino_shape).astype(np.float32)).cuda()
+    shape = P.img_shape if kind == "dd" else P.vol_shape
+    a = P.bp(y)
+    assert _rel(a, _per_output(P, "vir_ddcone_bp" if kind == "dd" else "vir_sf_bp", y, shape)) <= BAR
+    assert torch.equal(a, P.bp(y))
+    assert torch.allclose(P.bp(y, out=a.clone(), accumulate=True), 2 * a, rtol=1e-6, atol=0)
+
+
+@pytest.mark.parametrize("kind", ["dd", "sf"])
+def test_infinite_rows_of_thin_volumes(kind):
+    import torch
+    from vir_amd.sys_mat.dd import DDProjector
+    from vir_amd.sys_mat.pd import SFProjector
+    P = (DDProjector if kind == "dd" else SFProjector)((150, 149, 5), np.arange(5) * 1.3, 200, "cone", nv=9, DSO=600.0,
+                                                       DSD=1200.0, du=2.0, dv=2.0)
+    y = torch.ones(P.sino_shape, device="cuda")
+    y[2, 90, 4] = float("inf")
+    y[3, 91, 3] = float("nan")
+    a, b = P.bp(y), _per_output(P, "vir_ddcone_bp" if kind == "dd" else "vir_sf_bp", y, P.img_shape)
+    assert torch.isinf(b).any() and torch.isnan(b).any()
+    assert torch.equal(torch.isinf(a), torch.isinf(b)) and torch.equal(torch.isnan(a), torch.isnan(b))

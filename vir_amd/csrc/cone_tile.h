@@ -28,6 +28,8 @@
 // 128^3, 180 views of 192^2: 5.5 -> 0.82 ms / 2.7 -> 0.59 ms; separable footprint
 // 120 x 132 x 101, 150 views of 187 x 150: 8.3 -> 0.98 ms / 2.1 -> 0.55 ms.
 #pragma once
+#include <type_traits>
+
 #include "vir_common.h"
 
 namespace vir {
@@ -99,10 +101,12 @@ __device__ __forceinline__ double ct_sum(const float* __restrict__ p, const doub
 // The same where values of zero weight may be infinite: they do not count.
 template <int NS>
 __device__ __forceinline__ double ct_sum_some(const float* __restrict__ p, const double (&w)[NS]) {
+    float x[NS];
+#pragma unroll
+    for (int q = 0; q < NS; ++q) x[q] = p[q];
     double s = 0.0;
 #pragma unroll
-    for (int q = 0; q < NS; ++q)
-        if (w[q] > 0.0) s = __builtin_fma((double)p[q], w[q], s);
+    for (int q = 0; q < NS; ++q) s = __builtin_fma((double)(w[q] > 0.0 ? x[q] : 0.0f), w[q], s);
     return s;
 }
 
@@ -438,6 +442,25 @@ __global__ __launch_bounds__(256) void k_cone_bp_col(Geo G, const float* __restr
     vol[o] = res;
 }
 
+// One thread per voxel, with the column kernel's terms in its order: the same bits.
+template <class M, class Geo, int NS>
+__global__ __launch_bounds__(256) void k_cone_bp_vox(Geo G, const float* __restrict__ ang,
+                                                    const float* __restrict__ cs, const float* __restrict__ sn,
+                                                    const float* __restrict__ sino, float* __restrict__ vol,
+                                                    int accumulate, int64_t n) {
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (t >= n) return;
+    int64_t r = t / G.nz;
+    const int iz = (int)(t % G.nz), iy = (int)(r % G.ny);
+    r /= G.ny;
+    const int ix = (int)(r % G.nx);
+    sino += (r / G.nx) * (int64_t)G.na * G.nu * G.nv;
+    const double acc = ct_bp_one<M, Geo, NS>(G, ang, cs, sn, sino, ix, iy, iz);
+    float res = (float)(acc * (double)M::bp_unit(G)) * G.out_scale;
+    if (accumulate) res += vol[t];
+    vol[t] = res;
+}
+
 // Cells a v (z) interval of at most `len` cells can meet, as the NS of the
 // kernels above, or 0 where they do not apply (intervals longer than 2.9
 // cells, fewer than NS cells in all, or so many that ct_first's margin would
@@ -466,13 +489,26 @@ int ct_bp(const Geo& G, int nb, int ns, const float* ang, const float* cosv, con
           float* vol, int acc, hipStream_t st, const char* what) {
     const int nzt = (G.nz + 63) / 64;
     const int64_t ncol = (int64_t)nb * G.nx * G.ny * nzt;
-    const dim3 grd((unsigned)((ncol + 3) / 4)), blk(256);
-    if (ns == 2)
-        hipLaunchKernelGGL((k_cone_bp_col<M, Geo, 2>), grd, blk, 0, st, G, ang, cosv, sinv, sino, vol, acc, nzt, ncol);
-    else if (ns == 3)
-        hipLaunchKernelGGL((k_cone_bp_col<M, Geo, 3>), grd, blk, 0, st, G, ang, cosv, sinv, sino, vol, acc, nzt, ncol);
-    else
-        hipLaunchKernelGGL((k_cone_bp_col<M, Geo, 4>), grd, blk, 0, st, G, ang, cosv, sinv, sino, vol, acc, nzt, ncol);
+    // Thin volumes leave most lanes of a column idle: with more columns than fill
+    // the chip a thread a voxel is faster up to about 18 slabs.  A view costs
+    // about 0.1 us a thousand columns or 0.4 us and 0.33 a thousand waves of
+    // voxels.  Columns | voxels in us, distance driven, 60 views: 64^2 x 8 38 | 54;
+    // 128^2 x 4 106 | 55, x 12 105 | 83, x 16 105 | 101; 256^2 x 3 371 | 82, x 8 368 |
+    // 178, x 16 371 | 332; 512^2 x 16, 30 views, 772 | 638, x 70 1558 | 2708.  Both give
+    // the same bits, so the batch may count.
+    const int64_t n = (int64_t)nb * G.nx * G.ny * G.nz;
+    const bool thin = (double)G.nz / nzt < 19.0 - 8e4 / (double)ncol;
+    const dim3 grd((unsigned)(((thin ? (n + 63) / 64 : ncol) + 3) / 4)), blk(256);
+    const auto run = [&](auto slots) {
+        constexpr int NS = decltype(slots)::value;
+        if (thin)
+            hipLaunchKernelGGL((k_cone_bp_vox<M, Geo, NS>), grd, blk, 0, st, G, ang, cosv, sinv, sino, vol, acc, n);
+        else
+            hipLaunchKernelGGL((k_cone_bp_col<M, Geo, NS>), grd, blk, 0, st, G, ang, cosv, sinv, sino, vol, acc, nzt, ncol);
+    };
+    if (ns == 2) run(std::integral_constant<int, 2>{});
+    else if (ns == 3) run(std::integral_constant<int, 3>{});
+    else run(std::integral_constant<int, 4>{});
     return check_hip(hipGetLastError(), what);
 }
 
