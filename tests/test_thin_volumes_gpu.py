@@ -67,3 +67,17 @@ def test_infinite_rows_of_thin_volumes(kind):
     a, b = P.bp(y), _per_output(P, "vir_ddcone_bp" if kind == "dd" else "vir_sf_bp", y, P.img_shape)
     assert torch.isinf(b).any() and torch.isnan(b).any()
     assert torch.equal(torch.isinf(a), torch.isinf(b)) and torch.equal(torch.isnan(a), torch.isnan(b))
+
+
+@pytest.mark.parametrize("kind", ["dd", "sf"])
+@pytest.mark.parametrize("nv,na,nu", [(3, 140, 400), (3, 120, 400), (4, 177, 400), (4, 176, 400), (5, 180, 400)])
+def test_projection_onto_few_rows(nv, na, nu, kind):
+    """25 blocks a view: 3 rows of 132 views and 4 of 176 are on the line."""
+    import torch
+    from vir_amd.sys_mat.dd import DDProjector
+    from vir_amd.sys_mat.pd import SFProjector
+    n = 24
+    P = (DDProjector if kind == "dd" else SFProjector)((n, n + 1, 7), np.arange(na) * (2 * np.pi / na), nu, "cone", nv=nv,
+                                                       DSO=4.0 * n, DSD=8.0 * n, du=0.2, dv=2.0, sv=0.3)
+    x = torch.from_numpy(np.random.default_rng(nv).uniform(0.2, 1.0, P.img_shape).astype(np.float32)).cuda()
+    assert _rel(P.fp(x), _per_output(P, "vir_ddcone_fp" if kind == "dd" else "vir_sf_fp", x, P.sino_shape)) <= BAR

@@ -470,6 +470,17 @@ inline int ct_slots(double len, int n) {
     return n >= ns && n <= 20000 ? ns : 0;
 }
 
+// True when the forward tile, whose 64 lanes run along v, is slower than one
+// thread per output: up to four rows, and blocks of one item (so that its bits
+// don't depend on the batch) that fill the chip several times over.  Tile | per
+// output, us, rows as slabs, distance driven: 256^2, 360 views (8640 blocks) 3 rows
+// 1701 | 1305, 4: 1709 | 1522, 6: (32 slabs) 2041 | 2204; 128^2, 360 views (4320)
+// 3: 508 | 441, 4: 500 | 538; 256^2, 60 views (1440) 3: 371 | 630.
+template <class Geo>
+bool ct_few_rows(const Geo& G) {
+    return G.nv <= 4 && (int64_t)G.na * ((G.nu + kCtBins - 1) / kCtBins) > 1100 * (int64_t)G.nv;
+}
+
 template <class M, class Geo>
 int ct_fp(const Geo& G, int nb, int ns, const float* ang, const float* cosv, const float* sinv, const float* vol,
           float* sino, int acc, hipStream_t st, const char* what) {

@@ -482,10 +482,11 @@ __global__ __launch_bounds__(256) void k_ddcone_bp(DDGeo G, const float* __restr
 
 // Slabs a detector row (forward) or rows a slab (backward) can meet, from the
 // magnifications DSD/(DSO + R) and DSD/(DSO - R) of the grid's rim; 0: the
-// tiles do not apply.
+// tiles do not apply or do not pay.
 static int ddcone_slots(const DDGeo& G, bool fp, uint32_t flags) {
     if (flags & VIR_PER_OUTPUT) return 0;
     const double R = 0.5 * std::sqrt((double)G.nx * G.nx + (double)G.ny * G.ny) * G.d;
+    if (fp && ct_few_rows(G)) return 0;
     return fp ? ct_slots((double)G.dv * ((double)G.DSO + R) / ((double)G.DSD * G.d), G.nz)
               : ct_slots((double)G.d * G.DSD / (((double)G.DSO - R) * G.dv), G.nv);
 }

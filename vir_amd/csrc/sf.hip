@@ -1226,10 +1226,12 @@ __global__ __launch_bounds__(256) void k_sf_bp(SFGeo G, const float* __restrict_
 
 // Slabs a detector row (forward) or rows a slab (backward) of the cone
 // geometry can meet, from the magnifications at the grid's rim (times 1/cos of
-// the largest fan angle, tan <= R/sqrt(DSO^2 - R^2)); 0: the tiles do not apply.
+// the largest fan angle, tan <= R/sqrt(DSO^2 - R^2)); 0: the tiles do not apply or
+// do not pay.
 static int sf_cone_slots(const SFGeo& G, bool fp, uint32_t flags) {
     if (flags & VIR_PER_OUTPUT) return 0;
     const double R = 0.5 * std::sqrt((double)G.nx * G.nx + (double)G.ny * G.ny) * G.d, D = G.DSO;
+    if (fp && ct_few_rows(G)) return 0;
     return fp ? ct_slots((double)G.dv * (D + R) / ((double)G.DSD * G.d), G.nz)
               : ct_slots((double)G.d * G.DSD / (D - R) * (D / std::sqrt(D * D - R * R)) / G.dv, G.nv);
 }
