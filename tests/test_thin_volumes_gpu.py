@@ -81,3 +81,21 @@ def test_projection_onto_few_rows(nv, na, nu, kind):
                                                        DSO=4.0 * n, DSD=8.0 * n, du=0.2, dv=2.0, sv=0.3)
     x = torch.from_numpy(np.random.default_rng(nv).uniform(0.2, 1.0, P.img_shape).astype(np.float32)).cuda()
     assert _rel(P.fp(x), _per_output(P, "vir_ddcone_fp" if kind == "dd" else "vir_sf_fp", x, P.sino_shape)) <= BAR
+
+
+@pytest.mark.parametrize("joseph", [False, True])
+@pytest.mark.parametrize("nx,ny,nz", [(104, 200, 2), (100, 200, 2), (160, 200, 3), (156, 200, 3), (160, 200, 2), (160, 199, 4)])
+def test_ray_driven_backprojection_of_thin_volumes(nx, ny, nz, joseph):
+    """26 x 25 and 40 x 25 bricks: 650 and 1000 are on the lines.  Joseph's samples
+    are placed in voxel units here and along the ray there: a position of up to
+    4 n = 800 voxels rounds by 2^-24 * 800 = 5e-5 voxel, against weights of order
+    one, random over 7 views of a few rays each: bar 3e-5."""
+    import torch
+    from vir_amd.sys_mat.rd import RDProjector
+    nu = 300
+    P = RDProjector((nx, ny, nz), np.arange(7) * (2 * np.pi / 7), nu, "cone", nv=nz + 2, DSO=4.0 * ny, DSD=8.0 * ny, du=2.0,
+                    dv=2.0, su=0.25, sv=(nu - nz - 2) / 2.0, joseph=joseph)
+    y = torch.from_numpy(np.random.default_rng(nz).uniform(0.2, 1.0, P.sino_shape).astype(np.float32)).cuda()
+    a = P.bp(y)
+    assert _rel(a, _per_output(P, "vir_rd_bp", y, P.img_shape)) <= 3e-5
+    assert torch.equal(a, P.bp(y))

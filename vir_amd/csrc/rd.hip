@@ -785,6 +785,17 @@ static int rd_setup(const vir_rd_geom* g, RDGeo& G) {
     return VIR_OK;
 }
 
+// False for cone-beam volumes so thin that the table kernel, whose 64 lanes run
+// along z, is slower than one thread per voxel: two slabs, or three with
+// interpolation, in bricks enough to fill the chip.  Table | per voxel, us, 60
+// views, slabs: Joseph 128^2 (512 bricks) 2: equal; 150^2 (722) 2: 1206 | 1140; 180^2
+// (1035) 2: 1704 | 1142, 3: 2251 | 1964; 220^2 3: 3123 | 2484, 4: 3108 | 3453; path
+// lengths 180^2 2: 629 | 617, 256^2 2: 983 | 787, 3: 990 | 1426.
+static bool rd_tab_pays(const RDGeo& G, int mode, bool jo) {
+    if (mode != RD_CONE3 || G.nz > (jo ? 3 : 2)) return true;
+    return (int64_t)((G.nx + 3) / 4) * ((G.ny + 7) / 8) < (jo && G.nz == 2 ? 650 : 1000);
+}
+
 // The table kernels' launch.  Cone: four columns a wave (a 4 x 8 x 64 brick,
 // its rays set up once per 2048 voxels) where that gives the chip two blocks
 // a CU, else one column a wave.  2-D: sixteen waves share a tile's views
@@ -873,7 +884,8 @@ int vir_rd_bp(const vir_rd_geom* geom, const float* cosv, const float* sinv, con
     hipStream_t st = as_stream(stream);
     // VIR_COMPAT's clamped rays reach voxels they do not pass through: only
     // the per-voxel gather visits those
-    if (!G.compat && !(flags & VIR_PER_OUTPUT)) return rd_bp_tab(G, geom->mode, jo, cosv, sinv, sino, img, acc, st);
+    if (!G.compat && !(flags & VIR_PER_OUTPUT) && rd_tab_pays(G, geom->mode, jo))
+        return rd_bp_tab(G, geom->mode, jo, cosv, sinv, sino, img, acc, st);
     const int64_t n = (int64_t)G.nx * G.ny * G.nz;
     dim3 grd((unsigned)((n + 255) / 256));
 #define VIR_RD_BP(M)                                                                                        \
