@@ -589,6 +589,10 @@ int vir_tv_chambolle_pair(int32_t ndim, int32_t nx, int32_t ny, int32_t nz,
                           float weight, float tau, int32_t iters, float *dmax,
                           void *stream);
 
+/* 1 where vir_tv_chambolle_pair is the faster of the two for images of this
+ * size, else 0 (small and thin ones, one axis). */
+int vir_tv_pair_pays(int32_t ndim, int32_t nx, int32_t ny, int32_t nz);
+
 /* Chambolle-Pock iteration for TV-regularised reconstruction (tv.py:229-294),
  * on volumes (nx, ny, nz) with periodic differences (tv.py:207-224); nz == 1
  * is 2-D.  z holds ndim (2 or 3) planes of the volume's size.

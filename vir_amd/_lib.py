@@ -153,6 +153,7 @@ SIGNATURES = {
     "vir_tv": (ctypes.c_int, [P, I64, I32, I32, I32, F32, F32, P, P, P, U32, P]),
     "vir_sqdist": (ctypes.c_int, [P, P, P, I64, P, P, P]),
     "vir_tv_chambolle_pair": (ctypes.c_int, [I32, I32, I32, I32, P, P, P, P, F32, F32, I32, P, P]),
+    "vir_tv_pair_pays": (ctypes.c_int, [I32, I32, I32, I32]),
     "vir_tv_chambolle": (ctypes.c_int, [I32, I32, I32, I32, P, P, P, P, F32, F32, I32, P, P]),
     "vir_pdhg_dual_tv": (ctypes.c_int, [I32, I32, I32, P, P, F32, P]),
     "vir_pdhg_dual_data": (ctypes.c_int, [I64, P, P, P, F32, P, P]),

@@ -314,25 +314,57 @@ __global__ __launch_bounds__(256) void k_tvd_zero(float* __restrict__ dmax) {
     for (int i = threadIdx.x; i < kTvdBlocks; i += 256) dmax[i] = 0.0f;
 }
 
-// Iterations on two copies of q in turn; *cur: the copy that holds q.  A
-// volume's blocks (eight waves of three rows) run two to a CU; its chunks of
-// planes are as long as 512 blocks allow, since every chunk adds 3K - 1 planes
-// of lead (400 blocks: 4.27 ms for 50 iterations at 256^3, against 3.99).  An
-// image's waves work alone: 2048 of them.
+// Tiles, planes a chunk and chunks of a pass of K iterations.  A volume's blocks
+// (eight waves of three rows) run two to a CU; its chunks of planes are as long
+// as 512 blocks allow, since every chunk adds 3K - 1 planes of lead (400 blocks:
+// 4.27 ms for 50 iterations at 256^3, against 3.99).  An image's waves work
+// alone: 2048 of them.
+struct TvdPlan {
+    int ntz, nty, chunk;
+    int64_t n;  // blocks (3-D) or waves (2-D)
+};
+
+template <int ND, int K>
+static TvdPlan tvd_plan(const TvdShape& S) {
+    constexpr int R = ND == 3 ? 3 : 1, G = ND == 3 ? 8 : 4;
+    const int nz = ND == 3 ? S.n2 : S.n1, ny = ND == 3 ? S.n1 : 1;
+    TvdPlan P;
+    P.ntz = (nz + 63 - 2 * K) / (64 - 2 * K);
+    P.nty = ND == 3 ? (ny + G * R - 2 * K - 1) / (G * R - 2 * K) : 1;
+    const int64_t tiles = (int64_t)P.ntz * P.nty, want = std::max<int64_t>(1, (ND == 3 ? 512 : 2048) / tiles);
+    P.chunk = (int)std::max<int64_t>(ND == 3 ? 8 : 16, (S.n0 + want - 1) / want);
+    P.n = tiles * ((S.n0 + P.chunk - 1) / P.chunk);
+    return P;
+}
+
+// Iterations on two copies of q in turn; *cur: the copy that holds q.
 template <int ND, int K>
 static void tvd_march(const TvdShape& S, const float* g, float* const* q, int32_t* cur, float weight, float tau,
                       float* dmax, hipStream_t st) {
     constexpr int R = ND == 3 ? 3 : 1, G = ND == 3 ? 8 : 4;
-    const int nz = ND == 3 ? S.n2 : S.n1, ny = ND == 3 ? S.n1 : 1;
-    const int ntz = (nz + 63 - 2 * K) / (64 - 2 * K), nty = ND == 3 ? (ny + G * R - 2 * K - 1) / (G * R - 2 * K) : 1;
-    const int64_t tiles = (int64_t)ntz * nty, want = std::max<int64_t>(1, (ND == 3 ? 512 : 2048) / tiles);
-    const int chunk = (int)std::max<int64_t>(ND == 3 ? 8 : 16, (S.n0 + want - 1) / want);
-    const int64_t n = tiles * ((S.n0 + chunk - 1) / chunk);
+    const TvdPlan P = tvd_plan<ND, K>(S);
     if (dmax) hipLaunchKernelGGL(k_tvd_zero, dim3(1), dim3(256), 0, st, dmax);
-    hipLaunchKernelGGL((k_tvd_march<ND, K, R, G>), dim3((unsigned)(ND == 3 ? n : (n + G - 1) / G)), dim3(64 * G), 0, st,
-                       S, q[*cur], q[1 - *cur], g, tau, tau / weight, dmax, chunk, nty, ntz);
+    hipLaunchKernelGGL((k_tvd_march<ND, K, R, G>), dim3((unsigned)(ND == 3 ? P.n : (P.n + G - 1) / G)), dim3(64 * G), 0,
+                       st, S, q[*cur], q[1 - *cur], g, tau, tau / weight, dmax, P.chunk, P.nty, P.ntz);
     if (dmax) hipLaunchKernelGGL(k_tvd_max, dim3(1), dim3(256), 0, st, dmax, kTvdBlocks);
     *cur = 1 - *cur;
+}
+
+// Whether a pass of K iterations is faster than K times two launches.  It marches
+// plane by plane, in serial, and its lanes lie along the last axis, so small
+// and thin images are better off with the launches: those take about 3 us and
+// 11.5 (images 8) a million voxels an iteration, at least 8 (7.2); a pass 1.65
+// us a plane up to 256 blocks, 2.35 beyond (images 0.95), and at least 9 us a
+// million voxels.  Launches | passes for ten iterations in us: 64^3 87 | 109, 512
+// x 512 x 1 83 | 362, x 4 148 | 368, x 16 478 | 367, 256^3 2499 | 759, 200000 x 4 111 | 189,
+// 2048^2 370 | 96.  Of 644 sizes measured three take up to 1.2 times the other
+// way's time.
+template <int ND, int K>
+static bool tvd_pays(const TvdShape& S) {
+    const TvdPlan P = tvd_plan<ND, K>(S);
+    const double m = 1e-6 * (double)S.n, planes = std::min(P.chunk, S.n0) + 3 * K - 1;
+    if (ND == 2) return planes * 0.95 <= K * std::max(7.2, 3.0 + 8.0 * m);
+    return std::max(planes * (P.n <= 256 ? 1.65 : 2.35), 9.0 * m) <= K * std::max(8.0, 3.0 + 11.5 * m);
 }
 
 template <int ND, int K>
@@ -388,6 +420,12 @@ int vir_tv_chambolle(int32_t ndim, int32_t nx, int32_t ny, int32_t nz, const flo
     if (ndim == 1) return tvd_run<1>(S, g, q, v, u, weight, tau, iters, dmax, st);
     if (ndim == 2) return tvd_run<2>(S, g, q, v, u, weight, tau, iters, dmax, st);
     return tvd_run<3>(S, g, q, v, u, weight, tau, iters, dmax, st);
+}
+
+int vir_tv_pair_pays(int32_t ndim, int32_t nx, int32_t ny, int32_t nz) {
+    TvdShape S;
+    if (ndim < 2 || tvd_args(ndim, nx, ny, nz, 1.0f, 1.0f, 1, S)) return 0;
+    return ndim == 2 ? tvd_pays<2, 5>(S) : tvd_pays<3, 2>(S);
 }
 
 int vir_tv_chambolle_pair(int32_t ndim, int32_t nx, int32_t ny, int32_t nz, const float* g, float* q0, float* q1,

@@ -45,9 +45,9 @@ def denoise_tv_chambolle(image, weight=0.1, eps=2.0e-4, max_num_iter=200, tau=No
     q = torch.zeros((nd,) + shape, dtype=torch.float32, device=g.device)
     u = torch.empty_like(g)
     # a second copy of q lets a pass over memory do several iterations; where
-    # there is no room for it, one residual image does
+    # that does not pay or there is no room for it, one residual image does
     q2 = v = None
-    if nd > 1:
+    if _lib.lib().vir_tv_pair_pays(nd, dims[0], dims[1], dims[2]):
         try:
             q2 = torch.empty_like(q)
         except torch.OutOfMemoryError:
