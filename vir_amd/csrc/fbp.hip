@@ -23,6 +23,7 @@
 // detector; positions, weights and sums in double), times the caller's scale.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "vir_common.h"
 
@@ -30,61 +31,66 @@ namespace vir {
 
 constexpr int kFbpMaxBins = 4096;
 
-// Filtering: a Toeplitz product in float64.  A block computes 256 outputs (four
-// consecutive ones a lane) of two rows; its four waves take a quarter of every
-// chunk of the sum and add their parts in wave order.  The taps g[|i - j|] of
-// the tile lie in LDS as one float64 sequence, so moving to the next j shifts a
-// lane's four taps by one: per j a tap and two row values are read for eight
-// multiply-adds.  (One output a thread, converting a row value and a tap for
-// every multiply-add: 169 us for 720 rows of 888; 41 us.)
-constexpr int kFfOut = 256, kFfRows = 2, kFfChunk = 512, kFfWaves = 4;
-constexpr int kFfTaps = kFfOut + kFfChunk;
+// Filtering: a Toeplitz product in float64.  A block computes OUT outputs of
+// 512 / OUT rows: four consecutive ones of two rows a lane, OUT / 4 lanes a row.
+// Its four waves take a quarter of every chunk of the sum and add their parts in
+// wave order.  The taps g[|i - j|] of the tile lie in LDS as one float64 sequence,
+// so moving to the next j shifts a lane's four taps by one: per j a tap and two
+// row values are read for eight multiply-adds.  (One output a thread, converting
+// a row value and a tap for every multiply-add: 169 us for 720 rows of 888; 41 us.)
+// Rows of up to 128 values take the smallest OUT that holds them: 100000 rows of
+// 16, 64, 128 values 27, 48, 98 us, as two rows of 256 outputs 129, 223, 333.
+constexpr int kFfWaves = 4;
 
 // place of tap w in LDS: every four taps are followed by an empty one, which
 // puts the lanes' reads (four taps apart) on different banks
 __device__ __forceinline__ int ff_at(int w) { return w + (w >> 2); }
 
+template <int OUT>
 __global__ __launch_bounds__(64 * kFfWaves) void k_fbp_filter(const float* __restrict__ sino, int64_t nrows, int nu,
                                                              const float* __restrict__ weight,
                                                              const float* __restrict__ taps, float* __restrict__ out,
                                                              int ntile) {
-    __shared__ double h[kFfTaps + kFfTaps / 4 + 1];
-    __shared__ double row[kFfRows][kFfChunk];
-    __shared__ double red[kFfWaves][kFfRows * kFfOut];
-    const int tid = threadIdx.x, lane = tid & 63;
+    constexpr int ROWS = 512 / OUT, CHUNK = OUT < 256 ? OUT : 512, TAPS = OUT + CHUNK, LPR = OUT / 4;
+    constexpr int PITCH = CHUNK + (OUT < 256 ? 4 : 0);  // (rows that a wave reads together: different banks)
+    __shared__ double h[TAPS + TAPS / 4 + 1];
+    __shared__ double row[ROWS][PITCH];
+    __shared__ double red[kFfWaves][ROWS * OUT];
+    const int tid = threadIdx.x, sub = (tid & 63) % LPR, ra = 2 * ((tid & 63) / LPR);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int i0 = (int)(blockIdx.x % ntile) * kFfOut;
-    const int64_t r0 = (int64_t)(blockIdx.x / ntile) * kFfRows;
-    double acc[kFfRows][4] = {};
-    for (int jc = 0; jc < nu; jc += kFfChunk) {
+    const int i0 = (int)(blockIdx.x % ntile) * OUT;
+    const int64_t r0 = (int64_t)(blockIdx.x / ntile) * ROWS;
+    double acc[2][4] = {};
+    for (int jc = 0; jc < nu; jc += CHUNK) {
         __syncthreads();
-        // h[w] = g[|i0 + w - (jc + kFfChunk)|], w = 0 .. kFfTaps - 1: the tap of
-        // output i0 + i and input jc + j lies at w = kFfChunk + i - j
-        for (int w = tid; w < kFfTaps; w += 64 * kFfWaves) {
-            const int k = abs(i0 + w - (jc + kFfChunk));
+        // h[w] = g[|i0 + w - (jc + CHUNK)|], w = 0 .. TAPS - 1: the tap of output
+        // i0 + i and input jc + j lies at w = CHUNK + i - j
+        for (int w = tid; w < TAPS; w += 64 * kFfWaves) {
+            const int k = abs(i0 + w - (jc + CHUNK));
             h[ff_at(w)] = k < nu ? (double)taps[k] : 0.0;
         }
-        for (int e = tid; e < kFfRows * kFfChunk; e += 64 * kFfWaves) {
-            const int r = e / kFfChunk, j = jc + e % kFfChunk;
+        for (int e = tid; e < ROWS * CHUNK; e += 64 * kFfWaves) {
+            const int r = e / CHUNK, j = jc + e % CHUNK;
             float x = 0.0f;
             if (r0 + r < nrows && j < nu) {
                 x = sino[(r0 + r) * nu + j];
                 if (weight) x = x * weight[j];
             }
-            row[r][e % kFfChunk] = (double)x;
+            row[r][e % CHUNK] = (double)x;
         }
         __syncthreads();
         // this wave's quarter, four inputs at a time: taps w - 3 .. w + 3 of
-        // w = kFfChunk + 4 lane - j, of which the upper three stay from before
-        const int ja = wave * (kFfChunk / kFfWaves), jb = min(ja + kFfChunk / kFfWaves, nu - jc);
+        // w = CHUNK + 4 sub - j, of which the upper three stay from before
+        const int ja = wave * (CHUNK / kFfWaves), jb = min(ja + CHUNK / kFfWaves, nu - jc);
         if (ja >= jb) continue;
-        const double* hl = h + ff_at(kFfChunk + 4 * lane - ja);
+        const double* hl = h + ff_at(CHUNK + 4 * sub - ja);
         double t0 = hl[0], t1 = hl[1], t2 = hl[2], t3 = hl[3];
         for (int j = ja; j < jb; j += 4, hl -= 5) {
             const double s0 = hl[-5], s1 = hl[-4], s2 = hl[-3], s3 = hl[-2];  // w - 4 .. w - 1
 #pragma unroll
-            for (int r = 0; r < kFfRows; ++r) {
-                const double x0 = row[r][j], x1 = row[r][j + 1], x2 = row[r][j + 2], x3 = row[r][j + 3];
+            for (int r = 0; r < 2; ++r) {
+                const double* x = row[ra + r] + j;
+                const double x0 = x[0], x1 = x[1], x2 = x[2], x3 = x[3];
                 const auto f = [](double x, double y, double z) { return __builtin_fma(x, y, z); };
                 acc[r][0] = f(x3, s1, f(x2, s2, f(x1, s3, f(x0, t0, acc[r][0]))));
                 acc[r][1] = f(x3, s2, f(x2, s3, f(x1, t0, f(x0, t1, acc[r][1]))));
@@ -95,13 +101,13 @@ __global__ __launch_bounds__(64 * kFfWaves) void k_fbp_filter(const float* __res
         }
     }
 #pragma unroll
-    for (int r = 0; r < kFfRows; ++r)
+    for (int r = 0; r < 2; ++r)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) red[wave][r * kFfOut + 4 * lane + q] = acc[r][q];
+        for (int q = 0; q < 4; ++q) red[wave][(ra + r) * OUT + 4 * sub + q] = acc[r][q];
     __syncthreads();
-    for (int e = tid; e < kFfRows * kFfOut; e += 64 * kFfWaves) {
-        const int64_t r = r0 + e / kFfOut;
-        const int i = i0 + e % kFfOut;
+    for (int e = tid; e < ROWS * OUT; e += 64 * kFfWaves) {
+        const int64_t r = r0 + e / OUT;
+        const int i = i0 + e % OUT;
         if (r >= nrows || i >= nu) continue;
         double s = red[0][e];
 #pragma unroll
@@ -273,9 +279,17 @@ int vir_fbp_filter(const float* sino, int64_t nrows, int32_t nu, const float* we
     if (nrows == 0) return VIR_OK;
     if (!sino || !taps || !out) return fail_arg("NULL pointer argument");
     if (sino == out) return fail_arg("in-place filtering is not supported");
-    const int ntile = (nu + kFfOut - 1) / kFfOut;
-    hipLaunchKernelGGL(k_fbp_filter, dim3((unsigned)((nrows + kFfRows - 1) / kFfRows * ntile)), dim3(64 * kFfWaves), 0,
-                       as_stream(stream), sino, nrows, nu, weight, taps, out, ntile);
+    hipStream_t st = as_stream(stream);
+    const auto run = [&](auto width) {
+        constexpr int OUT = decltype(width)::value, ROWS = 512 / OUT;
+        const int ntile = (nu + OUT - 1) / OUT;
+        hipLaunchKernelGGL(k_fbp_filter<OUT>, dim3((unsigned)((nrows + ROWS - 1) / ROWS * ntile)), dim3(64 * kFfWaves), 0,
+                           st, sino, nrows, nu, weight, taps, out, ntile);
+    };
+    if (nu <= 32) run(std::integral_constant<int, 32>{});
+    else if (nu <= 64) run(std::integral_constant<int, 64>{});
+    else if (nu <= 128) run(std::integral_constant<int, 128>{});
+    else run(std::integral_constant<int, 256>{});
     return check_hip(hipGetLastError(), "vir_fbp_filter launch");
 }
 
