@@ -481,6 +481,13 @@ bool ct_few_rows(const Geo& G) {
     return G.nv <= 4 && (int64_t)G.na * ((G.nu + kCtBins - 1) / kCtBins) > 1100 * (int64_t)G.nv;
 }
 
+// Threads that one item's launch takes.
+template <class Geo>
+int64_t ct_threads(const Geo& G, bool fp) {
+    return fp ? (int64_t)G.na * ((G.nu + kCtBins - 1) / kCtBins) * ((G.nv + 63) / 64) * 256
+              : (int64_t)G.nx * G.ny * ((G.nz + 63) / 64) * 64 + 256;
+}
+
 template <class M, class Geo>
 int ct_fp(const Geo& G, int nb, int ns, const float* ang, const float* cosv, const float* sinv, const float* vol,
           float* sino, int acc, hipStream_t st, const char* what) {

@@ -484,7 +484,7 @@ __global__ __launch_bounds__(256) void k_ddcone_bp(DDGeo G, const float* __restr
 // magnifications DSD/(DSO + R) and DSD/(DSO - R) of the grid's rim; 0: the
 // tiles do not apply or do not pay.
 static int ddcone_slots(const DDGeo& G, bool fp, uint32_t flags) {
-    if (flags & VIR_PER_OUTPUT) return 0;
+    if ((flags & VIR_PER_OUTPUT) || ct_threads(G, fp) > kLaunchThreads) return 0;
     const double R = 0.5 * std::sqrt((double)G.nx * G.nx + (double)G.ny * G.ny) * G.d;
     if (fp && ct_few_rows(G)) return 0;
     return fp ? ct_slots((double)G.dv * ((double)G.DSO + R) / ((double)G.DSD * G.d), G.nz)
@@ -527,7 +527,7 @@ static int dd2d_fp(const vir_dd_geom* geom, const float* cosv, const float* sinv
     dim3 grd((unsigned)((n + 255) / 256));
     int acc = (flags & VIR_ACCUMULATE) ? 1 : 0;
     hipStream_t st = as_stream(stream);
-    if (!(flags & VIR_PER_OUTPUT)) {
+    if (!(flags & VIR_PER_OUTPUT) && ft_threads(G, true) <= kLaunchThreads) {
         if (geom->mode == DD_PAR)
             return ft_fp<DDFlat<DD_PAR>>(G, 1, nullptr, cosv, sinv, img, sino, acc, st, E, "vir_dd2d_fp launch");
         if (geom->mode == DD_FAN_FLAT)
@@ -553,7 +553,7 @@ static int dd2d_bp(const vir_dd_geom* geom, const float* cosv, const float* sinv
     dim3 grd((unsigned)((n + 255) / 256));
     int acc = (flags & VIR_ACCUMULATE) ? 1 : 0;
     hipStream_t st = as_stream(stream);
-    if (!(flags & VIR_PER_OUTPUT)) {
+    if (!(flags & VIR_PER_OUTPUT) && ft_threads(G, false) <= kLaunchThreads) {
         if (geom->mode == DD_PAR)
             return ft_bp<DDFlat<DD_PAR>>(G, 1, nullptr, cosv, sinv, sino, img, acc, st, E, "vir_dd2d_bp launch");
         if (geom->mode == DD_FAN_FLAT)

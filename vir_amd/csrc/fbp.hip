@@ -283,8 +283,12 @@ int vir_fbp_filter(const float* sino, int64_t nrows, int32_t nu, const float* we
     const auto run = [&](auto width) {
         constexpr int OUT = decltype(width)::value, ROWS = 512 / OUT;
         const int ntile = (nu + OUT - 1) / OUT;
-        hipLaunchKernelGGL(k_fbp_filter<OUT>, dim3((unsigned)((nrows + ROWS - 1) / ROWS * ntile)), dim3(64 * kFfWaves), 0,
-                           st, sino, nrows, nu, weight, taps, out, ntile);
+        const int64_t most = kLaunchThreads / (64 * kFfWaves) / ntile * ROWS;  // rows a launch takes
+        for (int64_t r = 0; r < nrows; r += most) {
+            const int64_t n = std::min(most, nrows - r);
+            hipLaunchKernelGGL(k_fbp_filter<OUT>, dim3((unsigned)((n + ROWS - 1) / ROWS * ntile)), dim3(64 * kFfWaves), 0,
+                               st, sino + r * nu, n, nu, weight, taps, out + r * nu, ntile);
+        }
     };
     if (nu <= 32) run(std::integral_constant<int, 32>{});
     else if (nu <= 64) run(std::integral_constant<int, 64>{});

@@ -368,6 +368,13 @@ __global__ __launch_bounds__(64 * NW) void k_bp2d_tile(Geo G, const float* __res
     }
 }
 
+// Threads that one item's launch takes (at most; fewer where a batch has more tiles).
+template <class Geo>
+int64_t ft_threads(const Geo& G, bool fp) {
+    const int64_t n = fp ? (int64_t)G.na * ((G.nu + kFtBins - 1) / kFtBins) : (int64_t)((G.nx + 15) / 16) * ((G.ny + 15) / 16);
+    return n * (n >= 2048 ? 256 : fp ? 512 : 1024);
+}
+
 // Waves that share a tile: four, or sixteen (eight forward) where the tiles
 // alone would leave CUs without work (forward: in less than about two rounds of
 // resident waves, the edge tiles' short bands leave some idle; four | eight

@@ -792,6 +792,10 @@ static int rd_setup(const vir_rd_geom* g, RDGeo& G) {
 // (1035) 2: 1704 | 1142, 3: 2251 | 1964; 220^2 3: 3123 | 2484, 4: 3108 | 3453; path
 // lengths 180^2 2: 629 | 617, 256^2 2: 983 | 787, 3: 990 | 1426.
 static bool rd_tab_pays(const RDGeo& G, int mode, bool jo) {
+    // (a launch can't have more threads)
+    const int64_t blocks = mode == RD_CONE3 ? (int64_t)((G.nx + 3) / 4) * ((G.ny + 7) / 8) * ((G.nz + 63) / 64)
+                                            : (int64_t)((G.nx + kRd2X - 1) / kRd2X) * ((G.ny + kRd2Y - 1) / kRd2Y);
+    if (blocks * (mode == RD_CONE3 ? 64 * kRdWaves : 256) > kLaunchThreads) return false;
     if (mode != RD_CONE3 || G.nz > (jo ? 3 : 2)) return true;
     return (int64_t)((G.nx + 3) / 4) * ((G.ny + 7) / 8) < (jo && G.nz == 2 ? 650 : 1000);
 }

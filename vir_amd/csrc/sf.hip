@@ -1236,6 +1236,44 @@ static int sf_cone_slots(const SFGeo& G, bool fp, uint32_t flags) {
               : ct_slots((double)G.d * G.DSD / (D - R) * (D / std::sqrt(D * D - R * R)) / G.dv, G.nv);
 }
 
+// Threads that one item's launch takes (at most; fewer in a batch of many).
+static int64_t sf_threads(const SFGeo& G, int mode, bool fp) {
+    if (mode == SF_PAR2 || mode == SF_FAN2) return ft_threads(G, fp);
+    if (mode == SF_CONE3) return ct_threads(G, fp);
+    if (fp) {
+        const int64_t n = (int64_t)((G.na + kVG - 1) / kVG) * ((G.nu + kTUB - 1) / kTUB) * ((G.nv + kTV - 1) / kTV);
+        return n * 64 * kVG * (n <= kParBlocks2 ? 2 : 1);
+    }
+    int shift;
+    const int64_t nzt = (G.nz + 63) / 64, n = (int64_t)((G.nx + 3) / 4) * ((G.ny + 3) / 4) * nzt;
+    return sf_par3_bp_ksteps(G, shift) ? n * (n < kParSplit ? 256 : 64) + 256 : (int64_t)G.nx * G.ny * nzt * 64 + 256;
+}
+
+// A batch in parts, where a launch can't have the threads of all items (items
+// don't depend on their batch); flags gets VIR_PER_OUTPUT where it can't have
+// those of one.
+template <class Call>
+static int sf_parts(const vir_sf_geom* geom, const SFGeo& G, bool fp, const float* src, float* dst, uint32_t& flags,
+                    Call&& call, bool& done) {
+    done = false;
+    if (flags & VIR_PER_OUTPUT) return VIR_OK;
+    const int64_t per = sf_threads(G, geom->mode, fp);
+    if (per > kLaunchThreads) {
+        flags |= VIR_PER_OUTPUT;
+        return VIR_OK;
+    }
+    const int64_t most = kLaunchThreads / per;
+    if (G.nb <= most) return VIR_OK;
+    done = true;
+    const int64_t vox = (int64_t)G.nx * G.ny * G.nz, bins = (int64_t)G.na * G.nu * G.nv;
+    for (int64_t b = 0; b < G.nb; b += most) {
+        vir_sf_geom g = *geom;
+        g.nbatch = (int32_t)std::min<int64_t>(most, G.nb - b);
+        if (const int rc = call(&g, src + b * (fp ? vox : bins), dst + b * (fp ? bins : vox))) return rc;
+    }
+    return VIR_OK;
+}
+
 static int sf_setup(const vir_sf_geom* g, SFGeo& G) {
     if (!g) return fail_arg("geometry is NULL");
     if (g->mode < 0 || g->mode > 3) return fail_arg("mode must be 0..3");
@@ -1296,6 +1334,12 @@ int vir_sf_fp(const vir_sf_geom* geom, const float* ang, const float* cosv, cons
     G.out_scale = out_scale;
     G.unit_amp = (flags & VIR_SF_UNIT_AMPLITUDE) ? 1 : 0;
     G.compat = (flags & VIR_COMPAT) ? 1 : 0;
+    bool done;
+    const uint32_t given = flags;
+    rc = sf_parts(geom, G, true, img, sino, flags, [&](const vir_sf_geom* g, const float* src, float* dst) {
+        return vir_sf_fp(g, ang, cosv, sinv, src, dst, out_scale, given, stream);
+    }, done);
+    if (rc || done) return rc;
     int64_t n = (int64_t)G.nb * G.na * G.nu * G.nv;
     dim3 grd((unsigned)((n + 255) / 256));
     hipStream_t st = as_stream(stream);
@@ -1342,6 +1386,12 @@ int vir_sf_bp(const vir_sf_geom* geom, const float* ang, const float* cosv, cons
     if ((G.na > 0 && (!ang || !cosv || !sinv || !sino)) || !img) return fail_arg("NULL pointer argument");
     G.out_scale = out_scale;
     G.unit_amp = (flags & VIR_SF_UNIT_AMPLITUDE) ? 1 : 0;
+    bool done;
+    const uint32_t given = flags;
+    rc = sf_parts(geom, G, false, sino, img, flags, [&](const vir_sf_geom* g, const float* src, float* dst) {
+        return vir_sf_bp(g, ang, cosv, sinv, src, dst, out_scale, given, stream);
+    }, done);
+    if (rc || done) return rc;
     int64_t n = (int64_t)G.nb * G.nx * G.ny * G.nz;
     dim3 grd((unsigned)((n + 255) / 256));
     hipStream_t st = as_stream(stream);

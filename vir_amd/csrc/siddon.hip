@@ -830,7 +830,7 @@ int vir_siddon_fill(const float* src, const float* trg, int64_t nrays, const vir
 // (records, batch, fused step) sums alike.
 static int fp_split(int64_t nrays, bool flat) {
     const int64_t waves = (nrays + 63) / 64;
-    if (flat) return waves < 1024 ? 8 : 4;
+    if (flat) return waves < 1024 ? 8 : waves * 4 * 64 <= kLaunchThreads ? 4 : 1;
     return waves < 2048 ? 4 : 1;
 }
 

@@ -362,6 +362,7 @@ static void tvd_march(const TvdShape& S, const float* g, float* const* q, int32_
 template <int ND, int K>
 static bool tvd_pays(const TvdShape& S) {
     const TvdPlan P = tvd_plan<ND, K>(S);
+    if (P.n * 512 > kLaunchThreads) return false;
     const double m = 1e-6 * (double)S.n, planes = std::min(P.chunk, S.n0) + 3 * K - 1;
     if (ND == 2) return planes * 0.95 <= K * std::max(7.2, 3.0 + 8.0 * m);
     return std::max(planes * (P.n <= 256 ? 1.65 : 2.35), 9.0 * m) <= K * std::max(8.0, 3.0 + 11.5 * m);

@@ -23,6 +23,9 @@ __device__ __forceinline__ int64_t xcd_remap(int64_t bid, int64_t nblocks) {
     return x * q + (x < r ? x : r) + i;
 }
 
+// Threads a launch can have.
+constexpr int64_t kLaunchThreads = 4294967295;
+
 int make_grid(const vir_grid* gp, GridK& g);
 
 // SIRT steps fused into a projector's write-back (sys_mat/sirt_dd.py:51-72),
