@@ -785,13 +785,18 @@ static int rd_setup(const vir_rd_geom* g, RDGeo& G) {
     return VIR_OK;
 }
 
-// False for cone-beam volumes so thin that the table kernel, whose 64 lanes run
-// along z, is slower than one thread per voxel: two slabs, or three with
-// interpolation, in bricks enough to fill the chip.  Table | per voxel, us, 60
-// views, slabs: Joseph 128^2 (512 bricks) 2: equal; 150^2 (722) 2: 1206 | 1140; 180^2
-// (1035) 2: 1704 | 1142, 3: 2251 | 1964; 220^2 3: 3123 | 2484, 4: 3108 | 3453; path
-// lengths 180^2 2: 629 | 617, 256^2 2: 983 | 787, 3: 990 | 1426.
+// False where the table kernels do not apply, and for cone-beam volumes so thin
+// that theirs, whose 64 lanes run along z, is slower than one thread per voxel:
+// two slabs, or three with interpolation, in bricks enough to fill the chip.
+// Table | per voxel, us, 60 views, slabs: Joseph 128^2 (512 bricks) 2: equal; 150^2
+// (722) 2: 1206 | 1140; 180^2 (1035) 2: 1704 | 1142, 3: 2251 | 1964; 220^2 3: 3123 |
+// 2484, 4: 3108 | 3453; path lengths 180^2 2: 629 | 617, 256^2 2: 983 | 787, 3: 990 |
+// 1426.
 static bool rd_tab_pays(const RDGeo& G, int mode, bool jo) {
+    // samples are counted in float32 there: exactly, and so that the count ends,
+    // below 2^24, a ray of 8.4 million units (grids in very small units)
+    const double nz = mode == RD_CONE3 ? G.nz : 0.0;
+    if (jo && std::sqrt((double)G.nx * G.nx + (double)G.ny * G.ny + nz * nz) * G.d > 8e6) return false;
     // (a launch can't have more threads)
     const int64_t blocks = mode == RD_CONE3 ? (int64_t)((G.nx + 3) / 4) * ((G.ny + 7) / 8) * ((G.nz + 63) / 64)
                                             : (int64_t)((G.nx + kRd2X - 1) / kRd2X) * ((G.ny + kRd2Y - 1) / kRd2Y);
