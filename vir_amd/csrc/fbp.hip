@@ -180,6 +180,13 @@ __global__ __launch_bounds__(64 * NW) void k_fbp_bp(FbpGeo G, const float* __res
                 v[2] = p;
                 v[3] = o;
             }
+            // a view without a finite angle: four bins off the detector's start,
+            // where it adds nothing (flat fan and atan2: tested per pixel)
+            if ((MODE == 0 || ARC) && !(fabs(p) + fabs(o) < (double)VIR_INF)) {
+                v[0] = v[1] = 0.0;
+                v[2] = ARC ? 1.0 : G.c0 - 4.0 / G.inv_du;
+                v[3] = ARC ? -4.0 : 0.0;
+            }
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // a wave's LDS accesses are in order
         const int nl = min(64, (G.na - g - wave + NW - 1) / NW);
