@@ -428,7 +428,8 @@ __global__ __launch_bounds__(256) void k_rd_bp(RDGeo G, const float* __restrict_
 
 // Bins [u0, u1] whose rays can meet the box [x0, x1] x [y0, y1] (the convex
 // hull of the projected corners, widened by G.mar for rounding), and the
-// least and largest magnification of its corners.
+// least and largest magnification of its corners.  u0 <= nu and u1 >= -1, also
+// for a view without a finite angle (none), so that lengths don't overflow.
 template <int MODE>
 __device__ __forceinline__ void rd_u_range(const RDGeo& G, float c, float s, float x0, float x1, float y0, float y1,
                                            int& u0, int& u1, float& mmin, float& mmax) {
@@ -447,8 +448,8 @@ __device__ __forceinline__ void rd_u_range(const RDGeo& G, float c, float s, flo
         mmax = fmaxf(mmax, m);
     }
     const float off = G.ucen - G.su;
-    u0 = (int)fmaxf(ceilf(umin * G.inv_du + off - G.mar), 0.0f);
-    u1 = (int)fminf(floorf(umax * G.inv_du + off + G.mar), (float)(G.nu - 1));
+    u0 = (int)fminf(fmaxf(ceilf(umin * G.inv_du + off - G.mar), 0.0f), (float)G.nu);
+    u1 = (int)fmaxf(fminf(floorf(umax * G.inv_du + off + G.mar), (float)(G.nu - 1)), -1.0f);
 }
 
 // Detector rows [v0, v1] of the heights [z0, z1] at magnifications [mmin, mmax].
@@ -456,8 +457,8 @@ __device__ __forceinline__ void rd_v_range(const RDGeo& G, float z0, float z1, f
                                            int& v1) {
     const float off = G.ucen - G.sv;
     const float lo = z0 * (z0 < 0.0f ? mmax : mmin), hi = z1 * (z1 < 0.0f ? mmin : mmax);
-    v0 = (int)fmaxf(ceilf(lo * G.inv_dv + off - G.mar), 0.0f);
-    v1 = (int)fminf(floorf(hi * G.inv_dv + off + G.mar), (float)(G.nv - 1));
+    v0 = (int)fminf(fmaxf(ceilf(lo * G.inv_dv + off - G.mar), 0.0f), (float)G.nv);
+    v1 = (int)fmaxf(fminf(floorf(hi * G.inv_dv + off + G.mar), (float)(G.nv - 1)), -1.0f);
 }
 
 // A ray of an LDS table.  Joseph: position at t0 (p) and step per sample (h)
