@@ -32,3 +32,30 @@ def test_ray_driven(geom, joseph, bad):
         kw.update(DSO=140.0, DSD=210.0, du=1.5)
     P, Q = (RDProjector(shape, a, 70, geom, joseph=joseph, **kw) for a in (_angles(bad), _angles(0.0)[KEEP]))
     _check_bp(P, Q, 2)
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+@pytest.mark.parametrize("kind,geom", [("dd", "par"), ("dd", "flat"), ("dd", "arc"), ("dd", "cone"), ("sf", "par"),
+                                       ("sf", "fan"), ("sf", "cone"), ("sf", "par3d"), ("sf", "par3d rows")])
+def test_footprints(kind, geom, bad):
+    import torch
+    from vir_amd.sys_mat.dd import DDProjector
+    from vir_amd.sys_mat.pd import SFProjector
+    shape, kw = (40, 41), {}
+    if geom in ("cone", "par3d", "par3d rows"):
+        shape, kw = (40, 41, 6), dict(nv=7 if geom == "cone" else 6)
+    if geom == "par3d rows":
+        kw.update(dv=0.9, sv=0.2)
+    if geom in ("flat", "arc", "fan", "cone"):
+        kw.update(DSO=140.0, DSD=210.0, du=1.5)
+    if kind == "dd":
+        if geom in ("flat", "arc"):
+            kw["detector"] = geom
+        make = lambda a: DDProjector(shape, a, 70, "fan" if geom in ("flat", "arc") else geom, **kw)
+    else:
+        make = lambda a: SFProjector(shape, a, 70, geom.split()[0], **kw)
+    P, Q = make(_angles(bad)), make(_angles(0.0)[KEEP])
+    x = torch.rand(shape, device="cuda", generator=torch.Generator("cuda").manual_seed(3))
+    a, b = P.fp(x), Q.fp(x)
+    assert torch.equal(a[KEEP], b) and not bool(a[[4, 8]].any())
+    _check_bp(P, Q, 4)

@@ -95,7 +95,8 @@ __global__ __launch_bounds__(64 * NW) void k_fp2d_tile(Geo G, const float* __res
     const int ia = (int)(row % G.na);
     img += (row / G.na) * G.nx * G.ny;
     const M V(G, typename M::Trig(cs[ia], sn[ia], ang ? ang[ia] : 0.0f));
-    const int nd = V.nd, no = V.no;
+    // (a view without a finite angle meets nothing)
+    const int nd = V.nd, no = fabsf(cs[ia]) + fabsf(sn[ia]) < VIR_INF ? V.no : 0;
     const float half = 0.5f * (float)nd, inv_d = 1.0f / G.d;
     const auto edge = [&](int j) { return G.du * (((float)j - 0.5f * (float)G.nu) + G.su); };
     // pixel range of the interval [u0, u1]: position p0 - oc q0 .. p1 - oc q1,
@@ -312,8 +313,11 @@ __global__ __launch_bounds__(64 * NW) void k_bp2d_tile(Geo G, const float* __res
         for (int g = 0; g < G.na; g += 64 * NW) {
             const int il = min(g + NW * lane + wave, G.na - 1);
             const typename M::Trig tl(cs[il], sn[il], ang ? ang[il] : 0.0f);  // lane = view
+            // (a comparison with infinity inside the ballot is compiled to one that NaN passes)
+            const uint64_t finite = __ballot(0.0f * cs[il] + 0.0f * sn[il] == 0.0f);
             const int nl = min(64, (G.na - g - wave + NW - 1) / NW);
             for (int l = ch; l < nl; l += STEP) {
+                if (!((finite >> l) & 1)) continue;
                 const M V(G, tl.lane(l));
                 const float* __restrict__ row = sino + (int64_t)(g + NW * l + wave) * G.nu;
                 float lo[4], hi[4], f[4];

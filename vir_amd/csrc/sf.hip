@@ -599,7 +599,8 @@ __global__ __launch_bounds__(64 * kVG * NG) __attribute__((amdgpu_waves_per_eu(4
     // views whose driving axis is that of the first view, then the others
     for (int pass = 0; pass < (mixed ? 2 : 1); ++pass) {
         const bool pxd = pass == 0 ? gxd[0] : !gxd[0];
-        const bool active = vwave && xd == pxd;
+        // (a view without a finite angle meets nothing)
+        const bool active = vwave && xd == pxd && fabsf(V.c) + fabsf(V.s) < VIR_INF;
         const int pnd = pxd ? G.nx : G.ny, pno = pxd ? G.ny : G.nx;
         const int64_t kstride = (int64_t)(pxd ? G.ny : 1) * G.nz, lstride = (int64_t)(pxd ? 1 : G.ny) * G.nz;
         for (int lb = 0; lb < pno; lb += 64) {
@@ -1012,7 +1013,7 @@ __global__ __launch_bounds__(256) void k_sf_bp_par3_mfma(SFGeo G, const float* _
             for (int kk = 0; kk < KS; ++kk) {
                 const int j = jb + 4 * kk + hi;
                 const float ou = ovl(u0, u1, sf_det(G.nu, G.du, G.su, j), sf_det(G.nu, G.du, G.su, j + 1));
-                T.w[kk] = ou > 0.0f ? (double)((ou * inv_du) * amp) : 0.0;
+                T.w[kk] = ou > 0.0f && h < VIR_INF ? (double)((ou * inv_du) * amp) : 0.0;
             }
         };
         const auto use = [&](const View& T) {
