@@ -14,6 +14,8 @@ CASES = [
     ("par", dict(shape=(64, 60), nu=92, na=90), 70),
     ("fan", dict(shape=(64, 60), nu=92, na=90, DSO=140.0, DSD=210.0, du=1.5), 70),
     ("fan", dict(shape=(16, 16), nu=140, na=9, DSO=40.0, DSD=60.0, du=0.3), 5),
+    ("par", dict(shape=(16, 24), nu=30, na=45), 100),                       # narrow detectors: per output in the batch
+    ("fan", dict(shape=(20, 16), nu=17, na=45, DSO=50.0, DSD=75.0, du=3.0), 600),
     ("par3d", dict(shape=(64, 60, 40), nu=96, nv=40, na=13), 40),
     ("par3d", dict(shape=(64, 60, 10), nu=96, nv=7, na=13, dv=0.8, sv=0.1), 40),
     ("par3d", dict(shape=(40, 44, 16), nu=30, nv=16, na=9, du=2.6), 40),

@@ -367,13 +367,13 @@ __global__ __launch_bounds__(256) void k_sf_fp(SFGeo G, const float* __restrict_
     bool slab_general = false;
     if (MODE == SF_PAR3) slab_general = !par3_row_slabs(G, iv, SW);
     double acc = 0.0;
-    for (int io = 0; io < no; ++io) {
+    const auto line = [&](int io) {
         const float oc = (sf_bnd(no, G.d, io) + sf_bnd(no, G.d, io + 1)) * 0.5f;
         float x0 = sf_invert<MODE>(G, xd, c, s, ul - G.wmax, oc);
         float x1 = sf_invert<MODE>(G, xd, c, s, ur + G.wmax, oc);
         float k0f = fminf(x0, x1) * inv_d + 0.5f * (float)nd - 0.5f;
         float k1f = fmaxf(x0, x1) * inv_d + 0.5f * (float)nd - 0.5f;
-        if (!(k0f < (float)nd + 1.0f) || !(k1f > -2.0f)) continue;
+        if (!(k0f < (float)nd + 1.0f) || !(k1f > -2.0f)) return;
         int k0 = (int)fmaxf(floorf(k0f) - 1.0f, 0.0f);
         int k1 = (int)fminf(floorf(k1f) + 2.0f, (float)(nd - 1));
         for (int k = k0; k <= k1; ++k) {
@@ -409,6 +409,22 @@ __global__ __launch_bounds__(256) void k_sf_fp(SFGeo G, const float* __restrict_
                 }
             }
         }
+    };
+    if (is3) {
+        for (int io = 0; io < no; ++io) line(io);
+    } else {
+        // in the tile's chains of lines: the same bits
+        double sum = 0.0;
+        for (int w = 0; w < 4; ++w) {
+            double part = 0.0;
+            for (int c = w; c < kFtLines; c += 4) {
+                acc = 0.0;
+                for (int io = c; io < no; io += kFtLines) line(io);
+                part += acc;
+            }
+            sum += part;
+        }
+        acc = sum;
     }
     float res = (float)acc * G.out_scale;
     if (accumulate) res += sino[t];
@@ -1323,6 +1339,17 @@ static int sf_setup(const vir_sf_geom* g, SFGeo& G) {
 
 using namespace vir;
 
+// Small images on detectors a fraction of the 2-D tile's 128 bins wide: with rows
+// enough to fill the chip one thread per bin is faster.  (Lines the tile stages at
+// once, so both give the same bits and the batch may count.)  Tile | per output, us:
+// parallel 16^2, 11520 rows of 24 bins 53 | 40, of 48 53 | 60, 92160 rows of 24 356 | 182;
+// 64^2, 128000 rows of 33 bins 1895 | 1570, of 48 1718 | 2006; fan 64^2, 128000 rows of 16
+// bins 8908 | 6700, of 24 8203 | 8190.
+static bool sf_narrow(const SFGeo& G, int mode) {
+    const int64_t rows = (int64_t)G.nb * G.na;
+    return std::max(G.nx, G.ny) <= 64 && (mode == SF_PAR2 ? G.nu <= 36 && rows >= 8192 : G.nu <= 20 && rows >= 50000);
+}
+
 extern "C" {
 
 int vir_sf_fp(const vir_sf_geom* geom, const float* ang, const float* cosv, const float* sinv, const float* img,
@@ -1346,7 +1373,7 @@ int vir_sf_fp(const vir_sf_geom* geom, const float* ang, const float* cosv, cons
     hipStream_t st = as_stream(stream);
     int acc = (flags & VIR_ACCUMULATE) ? 1 : 0;
     // VIR_COMPAT's amplitudes depend on the pixels before: the gather looks back
-    const bool flat = !G.compat && !(flags & VIR_PER_OUTPUT);
+    const bool flat = !G.compat && !(flags & VIR_PER_OUTPUT) && !sf_narrow(G, geom->mode);
     if (flat && geom->mode == SF_PAR2)
         return ft_fp<SFFlat<SF_PAR2>>(G, G.nb, ang, cosv, sinv, img, sino, acc, st, SirtEpi{}, "vir_sf_fp launch");
     if (flat && geom->mode == SF_FAN2)
