@@ -713,13 +713,19 @@ struct BpPlan {
     int nchunks, views_per_chunk;
 };
 
-// Workgroups aimed at for 3-D grids: eight a CU, two rounds of the four that
-// are resident, so that a round's last blocks overlap the next one's; 1024 left
-// the slowest block to bound the call.  Only while the partial volumes fit
-// VIR_SIDDON_BP_SCRATCH_BYTES (a plan that needed more for 1024 keeps those).
-// Projection pair, 100 views of 1.45 n x 1.3 n, 1024 | 2048 in us: 48^3 220 | 185,
-// 64^3 552 | 458, 96^3 784 | 762, 128^3 1790 | 1540; 160^3 has the same plan.
-constexpr int64_t kBp3Target = 2048;
+// Workgroups aimed at for 3-D grids: four a CU, as many as are resident, or twice
+// that, where the second half's blocks fill in behind the first's (while the
+// partial volumes fit VIR_SIDDON_BP_SCRATCH_BYTES).  A wave walks two views at a
+// time (NS), so the shorter chunks have an even number of views.  Not where one
+// chunk needs no partial volumes, where a chunk is a single view and the chip not
+// full, or where the first plan fills the chip just so and has at most eight views a
+// chunk, in pairs, or the second would fill little more.  1024 | 2048 (views a
+// chunk), us: 64^3, 90 views 361 (6) | 329 (4), 48 x 48 x 32, 90 views 215 (3) | 155 (2),
+// 200 x 200 x 24, 60 views 901 (15) | 689 (8), 128^3, 90 views 1704 | 1502; kept 96 x 96 x
+// 64, 10 views 117 (2) | with one view 182, 128 x 128 x 32, 40 views 309 (5) | 340 (4).
+// Over 206 grids of 4 to 128 slabs and 10 to 120 views 7 % faster in the mean than
+// 1024, none slower by more than 1.5 %.
+constexpr int64_t kBp3Target = 1024;
 
 template <class S>
 static void bp_regions(BpPlan& p, const GridK& g) {
@@ -736,7 +742,8 @@ static void bp_regions(BpPlan& p, const GridK& g) {
 // 256 (360 views) 242 | 189, 512 812 | 660.
 static BpPlan plan_bp(const GridK& g, int nviews) {
     BpPlan p;
-    int target = 1024, most = nviews;
+    int64_t target = kBp3Target;
+    int most = nviews;
     if (g.n[2] == 1) {
         p.kind = 1;
         bp_regions<BpShape2>(p, g);
@@ -750,15 +757,26 @@ static BpPlan plan_bp(const GridK& g, int nviews) {
         p.kind = 0;
         bp_regions<BpShape3>(p, g);
     }
-    int64_t nb = (int64_t)p.nbx * p.nby * p.nbz;
-    int64_t nch = (target + nb - 1) / nb;
-    if (p.kind == 0) {
+    const int64_t nb = (int64_t)p.nbx * p.nby * p.nbz;
+    const auto views = [&](int64_t nch) {
+        nch = std::min<int64_t>(most, std::max<int64_t>(1, nch));
+        return (int)((nviews + nch - 1) / nch);
+    };
+    const auto chunks = [&](int v) { return (nviews + v - 1) / v; };
+    p.views_per_chunk = views((target + nb - 1) / nb);
+    p.nchunks = chunks(p.views_per_chunk);
+    if (p.kind == 0 && p.nchunks > 1) {
         const int64_t fit = (int64_t)VIR_SIDDON_BP_SCRATCH_BYTES / ((int64_t)g.n[0] * g.n[1] * g.n[2] * (int64_t)sizeof(float));
-        nch = std::max(nch, std::min((kBp3Target + nb - 1) / nb, fit));
+        const int v = p.views_per_chunk;
+        int v2 = views(std::min((2 * kBp3Target + nb - 1) / nb, fit));
+        v2 += v2 & 1;
+        const int64_t blocks = nb * p.nchunks, blocks2 = nb * chunks(v2);
+        const bool full = blocks >= 1000 && blocks <= kBp3Target;
+        if (v2 < v && !(full && ((v % 2 == 0 && v <= 8) || blocks2 < 1400))) {
+            p.views_per_chunk = v2;
+            p.nchunks = chunks(v2);
+        }
     }
-    nch = std::min<int64_t>(most, std::max<int64_t>(1, nch));
-    p.views_per_chunk = (int)((nviews + nch - 1) / nch);
-    p.nchunks = (nviews + p.views_per_chunk - 1) / p.views_per_chunk;
     return p;
 }
 
