@@ -28,6 +28,7 @@
 // 128^3, 180 views of 192^2: 5.5 -> 0.82 ms / 2.7 -> 0.59 ms; separable footprint
 // 120 x 132 x 101, 150 views of 187 x 150: 8.3 -> 0.98 ms / 2.1 -> 0.55 ms.
 #pragma once
+#include <algorithm>
 #include <type_traits>
 
 #include "vir_common.h"
@@ -508,14 +509,15 @@ int ct_bp(const Geo& G, int nb, int ns, const float* ang, const float* cosv, con
     const int nzt = (G.nz + 63) / 64;
     const int64_t ncol = (int64_t)nb * G.nx * G.ny * nzt;
     // Thin volumes leave most lanes of a column idle: with more columns than fill
-    // the chip a thread a voxel is faster up to about 18 slabs.  A view costs
-    // about 0.1 us a thousand columns or 0.4 us and 0.33 a thousand waves of
-    // voxels.  Columns | voxels in us, distance driven, 60 views: 64^2 x 8 38 | 54;
+    // the chip a thread a voxel is faster up to about 18 slabs, and with few
+    // views, for which a column's lists cost as much as for 64, up to more.  A
+    // thousand columns take about 0.42 us every 64 views and 0.09 a view; a view
+    // 0.4 us and 0.33 a thousand waves of voxels.  Columns | voxels in us, distance driven, 60 views: 64^2 x 8 38 | 54;
     // 128^2 x 4 106 | 55, x 12 105 | 83, x 16 105 | 101; 256^2 x 3 371 | 82, x 8 368 |
     // 178, x 16 371 | 332; 512^2 x 16, 30 views, 772 | 638, x 70 1558 | 2708.  Both give
     // the same bits, so the batch may count.
     const int64_t n = (int64_t)nb * G.nx * G.ny * G.nz;
-    const bool thin = (double)G.nz / nzt < 19.0 - 8e4 / (double)ncol;
+    const bool thin = (double)G.nz / nzt < 17.5 + 82.0 * ((G.na + 63) / 64) / std::max(G.na, 1) - 7.8e4 / (double)ncol;
     const dim3 grd((unsigned)(((thin ? (n + 63) / 64 : ncol) + 3) / 4)), blk(256);
     const auto run = [&](auto slots) {
         constexpr int NS = decltype(slots)::value;
