@@ -70,9 +70,9 @@ def test_infinite_rows_of_thin_volumes(kind):
 
 
 @pytest.mark.parametrize("kind", ["dd", "sf"])
-@pytest.mark.parametrize("nv,na,nu", [(3, 140, 400), (3, 120, 400), (4, 177, 400), (4, 176, 400), (5, 180, 400)])
+@pytest.mark.parametrize("nv,na,nu", [(3, 93, 400), (3, 92, 400), (4, 177, 400), (4, 176, 400), (5, 180, 400)])
 def test_projection_onto_few_rows(nv, na, nu, kind):
-    """25 blocks a view: 3 rows of 132 views and 4 of 176 are on the line."""
+    """25 blocks a view: 3 rows of 92 views and 4 of 176 are on the line."""
     import torch
     from vir_amd.sys_mat.dd import DDProjector
     from vir_amd.sys_mat.pd import SFProjector

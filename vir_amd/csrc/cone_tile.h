@@ -476,10 +476,11 @@ inline int ct_slots(double len, int n) {
 // don't depend on the batch) that fill the chip several times over.  Tile | per
 // output, us, rows as slabs, distance driven: 256^2, 360 views (8640 blocks) 3 rows
 // 1701 | 1305, 4: 1709 | 1522, 6: (32 slabs) 2041 | 2204; 128^2, 360 views (4320)
-// 3: 508 | 441, 4: 500 | 538; 256^2, 60 views (1440) 3: 371 | 630.
+// 3: 508 | 441, 4: 500 | 538; 256^2, 60 views (1440) 3: 371 | 630; 181 x 94 x 2, 306
+// views of 123 x 3 (2448) 537 | 466.
 template <class Geo>
 bool ct_few_rows(const Geo& G) {
-    return G.nv <= 4 && (int64_t)G.na * ((G.nu + kCtBins - 1) / kCtBins) > 1100 * (int64_t)G.nv;
+    return G.nv <= 4 && (int64_t)G.na * ((G.nu + kCtBins - 1) / kCtBins) > (G.nv < 4 ? 2300 : 4400);
 }
 
 // Threads that one item's launch takes.
