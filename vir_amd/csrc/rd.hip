@@ -428,8 +428,8 @@ __global__ __launch_bounds__(256) void k_rd_bp(RDGeo G, const float* __restrict_
 
 // Bins [u0, u1] whose rays can meet the box [x0, x1] x [y0, y1] (the convex
 // hull of the projected corners, widened by G.mar for rounding), and the
-// least and largest magnification of its corners.  u0 <= nu and u1 >= -1, also
-// for a view without a finite angle (none), so that lengths don't overflow.
+// least and largest magnification of its corners.  (A view without a finite
+// angle: [INT_MAX, INT_MIN].)
 template <int MODE>
 __device__ __forceinline__ void rd_u_range(const RDGeo& G, float c, float s, float x0, float x1, float y0, float y1,
                                            int& u0, int& u1, float& mmin, float& mmax) {
@@ -448,8 +448,8 @@ __device__ __forceinline__ void rd_u_range(const RDGeo& G, float c, float s, flo
         mmax = fmaxf(mmax, m);
     }
     const float off = G.ucen - G.su;
-    u0 = (int)fminf(fmaxf(ceilf(umin * G.inv_du + off - G.mar), 0.0f), (float)G.nu);
-    u1 = (int)fmaxf(fminf(floorf(umax * G.inv_du + off + G.mar), (float)(G.nu - 1)), -1.0f);
+    u0 = (int)fmaxf(ceilf(umin * G.inv_du + off - G.mar), 0.0f);
+    u1 = (int)fminf(floorf(umax * G.inv_du + off + G.mar), (float)(G.nu - 1));
 }
 
 // Detector rows [v0, v1] of the heights [z0, z1] at magnifications [mmin, mmax].
@@ -457,8 +457,8 @@ __device__ __forceinline__ void rd_v_range(const RDGeo& G, float z0, float z1, f
                                            int& v1) {
     const float off = G.ucen - G.sv;
     const float lo = z0 * (z0 < 0.0f ? mmax : mmin), hi = z1 * (z1 < 0.0f ? mmin : mmax);
-    v0 = (int)fminf(fmaxf(ceilf(lo * G.inv_dv + off - G.mar), 0.0f), (float)G.nv);
-    v1 = (int)fmaxf(fminf(floorf(hi * G.inv_dv + off + G.mar), (float)(G.nv - 1)), -1.0f);
+    v0 = (int)fmaxf(ceilf(lo * G.inv_dv + off - G.mar), 0.0f);
+    v1 = (int)fminf(floorf(hi * G.inv_dv + off + G.mar), (float)(G.nv - 1));
 }
 
 // A ray of an LDS table.  Joseph: position at t0 (p) and step per sample (h)
@@ -693,6 +693,8 @@ __global__ __launch_bounds__(64 * NW) void k_rd_bp_2d_tab(RDGeo G, const float* 
         int U0, U1;
         float m0, m1;
         rd_u_range<MODE>(G, cs[ia], sn[ia], X0, X1, Y0, Y1, U0, U1, m0, m1);
+        U0 = min(U0, G.nu);   // lengths and indexes below don't overflow
+        U1 = max(U1, -1);
         if (a0 + slot >= G.na) U1 = U0 - 1;
         // the two views' ranges, the same in every lane
         const int A0 = __builtin_amdgcn_readlane(U0, 0), A1 = __builtin_amdgcn_readlane(U1, 0);
