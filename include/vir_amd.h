@@ -305,15 +305,18 @@ typedef struct vir_dd_geom {
 } vir_dd_geom;
 
 /* sino[a, u] = out_scale * sum_pixels img * overlap * ray_scale, a gather per
- * bin in tiles of 128 bins (VIR_PER_OUTPUT: one thread per bin).  The reference's dd_fp_par_2d / dd_fp_fan_2d use
- * out_scale = d_pix/du (dd.py:725, 803). */
+ * bin in tiles of 128 bins (VIR_PER_OUTPUT: one thread per bin).  The
+ * reference's dd_fp_par_2d / dd_fp_fan_2d use out_scale = d_pix/du (dd.py:725,
+ * 803). */
 int vir_dd2d_fp(const vir_dd_geom *geom, const float *cosv, const float *sinv,
                 const float *img, float *sino, float out_scale, uint32_t flags,
                 void *stream);
 
-/* Exact transpose of vir_dd2d_fp (same weights), a gather per pixel in tiles
- * of 16 x 16 pixels (VIR_PER_OUTPUT: one thread per pixel).  The reference's dd_bp_par_2d / dd_bp_fan_2d use out_scale = 1/(na*d_pix)
- * (dd.py:721-722, 799-800); out_scale = d_pix/du gives the exact adjoint. */
+/* Transpose of vir_dd2d_fp, to the float32 rounding of the weights (exact with
+ * VIR_PER_OUTPUT in both), a gather per pixel in tiles of 16 x 16 pixels
+ * (VIR_PER_OUTPUT: one thread per pixel).  The reference's dd_bp_par_2d /
+ * dd_bp_fan_2d use out_scale = 1/(na*d_pix) (dd.py:721-722, 799-800); out_scale
+ * = d_pix/du gives the adjoint. */
 int vir_dd2d_bp(const vir_dd_geom *geom, const float *cosv, const float *sinv,
                 const float *sino, float *img, float out_scale, uint32_t flags,
                 void *stream);
@@ -335,8 +338,10 @@ int vir_ddcone_fp(const vir_dd_geom *geom, const float *cosv, const float *sinv,
                   const float *vol, float *sino, float out_scale, uint32_t flags,
                   void *stream);
 
-/* Exact transpose of vir_ddcone_fp (of its default mode; VIR_COMPAT is
- * ignored); reference scaling 1/(na*d_pix). */
+/* Transpose of vir_ddcone_fp (of its default mode; VIR_COMPAT is ignored) to
+ * the float32 rounding of the weights (exact with VIR_PER_OUTPUT in both);
+ * reference scaling 1/(na*d_pix).  Both take tiles where a row meets at most
+ * four slabs (a slab four rows), else one thread per output. */
 int vir_ddcone_bp(const vir_dd_geom *geom, const float *cosv, const float *sinv,
                   const float *sino, float *vol, float out_scale, uint32_t flags,
                   void *stream);
@@ -384,17 +389,23 @@ typedef struct vir_sf_geom {
 
 /* sino = out_scale * sum over pixels of img * amplitude * overlap/du
  * (* overlap_v/dv).  The reference scales by d_pix (pd.py:234, 350, 485).
- * Parallel 3-D with rows no taller than a voxel runs a tiled kernel that
- * stages each orthogonal line's pixels in LDS (same bits as the one-thread-
- * per-bin gather, which VIR_PER_OUTPUT selects). */
+ * Sums are float64.  2-D takes tiles of 128 bins (not with VIR_COMPAT); cone
+ * beam tiles where a row meets at most four slabs; parallel 3-D float64 matrix
+ * products where rows are no taller than a voxel, there are at least six and
+ * bins are at most 2.5 pixels wide (up to 3.2 for items of many blocks).  Else,
+ * and with VIR_PER_OUTPUT, one thread per bin.  The forms agree to the float32
+ * rounding of the weights, the parallel 3-D ones to that of the result; an
+ * item's bits do not depend on its batch. */
 int vir_sf_fp(const vir_sf_geom *geom, const float *ang, const float *cosv,
               const float *sinv, const float *img, float *sino, float out_scale,
               uint32_t flags, void *stream);
 
-/* Exact transpose of vir_sf_fp, one thread per pixel/voxel (parallel 3-D
- * with rows at least half a voxel tall: one wave per pixel column with the
- * footprints of 64 views computed at once, same bits; VIR_PER_OUTPUT selects
- * the per-voxel kernel).  The reference's
+/* Transpose of vir_sf_fp to the float32 rounding of the weights (exact with
+ * VIR_PER_OUTPUT in both).  2-D takes tiles of 16 x 16 pixels; cone beam a wave
+ * per column where a slab meets at most four rows, a thread per voxel for thin
+ * volumes (same bits); parallel 3-D float64 matrix products where rows align
+ * with the slabs, else, with rows at least half a voxel tall, one wave per pixel
+ * column.  VIR_PER_OUTPUT: one thread per pixel/voxel.  The reference's
  * backprojectors use out_scale = du/(na*d_pix) (2-D, pd.py:231-232, 347-348)
  * and du*dv/(na*d_pix) (cone, pd.py:482-483). */
 int vir_sf_bp(const vir_sf_geom *geom, const float *ang, const float *cosv,

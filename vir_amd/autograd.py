@@ -1,6 +1,6 @@
 """Differentiable projection and reconstruction losses.
 
-`project(x, P)` applies any projector with an exact adjoint pair
+`project(x, P)` applies any projector with an adjoint pair
 (SFProjector, DDProjector, SiddonProjector): forward P.fp, backward P.bp,
 both hand-written HIP kernels.  `least_squares` and `total_variation` are
 loss terms whose values are reduced in double on the device and whose

@@ -10,7 +10,9 @@ Every HIP translation unit is compiled with:
                                keep the compiler from emitting packed FP32 ops
   -mllvm -amdgpu-mfma-vgpr-form=1
                                matrix accumulators stay in VGPRs (copies to and
-                               from AGPRs cost a float64 product 60 % more time)
+                               from AGPRs cost a float64 product 60 % more time);
+                               an option of this compiler: for one that does not
+                               know it leave it out, the results are the same
 """
 import os
 import subprocess

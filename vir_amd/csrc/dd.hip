@@ -9,11 +9,13 @@
 // in-plane source distance of the row centre).  The cone variant multiplies
 // by the overlap of the slab's magnified z interval with the detector row.
 //
-// Both directions are gathers (no atomics): the forward kernel runs one
-// thread per detector bin and finds the pixels whose shadows meet it by
-// inverting the projection; the backward kernel runs one thread per pixel
-// (voxel) and visits the bins its shadow meets.  Both evaluate every weight
-// through the same functions, so they are exact transposes.
+// Both directions are gathers (no atomics): forward, a detector bin finds the
+// pixels whose shadows meet it by inverting the projection; backward, a pixel
+// (voxel) visits the bins its shadow meets.  The one-thread-per-output kernels
+// here evaluate every weight through the same functions, so they are exact
+// transposes; the tiles (flat_tile.h, cone_tile.h), which calls take by default,
+// form the same projected edges but the overlaps in their own units and order,
+// and are transposes to the float32 rounding of the weights.
 #include <algorithm>
 #include <cmath>
 

@@ -12,11 +12,15 @@
 // weight per bin = overlap/du (* overlap_v/dv); the forward output is
 // scaled by d_pix (pd.py:234, 350, 485).
 //
-// Forward: one thread per (batch, view, bin[, row]) gathers the pixels whose
-// footprints meet the bin (centre projection inverted along the driving axis,
-// widened by the largest footprint half-width).  Backward: one thread per
-// (batch, pixel[, slab]) visits the bins its footprint meets.  Both evaluate
-// every weight with the same functions: exact transposes, no atomics.
+// Forward: a (batch, view, bin[, row]) gathers the pixels whose footprints meet
+// the bin (centre projection inverted along the driving axis, widened by the
+// largest footprint half-width).  Backward: a (batch, pixel[, slab]) visits the
+// bins its footprint meets.  No atomics.  One thread per output (VIR_PER_OUTPUT,
+// and where nothing else applies) every weight comes from the same functions in
+// both directions, an exact transpose.  Most calls take tiles: flat_tile.h (2-D),
+// cone_tile.h, and for parallel 3-D the matrix kernels below, whose footprints are
+// the same but whose overlaps are formed in their own units and order, so that
+// the pair is a transpose to the float32 rounding of the weights.
 //
 // VIR_COMPAT (fan forward only): the reference skips a zero pixel without
 // advancing its o boundary (pd.py:321-325), so the next nonzero pixel's

@@ -210,7 +210,7 @@ __global__ __launch_bounds__(kRayThreads) __attribute__((amdgpu_waves_per_eu(NB 
 }
 
 // k_siddon_fp with each ray's walk divided among the S waves of a workgroup of
-// 64 rays: wave i takes the pairs whose left element lies in (T_i, T_i+1],
+// 64 rays: wave i takes the pairs whose right element lies in (T_i, T_i+1],
 // T_i = amin + i/S (amax - amin), entering at T_i with walker_seek, which
 // recomputes the same plane alphas.  A walk that ends past T_i+1 has also
 // visited the pair across it, the next wave's first; that one is taken back

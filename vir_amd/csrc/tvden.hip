@@ -118,10 +118,10 @@ __global__ __launch_bounds__(256) void k_tvd_max(float* __restrict__ dmax, int n
 // g once, runs K iterations and writes q once, into a second array.
 //
 // At 256^3 two iterations take 150 us, 600 MB of HBM traffic (380 read with
-// the tiles' margins): 4.0 of the 5.2 TB/s of a copy.  With one iteration a
-// pass a launch takes longer still (170 us), with two or four rows a lane
-// instead of three 50 iterations take 4.5 or 9.6 ms (spills) against 3.99, and
-// without the XCD placement 4.3.
+// the tiles' margins; 36 B a voxel, where q and g read and q written once are 28):
+// 4.0 of the 5.2 TB/s of a copy.  With one iteration a pass a launch takes longer
+// still (170 us), with two or four rows a lane instead of three 50 iterations take
+// 4.5 or 9.6 ms (spills) against 3.99, and without the XCD placement 4.3.
 //
 // A wave covers 64 voxels along the last axis (lane = voxel) and marches along
 // axis 0; in 3-D each lane holds R rows along axis 1 and the G waves of a

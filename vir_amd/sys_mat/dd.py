@@ -18,8 +18,8 @@ output scaling:
 
 The reference's backprojectors are A^T scaled by du/(na*d_pix^2) (2-D) and
 du*dv/(na*d_pix^3) (cone); these functions keep that scaling.  DDProjector is
-the device-resident operator pair with the exact adjoint (bp = A^T), plus an
-equiangular-detector fan variant (detector="arc").
+the device-resident operator pair with the adjoint (bp = A^T to the float32
+rounding of the weights), plus an equiangular-detector fan variant (detector="arc").
 
 numpy in -> numpy out; CUDA tensors in -> CUDA tensors out.
 """
@@ -46,7 +46,8 @@ def as_float32(*args):
 
 
 class DDProjector:
-    """Distance-driven forward projector A and its exact adjoint A^T.
+    """Distance-driven forward projector A and its adjoint A^T (a transpose to
+    the float32 rounding of the weights).
 
     geom: "par", "fan" or "cone"; detector: "flat" (the reference's) or
     "arc" (equiangular fan, du = arc length at radius DSD).  Angles in

@@ -15,8 +15,8 @@ output scaling:
 Forward projections are d_pix * W img; the reference's backprojections are
 du/(na*d_pix) * W^T sino (2-D) and du*dv/(na*d_pix) * W^T sino (cone).
 
-SFProjector is the device-resident operator pair (fp = A, bp = A^T exactly)
-with a batch dimension, and adds geometry "par3d": 3-D parallel beam with
+SFProjector is the device-resident operator pair (fp = A, bp = A^T to the
+float32 rounding of the weights) with a batch dimension, and adds geometry "par3d": 3-D parallel beam with
 the detector rows along z (each z-slice projected like pd_p_par_2d,
 weighted by the overlap of the slab with the rows of height dv).
 
@@ -39,7 +39,8 @@ _MODES = {"par": 0, "fan": 1, "cone": 2, "par3d": 3}
 
 
 class SFProjector:
-    """Separable-footprint forward projector A and its exact adjoint A^T.
+    """Separable-footprint forward projector A and its adjoint A^T (a transpose
+    to the float32 rounding of the weights).
 
     img_shape: (nx, ny) for "par"/"fan", (nx, ny, nz) for "cone"/"par3d".
     batch: number of volumes projected per call (leading dimension when
